@@ -29,7 +29,7 @@ HIP_FLAGS = [
     "-I", os.path.join(ROOT, "include"), "-I", os.path.join(HERE, "csrc"),
     "-Wno-unused-result", "-Wno-unused-value",
 ]
-# per source: the FP64 plain path is compiled without FMA contraction so it
+# per source: the FP64 path is compiled without FMA contraction so it
 # rounds like the CPU oracle; the FP32 transport kernel may contract and uses
 # the hardware transcendental instructions (v_exp_f32, v_log_f32, v_sin_f32,
 # v_cos_f32) and reciprocal-based division and square root, and flushes FP32
@@ -39,6 +39,7 @@ HIP_SOURCES = {
     "dxmc_hip.hip": ["-ffp-contract=off"],
     "tables.hip": ["-ffp-contract=off"],
     "transport_fp32.hip": ["-fgpu-approx-transcendentals", "-fno-hip-fp32-correctly-rounded-divide-sqrt", "-fgpu-flush-denormals-to-zero"],
+    "transport_fp64.hip": ["-ffp-contract=off"],
     "autotune.hip": [],
     "world.hip": [],
     "noalloc.hip": ["-ffp-contract=off"],

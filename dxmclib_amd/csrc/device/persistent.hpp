@@ -1,0 +1,175 @@
+// Pieces shared by the two persistent transport kernels (transport_fp32.hip,
+// transport_fp64.hip): lane phases, ranks among lanes, table access by 32-bit
+// offsets, and the copy of tables into LDS.
+#pragma once
+#include "physics.hpp"
+
+namespace dxmc_dev {
+
+// A lane of a persistent kernel holds no photon (waits for regeneration),
+// advances Woodcock flights, or has a real interaction due.
+enum : uint32_t { DEAD = 0, FLYING = 1, PENDING = 2 };
+
+// World kinds the persistent kernels are compiled for: the two common layouts
+// get their code width, record width, 24-bit index and bounds table fixed at
+// compile time, so a flight carries no branches on them
+//   WORLD_CODES8    1-byte bounded-density codes (and their block codes
+//                   when the run uses them), 8-byte records, the
+//                   attenuation bounds table, 24-bit index (CT-sized worlds)
+//   WORLD_PALETTE8  1-byte palette indices, no codes, 24-bit index
+//   WORLD_ANY       every other world (branches at run time)
+enum : uint32_t { WORLD_ANY = 0, WORLD_CODES8 = 1, WORLD_PALETTE8 = 2 };
+
+__device__ inline uint32_t rankBelow(uint64_t mask)
+{
+    return __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(mask >> 32), __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(mask), 0u));
+}
+
+// inside the safe extent, without short-circuit branches
+template <typename T>
+__device__ inline bool insideFast(const World<T>& w, const T* pos)
+{
+    return (pos[0] > w.extent[0]) & (pos[0] < w.extent[1]) & (pos[1] > w.extent[2]) & (pos[1] < w.extent[3]) & (pos[2] > w.extent[4])
+        & (pos[2] < w.extent[5]);
+}
+
+// linear voxel index; with 24-bit products where the grid allows (the
+// compiler turns a 24-bit multiply-add into a 64-bit one, so the three terms
+// are summed instead)
+template <typename T>
+__device__ inline uint64_t voxelIndexFast(const World<T>& w, uint3 v, bool index24)
+{
+    if (index24)
+        return __umul24(v.z, w.nxy) + __umul24(v.y, w.nx) + v.x;
+    return (static_cast<uint64_t>(v.z) * w.ny + v.y) * w.nx + v.x;
+}
+
+// element 'index' of a table addressed by a 32-bit byte offset from its
+// base (tables below 4 GiB): the load takes the base from scalar registers
+// and the offset from one vector register, with no 64-bit address
+// arithmetic per lane
+template <typename T>
+__device__ inline T loadAt(const T* base, uint32_t index)
+{
+    return *reinterpret_cast<const T*>(reinterpret_cast<const unsigned char*>(base) + index * static_cast<uint32_t>(sizeof(T)));
+}
+
+// block of a voxel (1-byte code worlds: 24-bit products hold)
+template <typename T>
+__device__ inline uint32_t blockIndexFast(const World<T>& w, uint3 v)
+{
+    return __umul24(v.z >> w.blockShift, w.bnxy) + __umul24(v.y >> w.blockShift, w.bnx) + (v.x >> w.blockShift);
+}
+
+// ------------------------------------------------------ LDS-staged tables
+// The tables the samplers read with data-dependent indices (RITA, spline,
+// shells, spectrum alias tables, heel and bowtie filters, the majorant and
+// the segment bounds or nodes, optionally the attenuation coefficients) are copied
+// into LDS at kernel start, one copy per block: their lookups then cost LDS
+// latency instead of L2 latency, also while the world gathers keep evicting
+// them from L1. Staging level: 1 none, 2 all but the attenuation
+// coefficients, 3 all. Of the interaction tables only those of the run's
+// low-energy model are staged (RITA for L >= 1, the scatter-function spline
+// for L = 1, the shells for L = 2). The total-attenuation bounds stay in
+// global memory: in LDS they cost a resident block per CU.
+enum : uint32_t { STAGE_NONE = 1, STAGE_SMALL = 2, STAGE_ALL = 3 };
+
+__host__ __device__ constexpr uint32_t ldsAlign(uint64_t bytes) { return static_cast<uint32_t>((bytes + 15) & ~uint64_t(15)); }
+
+// bytes of LDS a staging level needs for low-energy model L (the same walk
+// as stageTables)
+template <typename T>
+__host__ __device__ inline uint32_t ldsBytes(const Tables<T>& t, uint32_t level, int L)
+{
+    if (level <= STAGE_NONE)
+        return 0;
+    uint32_t b = 0;
+    if (L >= 1)
+        b += ldsAlign(uint64_t(t.nMaterials) * 4 * 56 * sizeof(T));
+    if (L == 1)
+        b += ldsAlign(uint64_t(t.nMaterials) * 63 * sizeof(T));
+    if (L == 2)
+        b += ldsAlign(uint64_t(t.nMaterials) * 12 * sizeof(Shell<T>));
+    b += ldsAlign(uint64_t(t.lutNodes) * 2 * sizeof(T));
+    b += sizeof(T) == 4 ? 2 * ldsAlign(uint64_t(t.lutNodes) * sizeof(float)) : ldsAlign(uint64_t(t.lutNodes) * sizeof(double));
+    b += ldsAlign(uint64_t(t.nSpectra + 1) * sizeof(uint32_t));
+    b += ldsAlign(uint64_t(t.nSpectra ? t.nSpectra : 1) * sizeof(uint32_t));
+    b += 2 * ldsAlign(uint64_t(t.specTotal) * sizeof(T)) + ldsAlign(uint64_t(t.specTotal) * sizeof(uint32_t));
+    b += ldsAlign(uint64_t(t.nHeel) * sizeof(Heel<T>)) + ldsAlign(uint64_t(t.heelWeightTotal) * sizeof(T));
+    b += ldsAlign(uint64_t(t.nBowtie + 1) * sizeof(uint32_t)) + 2 * ldsAlign(uint64_t(t.bowtieTotal) * sizeof(T));
+    if (level >= STAGE_ALL)
+        b += ldsAlign(uint64_t(t.nMaterials) * t.lutNodes * 6 * sizeof(T));
+    return b;
+}
+
+// a table's copy in LDS at the cursor, made by all threads of the block
+template <typename T>
+__device__ inline const T* stageArray(const T* src, uint64_t count, unsigned char*& cursor)
+{
+    static_assert(sizeof(T) % 4 == 0);
+    T* dst = reinterpret_cast<T*>(cursor);
+    const uint64_t words = count * sizeof(T) / 4;
+    const uint32_t* s = reinterpret_cast<const uint32_t*>(src);
+    uint32_t* d = reinterpret_cast<uint32_t*>(dst);
+    for (uint64_t i = threadIdx.x; i < words; i += blockDim.x)
+        d[i] = s[i];
+    cursor += ldsAlign(count * sizeof(T));
+    return dst;
+}
+
+// copies the tables into LDS and points t at the copies (all threads of the
+// block call it; ends with a barrier). The level is a template parameter so
+// that the compiler sees which pointers address LDS.
+template <typename T, uint32_t level, int L>
+__device__ inline void stageTables(Tables<T>& t, unsigned char* lds)
+{
+    if constexpr (level <= STAGE_NONE)
+        return;
+    unsigned char* c = lds;
+    if constexpr (L >= 1)
+        t.rita = stageArray(t.rita, uint64_t(t.nMaterials) * 4 * 56, c);
+    if constexpr (L == 1)
+        t.spline = stageArray(t.spline, uint64_t(t.nMaterials) * 63, c);
+    if constexpr (L == 2)
+        t.shells = stageArray(t.shells, uint64_t(t.nMaterials) * 12, c);
+    t.lutMajorant = stageArray(t.lutMajorant, uint64_t(t.lutNodes) * 2, c);
+    if constexpr (sizeof(T) == 4) {
+        t.lutBoundUp = stageArray(t.lutBoundUp, t.lutNodes, c);
+        t.lutAnchor = stageArray(t.lutAnchor, t.lutNodes, c);
+    } else {
+        t.lutGrid = stageArray(t.lutGrid, t.lutNodes, c);
+    }
+    t.specOffset = stageArray(t.specOffset, t.nSpectra + 1, c);
+    t.specThreshold = stageArray(t.specThreshold, t.nSpectra ? t.nSpectra : 1, c);
+    t.specProb = stageArray(t.specProb, t.specTotal, c);
+    t.specEnergy = stageArray(t.specEnergy, t.specTotal, c);
+    t.specAlias = stageArray(t.specAlias, t.specTotal, c);
+    t.heel = stageArray(t.heel, t.nHeel, c);
+    t.heelWeight = stageArray(t.heelWeight, t.heelWeightTotal, c);
+    t.bowtieOffset = stageArray(t.bowtieOffset, t.nBowtie + 1, c);
+    t.bowtieAngle = stageArray(t.bowtieAngle, t.bowtieTotal, c);
+    t.bowtieWeight = stageArray(t.bowtieWeight, t.bowtieTotal, c);
+    if constexpr (level >= STAGE_ALL)
+        t.lutCoef = stageArray(t.lutCoef, uint64_t(t.nMaterials) * t.lutNodes * 6, c);
+    __syncthreads();
+}
+
+// The wave's next histories from the launch's global counter: 'pool' at a
+// time, one atomic by lane 0. False when the launch has none left. The
+// bounds are wave-uniform and live in scalar registers.
+__device__ inline bool claimHistories(unsigned long long* next, uint32_t pool, uint64_t span, uint64_t hBegin, uint32_t lane, uint64_t& poolNext,
+    uint64_t& poolEnd)
+{
+    unsigned long long base = 0;
+    if (lane == 0)
+        base = atomicAdd(next, static_cast<unsigned long long>(pool));
+    base = __shfl(base, 0);
+    base = (static_cast<unsigned long long>(__builtin_amdgcn_readfirstlane(static_cast<uint32_t>(base >> 32))) << 32)
+        | __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(base));
+    if (base >= span)
+        return false;
+    poolNext = hBegin + base;
+    poolEnd = hBegin + (base + pool < span ? base + pool : span);
+    return true;
+}
+}

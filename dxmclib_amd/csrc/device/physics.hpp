@@ -538,18 +538,6 @@ __device__ inline bool transportToWorld(const World<T>& w, Particle<T>& p)
     return false;
 }
 
-template <typename T>
-__device__ inline uint64_t voxelIndex(const World<T>& w, const T* pos)
-{
-    uint32_t ix = static_cast<uint32_t>((pos[0] - w.extent[0]) / w.spacing[0]);
-    uint32_t iy = static_cast<uint32_t>((pos[1] - w.extent[2]) / w.spacing[1]);
-    uint32_t iz = static_cast<uint32_t>((pos[2] - w.extent[4]) / w.spacing[2]);
-    ix = ix < w.nx ? ix : w.nx - 1;
-    iy = iy < w.ny ? iy : w.ny - 1;
-    iz = iz < w.nz ? iz : w.nz - 1;
-    return (static_cast<uint64_t>(iz) * w.ny + iy) * w.nx + ix;
-}
-
 // safeValueAdd x3 (transport.hpp:208-214): hardware FP64 / u32 atomics
 __device__ inline void score(Scorer& sc, uint64_t idx, double e)
 {
@@ -892,37 +880,13 @@ __device__ inline bool computeInteractionsForced(const Tables<T>& t, T eventProb
     return true;
 }
 
-template <typename T>
-__device__ inline void readVoxel(const World<T>& w, uint64_t idx, uint32_t& mat, T& density, uint32_t& meas);
-
-template <>
-__device__ inline void readVoxel<double>(const World<double>& w, uint64_t idx, uint32_t& mat, double& density, uint32_t& meas)
-{
-    mat = w.material[idx];
-    density = w.density[idx];
-    meas = w.measurement ? w.measurement[idx] : 0u;
-}
-template <>
-__device__ inline void readVoxel<float>(const World<float>& w, uint64_t idx, uint32_t& mat, float& density, uint32_t& meas)
-{
-    uint2 v;
-    if (w.voxelBytes == 1)
-        v = w.palette[static_cast<const uint8_t*>(w.voxels)[idx]];
-    else if (w.voxelBytes == 2)
-        v = w.palette[static_cast<const uint16_t*>(w.voxels)[idx]];
-    else
-        v = static_cast<const uint2*>(w.voxels)[idx];
-    density = __uint_as_float(v.x);
-    mat = v.y & 0xffu;
-    meas = v.y >> 24;
-}
-
 // The FP32 record's material and measurement flag as they are stored,
 // material | measurement << 24 (the FP32 kernel keeps them in one register:
 // 24-bit products with the material, as the LUT row index, ignore the flag)
 // (the record is read as one 8-byte integer: read as a uint2 whose halves
 // are used apart, the compiler issues two 4-byte loads)
-__device__ inline void readVoxelPacked(const World<float>& w, uint32_t voxelBytes, uint64_t idx, uint32_t& matMeas, float& density)
+template <typename T>
+__device__ inline void readVoxelPacked(const World<T>& w, uint32_t voxelBytes, uint64_t idx, uint32_t& matMeas, float& density)
 {
     const uint64_t* rec = reinterpret_cast<const uint64_t*>(w.palette);
     uint64_t v;
@@ -934,59 +898,5 @@ __device__ inline void readVoxelPacked(const World<float>& w, uint32_t voxelByte
         v = static_cast<const uint64_t*>(w.voxels)[idx];
     density = __uint_as_float(static_cast<uint32_t>(v));
     matMeas = static_cast<uint32_t>(v >> 32);
-}
-
-// One Woodcock delta-tracking step (body of the loop in transport.hpp:650-699):
-// refresh the majorant after an energy change, fly an exponential distance
-// under the majorant, then a real or virtual interaction in the voxel
-// reached, then Russian roulette. Returns false when the photon is gone.
-template <typename T, int L>
-__device__ inline bool woodcockStep(const World<T>& w, const Tables<T>& t, Particle<T>& p, T& majInv, bool& update, Rng& rng, Scorer& sc,
-    uint32_t& steps)
-{
-    if (update) {
-        majInv = majorantInverse(t, p.energy);
-        update = false;
-    }
-    const T r1 = rng.uniform<T>();
-    const T step = -log(r1) * majInv * T(10); // cm -> mm
-    for (int i = 0; i < 3; ++i)
-        p.pos[i] += p.dir[i] * step;
-    if (!inside(w, p.pos))
-        return false;
-    ++steps;
-    const uint64_t idx = voxelIndex(w, p.pos);
-    uint32_t mat, meas;
-    T density;
-    readVoxel(w, idx, mat, density, meas);
-    T att[3];
-    attenuation(t, mat, p.energy, att);
-    const T prob = ((att[0] + att[1]) + att[2]) * density * majInv;
-    bool alive = true;
-    if (meas == 0) {
-        const T r2 = rng.uniform<T>();
-        if (r2 < prob)
-            alive = computeInteractions<T, L>(t, att, p, mat, sc, idx, rng, update);
-    } else {
-        alive = computeInteractionsForced<T, L>(t, prob, att, p, mat, sc, idx, rng, update);
-    }
-    if (alive && p.energy * p.weight < T(5)) { // Russian roulette
-        const T r4 = rng.uniform<T>();
-        if (r4 < T(0.8))
-            alive = false;
-        else
-            p.weight *= T(1) / (T(1) - T(0.8));
-    }
-    return alive;
-}
-
-// Woodcock tracking of one photon until it leaves the world, is absorbed or
-// is killed by Russian roulette (transport.hpp:640-700).
-template <typename T, int L>
-__device__ inline void woodcock(const World<T>& w, const Tables<T>& t, Particle<T>& p, Rng& rng, Scorer& sc, uint32_t& steps)
-{
-    T majInv = 0;
-    bool update = true;
-    for (uint32_t n = 0; n < MAX_STEPS && woodcockStep<T, L>(w, t, p, majInv, update, rng, sc, steps); ++n) { }
 }
 }

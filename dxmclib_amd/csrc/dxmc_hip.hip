@@ -2,17 +2,16 @@
 // the C ABI declared in include/dxmc_hip.h.
 //
 // Kernels in this file:
-//   transportPlain<T,L>   one thread per history (the plain method for
-//                         T = double; also instantiated for float)
 //   rngStreams            PCG32 stream dump (parity)
 //   lutLookup<T>          attenuation + majorant lookups (parity)
 //   interact<T,L>         single interactions (parity)
 //   sampleParticles<T>    source sampling + world entry (parity)
 //   normalizeTally        FP64 normalisation (eV/history or dose)
-// The persistent FP32 transport kernel lives in transport_fp32.hip.
+// The persistent transport kernels live in transport_fp32.hip and
+// transport_fp64.hip.
 //
 // This file is compiled without FMA contraction (-ffp-contract=off) so the
-// FP64 path rounds like the CPU oracle.
+// FP64 entry points round like the CPU oracle.
 #include "dxmc_hip.h"
 #include "internal.hpp"
 
@@ -32,25 +31,6 @@ using namespace dxmc_backend;
 namespace {
 
 // ---------------------------------------------------------------- kernels
-
-template <typename T, int L>
-__global__ __launch_bounds__(256) void transportPlain(World<T> w, Tables<T> t, const Exposure<T>* exps, const uint64_t* expStart,
-    uint32_t nExp, uint64_t hBegin, uint64_t hEnd, uint64_t seed, uint64_t firstHistory, Tally tally, Counters* ctr)
-{
-    const uint64_t h = hBegin + static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-    Scorer sc { tally, 0 };
-    uint32_t steps = 0;
-    if (h < hEnd) {
-        const uint32_t e = upperBound(expStart, nExp + 1, h) - 1;
-        Rng rng = Rng::forHistory(seed, firstHistory + h);
-        Particle<T> p;
-        sampleParticle(exps[e], t, rng, p);
-        if (transportToWorld(w, p))
-            woodcock<T, L>(w, t, p, rng, sc, steps);
-    }
-    if (ctr)
-        accumulateCounters(ctr, steps, sc.events);
-}
 
 __global__ void rngStreams(uint64_t seed, uint64_t first, uint64_t n, uint32_t draws, uint32_t* out)
 {
@@ -243,26 +223,6 @@ __host__ __device__ Exposure<T> toDevice(const dxmc_exposure& e)
     x.bowtie = e.bowtie;
     x.pad = 0;
     return x;
-}
-
-template <typename T, int L>
-void launchPlain(const World<T>& w, const Tables<T>& t, const Exposure<T>* exps, const uint64_t* expStart, uint32_t nExp, uint64_t hb, uint64_t he,
-    uint64_t seed, uint64_t first, const Tally& tally, Counters* ctr, uint32_t block, hipStream_t s)
-{
-    const uint64_t n = he - hb;
-    hipLaunchKernelGGL((transportPlain<T, L>), dim3(gridFor(n, block)), dim3(block), 0, s, w, t, exps, expStart, nExp, hb, he, seed, first, tally, ctr);
-}
-
-template <typename T>
-void launchPlainL(int L, const World<T>& w, const Tables<T>& t, const Exposure<T>* exps, const uint64_t* expStart, uint32_t nExp, uint64_t hb,
-    uint64_t he, uint64_t seed, uint64_t first, const Tally& tally, Counters* ctr, uint32_t block, hipStream_t s)
-{
-    if (L == 0)
-        launchPlain<T, 0>(w, t, exps, expStart, nExp, hb, he, seed, first, tally, ctr, block, s);
-    else if (L == 1)
-        launchPlain<T, 1>(w, t, exps, expStart, nExp, hb, he, seed, first, tally, ctr, block, s);
-    else
-        launchPlain<T, 2>(w, t, exps, expStart, nExp, hb, he, seed, first, tally, ctr, block, s);
 }
 
 template <typename T>
@@ -840,10 +800,9 @@ int runLaunches(dxmc_ctx* c, const dxmc_world* w, const dxmc_tables* t, uint64_t
     tally->arraysCurrent = false;
     uint64_t chunk = cfg.histories_per_launch;
     if (chunk == 0)
-        chunk = cfg.precision == DXMC_PRECISION_FP64 ? (uint64_t(1) << 22) : (uint64_t(1) << 27);
-    // the FP32 kernel keeps a history's offset in its launch in 32 bits
-    if (cfg.precision != DXMC_PRECISION_FP64)
-        chunk = std::min<uint64_t>(chunk, uint64_t(1) << 32);
+        chunk = cfg.precision == DXMC_PRECISION_FP64 ? (uint64_t(1) << 25) : (uint64_t(1) << 27);
+    // the kernels keep a history's offset in its launch in 32 bits
+    chunk = std::min<uint64_t>(chunk, uint64_t(1) << 32);
     const uint32_t block = cfg.block_size ? cfg.block_size : 256;
     if (block % 64 != 0 || block > 256)
         return c->fail(DXMC_ERR_ARGUMENT, "run: block size must be a multiple of 64 up to 256");
@@ -860,8 +819,7 @@ int runLaunches(dxmc_ctx* c, const dxmc_world* w, const dxmc_tables* t, uint64_t
         const uint64_t he = std::min(in.total, hb + chunk);
         DXMC_CHECK(c, hipEventRecord(c->ev0, c->stream));
         if (cfg.precision == DXMC_PRECISION_FP64)
-            launchPlainL<double>(cfg.low_energy_correction, w64, t->f64, in.exp64, in.startDev, static_cast<uint32_t>(nExp), hb, he, cfg.seed,
-                cfg.first_history, tl, in.ctr, block, c->stream);
+            launchFp64(c, cfg, w64, t->f64, t->f32, in.exp64, in.startDev, static_cast<uint32_t>(nExp), hb, he, tl, in.ctr, in.historyCounter);
         else
             launchFp32(c, cfg, w32, t->f32, in.exp32, in.startDev, static_cast<uint32_t>(nExp), hb, he, tl, in.ctr, in.historyCounter);
         DXMC_CHECK(c, hipGetLastError());

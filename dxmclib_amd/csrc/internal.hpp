@@ -415,4 +415,9 @@ int noallocScratch(int device, void** out);
 void launchFp32(dxmc_ctx* c, const dxmc_run_cfg& cfg, const dxmc_dev::World<float>& w, const dxmc_dev::Tables<float>& t,
     const dxmc_dev::Exposure<float>* exps, const uint64_t* expStart, uint32_t nExp, uint64_t hb, uint64_t he, const dxmc_dev::Tally& tally,
     dxmc_dev::Counters* ctr, unsigned long long* historyCounter);
+// FP64 transport launch (transport_fp64.hip); t32: the FP32 copy of the tables,
+// whose attenuation bounds and coefficients filter the FP64 decisions
+void launchFp64(dxmc_ctx* c, const dxmc_run_cfg& cfg, const dxmc_dev::World<double>& w, const dxmc_dev::Tables<double>& t,
+    const dxmc_dev::Tables<float>& t32, const dxmc_dev::Exposure<double>* exps, const uint64_t* expStart, uint32_t nExp, uint64_t hb, uint64_t he,
+    const dxmc_dev::Tally& tally, dxmc_dev::Counters* ctr, unsigned long long* historyCounter);
 }

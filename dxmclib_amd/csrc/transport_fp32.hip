@@ -34,149 +34,19 @@
 // each scoring event is added to the FP64 tallies with hardware FP64
 // atomics. The kernel is compiled per low-energy model, register budget
 // (5, 6 or 7 waves per SIMD), LDS staging level and world kind.
+#include "device/persistent.hpp"
 #include "internal.hpp"
 
 using namespace dxmc_dev;
 
 namespace {
 
-enum : uint32_t { DEAD = 0, FLYING = 1, PENDING = 2 };
-
-// World kinds the kernel is compiled for: the two common layouts get their
-// code width, record width, 24-bit index and bounds table fixed at compile
-// time, so a flight carries no branches on them
-//   WORLD_CODES8    1-byte bounded-density codes (and their block codes
-//                   when the run uses them), 8-byte records, the
-//                   attenuation bounds table, 24-bit index (CT-sized worlds)
-//   WORLD_PALETTE8  1-byte palette indices, no codes, 24-bit index
-//   WORLD_ANY       every other world (branches at run time)
-enum : uint32_t { WORLD_ANY = 0, WORLD_CODES8 = 1, WORLD_PALETTE8 = 2 };
-
-
-__device__ inline uint32_t rankBelow(uint64_t mask)
-{
-    return __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(mask >> 32), __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(mask), 0u));
-}
-
-// voxel index with the reciprocal spacing (FP32 path), kept inside the grid
-// (the float-to-unsigned conversion clamps negative values to 0); with
-// 24-bit products where the grid allows (the compiler turns a 24-bit
-// multiply-add into a 64-bit one, so the three terms are summed instead)
+// voxel coordinates with the reciprocal spacing (FP32 path), kept inside the
+// grid (the float-to-unsigned conversion clamps negative values to 0)
 __device__ inline uint3 voxelCoordsFast(const World<float>& w, const float* pos, const float* inv)
 {
     return make_uint3(min(static_cast<uint32_t>((pos[0] - w.extent[0]) * inv[0]), w.nx - 1),
         min(static_cast<uint32_t>((pos[1] - w.extent[2]) * inv[1]), w.ny - 1), min(static_cast<uint32_t>((pos[2] - w.extent[4]) * inv[2]), w.nz - 1));
-}
-
-__device__ inline uint64_t voxelIndexFast(const World<float>& w, uint3 v, bool index24)
-{
-    if (index24)
-        return __umul24(v.z, w.nxy) + __umul24(v.y, w.nx) + v.x;
-    return (static_cast<uint64_t>(v.z) * w.ny + v.y) * w.nx + v.x;
-}
-
-// element 'index' of a table addressed by a 32-bit byte offset from its
-// base (tables below 4 GiB): the load takes the base from scalar registers
-// and the offset from one vector register, with no 64-bit address
-// arithmetic per lane
-template <typename T>
-__device__ inline T loadAt(const T* base, uint32_t index)
-{
-    return *reinterpret_cast<const T*>(reinterpret_cast<const unsigned char*>(base) + index * static_cast<uint32_t>(sizeof(T)));
-}
-
-// block of a voxel (1-byte code worlds: 24-bit products hold)
-__device__ inline uint32_t blockIndexFast(const World<float>& w, uint3 v)
-{
-    return __umul24(v.z >> w.blockShift, w.bnxy) + __umul24(v.y >> w.blockShift, w.bnx) + (v.x >> w.blockShift);
-}
-
-// ------------------------------------------------------ LDS-staged tables
-// The tables the samplers read with data-dependent indices (RITA, spline,
-// shells, spectrum alias tables, heel and bowtie filters, the majorant and
-// the segment bounds, optionally the attenuation coefficients) are copied
-// into LDS at kernel start, one copy per block: their lookups then cost LDS
-// latency instead of L2 latency, also while the world gathers keep evicting
-// them from L1. Staging level: 1 none, 2 all but the attenuation
-// coefficients, 3 all. Of the interaction tables only those of the run's
-// low-energy model are staged (RITA for L >= 1, the scatter-function spline
-// for L = 1, the shells for L = 2). The total-attenuation bounds stay in
-// global memory: in LDS they cost a resident block per CU.
-enum : uint32_t { STAGE_NONE = 1, STAGE_SMALL = 2, STAGE_ALL = 3 };
-
-__host__ __device__ constexpr uint32_t ldsAlign(uint64_t bytes) { return static_cast<uint32_t>((bytes + 15) & ~uint64_t(15)); }
-
-// bytes of LDS a staging level needs for low-energy model L (the same walk
-// as stageTables)
-__host__ __device__ inline uint32_t ldsBytes(const Tables<float>& t, uint32_t level, int L)
-{
-    if (level <= STAGE_NONE)
-        return 0;
-    uint32_t b = 0;
-    if (L >= 1)
-        b += ldsAlign(uint64_t(t.nMaterials) * 4 * 56 * sizeof(float));
-    if (L == 1)
-        b += ldsAlign(uint64_t(t.nMaterials) * 63 * sizeof(float));
-    if (L == 2)
-        b += ldsAlign(uint64_t(t.nMaterials) * 12 * sizeof(Shell<float>));
-    b += ldsAlign(uint64_t(t.lutNodes) * 2 * sizeof(float));
-    b += ldsAlign(uint64_t(t.lutNodes) * sizeof(float));
-    b += ldsAlign(uint64_t(t.lutNodes) * sizeof(float));
-    b += ldsAlign(uint64_t(t.nSpectra + 1) * sizeof(uint32_t));
-    b += ldsAlign(uint64_t(t.nSpectra ? t.nSpectra : 1) * sizeof(uint32_t));
-    b += 2 * ldsAlign(uint64_t(t.specTotal) * sizeof(float)) + ldsAlign(uint64_t(t.specTotal) * sizeof(uint32_t));
-    b += ldsAlign(uint64_t(t.nHeel) * sizeof(Heel<float>)) + ldsAlign(uint64_t(t.heelWeightTotal) * sizeof(float));
-    b += ldsAlign(uint64_t(t.nBowtie + 1) * sizeof(uint32_t)) + 2 * ldsAlign(uint64_t(t.bowtieTotal) * sizeof(float));
-    if (level >= STAGE_ALL)
-        b += ldsAlign(uint64_t(t.nMaterials) * t.lutNodes * 6 * sizeof(float));
-    return b;
-}
-
-template <typename T>
-__device__ inline const T* stageArray(const T* src, uint64_t count, unsigned char*& cursor)
-{
-    static_assert(sizeof(T) % 4 == 0);
-    T* dst = reinterpret_cast<T*>(cursor);
-    const uint64_t words = count * sizeof(T) / 4;
-    const uint32_t* s = reinterpret_cast<const uint32_t*>(src);
-    uint32_t* d = reinterpret_cast<uint32_t*>(dst);
-    for (uint64_t i = threadIdx.x; i < words; i += blockDim.x)
-        d[i] = s[i];
-    cursor += ldsAlign(count * sizeof(T));
-    return dst;
-}
-
-// copies the tables into LDS and points t at the copies (all threads of the
-// block call it; ends with a barrier). The level is a template parameter so
-// that the compiler sees which pointers address LDS.
-template <uint32_t level, int L>
-__device__ inline void stageTables(Tables<float>& t, unsigned char* lds)
-{
-    if constexpr (level <= STAGE_NONE)
-        return;
-    unsigned char* c = lds;
-    if constexpr (L >= 1)
-        t.rita = stageArray(t.rita, uint64_t(t.nMaterials) * 4 * 56, c);
-    if constexpr (L == 1)
-        t.spline = stageArray(t.spline, uint64_t(t.nMaterials) * 63, c);
-    if constexpr (L == 2)
-        t.shells = stageArray(t.shells, uint64_t(t.nMaterials) * 12, c);
-    t.lutMajorant = stageArray(t.lutMajorant, uint64_t(t.lutNodes) * 2, c);
-    t.lutBoundUp = stageArray(t.lutBoundUp, t.lutNodes, c);
-    t.lutAnchor = stageArray(t.lutAnchor, t.lutNodes, c);
-    t.specOffset = stageArray(t.specOffset, t.nSpectra + 1, c);
-    t.specThreshold = stageArray(t.specThreshold, t.nSpectra ? t.nSpectra : 1, c);
-    t.specProb = stageArray(t.specProb, t.specTotal, c);
-    t.specEnergy = stageArray(t.specEnergy, t.specTotal, c);
-    t.specAlias = stageArray(t.specAlias, t.specTotal, c);
-    t.heel = stageArray(t.heel, t.nHeel, c);
-    t.heelWeight = stageArray(t.heelWeight, t.heelWeightTotal, c);
-    t.bowtieOffset = stageArray(t.bowtieOffset, t.nBowtie + 1, c);
-    t.bowtieAngle = stageArray(t.bowtieAngle, t.bowtieTotal, c);
-    t.bowtieWeight = stageArray(t.bowtieWeight, t.bowtieTotal, c);
-    if constexpr (level >= STAGE_ALL)
-        t.lutCoef = stageArray(t.lutCoef, uint64_t(t.nMaterials) * t.lutNodes * 6, c);
-    __syncthreads();
 }
 
 constexpr float LN2F = 0.693147180559945309f;
@@ -193,13 +63,6 @@ constexpr int QUEUE_FIELDS = 12;
 // launch passes (48, or less where the staged tables are larger)
 __host__ __device__ constexpr uint32_t queueBytes(uint32_t capacity) { return QUEUE_FIELDS * capacity * 4; }
 constexpr uint32_t WAVES_PER_BLOCK = 4;
-
-// inside the safe extent, without short-circuit branches
-__device__ inline bool insideFast(const World<float>& w, const float* pos)
-{
-    return (pos[0] > w.extent[0]) & (pos[0] < w.extent[1]) & (pos[1] > w.extent[2]) & (pos[1] < w.extent[3]) & (pos[2] > w.extent[4])
-        & (pos[2] < w.extent[5]);
-}
 
 // Russian roulette after a step that left the photon alive (transport.hpp:684-694)
 __device__ inline bool roulette(Particle<float>& p, Rng& rng)
@@ -224,7 +87,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(W, 8))) voi
 {
     extern __shared__ __align__(16) unsigned char lds[];
     Tables<float> t = tg;
-    stageTables<S, L>(t, lds);
+    stageTables<float, S, L>(t, lds);
     Particle<float> p;
     Rng rng { 0, 1 };
     float majInv = 0;
@@ -283,19 +146,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(W, 8))) voi
                 if (poolNext >= poolEnd) {
                     if (claimedAll)
                         break;
-                    unsigned long long base = 0;
-                    if (lane == 0)
-                        base = atomicAdd(next, static_cast<unsigned long long>(poolSize));
-                    base = __shfl(base, 0);
-                    // wave-uniform: the pool bounds live in scalar registers
-                    base = (static_cast<unsigned long long>(__builtin_amdgcn_readfirstlane(static_cast<uint32_t>(base >> 32))) << 32)
-                        | __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(base));
-                    if (base >= span) {
+                    if (!claimHistories(next, poolSize, span, hBegin, lane, poolNext, poolEnd)) {
                         claimedAll = true;
                         break;
                     }
-                    poolNext = hBegin + base;
-                    poolEnd = hBegin + (base + poolSize < span ? base + poolSize : span);
                     if (poolEnd == hEnd)
                         claimedAll = true;
                     poolExp = upperBound(expStart, nExp + 1, poolNext) - 1;
@@ -682,11 +536,11 @@ void launchFp32(dxmc_ctx* c, const dxmc_run_cfg& cfg, const World<float>& w, con
     // spiral 2.39e9 at 20, 2.49e9 at 28, 2.52e9 at 32, 2.45e9 at 40; at
     // L = 1, 32 cost 3 % and 24 0.5 %)
     const uint32_t interact = cfg.interaction_threshold ? std::min<uint32_t>(cfg.interaction_threshold, 64u) : cfg.low_energy_correction == 2 ? 32u : 20u;
-    // histories a wave claims per atomic on the global counter
-    const uint32_t pool = cfg.queue_depth ? std::clamp<uint32_t>(cfg.queue_depth, 64u, 1u << 16) : 512u;
     uint64_t grid = static_cast<uint64_t>(c->numCU) * perCU;
     const uint64_t lanesNeeded = (he - hb + 63) / 64 * 64;
     grid = std::max<uint64_t>(1, std::min<uint64_t>(grid, (lanesNeeded + block - 1) / block));
+    // histories a wave claims per atomic on the global counter
+    const uint32_t pool = cfg.queue_depth ? std::clamp<uint32_t>(cfg.queue_depth, 64u, 1u << 16) : 512u;
     hipLaunchKernelGGL(kernelFor(cfg.low_energy_correction, waves, stage, kind), dim3(static_cast<uint32_t>(grid)), dim3(block), lds, c->stream, world, tables,
         exps, expStart, nExp, hb, he, cfg.seed, cfg.first_history, tally, ctr, nx, regen, interact, pool, cap);
 }

@@ -42,7 +42,7 @@ enum dxmc_status {
 };
 
 enum dxmc_precision {
-    DXMC_PRECISION_FP64 = 0, /* plain method: FP64 throughout, one thread per history */
+    DXMC_PRECISION_FP64 = 0, /* plain method: every value that decides a history in FP64 */
     DXMC_PRECISION_FP32 = 1 /* FP32 transport, persistent kernel, FP64 tallies */
 };
 
@@ -209,7 +209,7 @@ typedef struct {
     int32_t low_energy_correction; /* 0 NONE, 1 LIVERMORE, 2 IA (lowenergycorrectionmodel.hpp) */
     uint64_t seed; /* history h uses state1 = 2h+1, state0 = splitmix64(seed ^ splitmix64(h)) */
     uint64_t first_history; /* global index of the first history of exposure 0 */
-    uint64_t histories_per_launch; /* 0: automatic; bounds cancel/progress latency; FP32 at most 2^32 */
+    uint64_t histories_per_launch; /* 0: automatic; bounds cancel/progress latency; at most 2^32 */
     uint32_t block_size; /* 0: tuned default */
     uint32_t blocks_per_cu; /* FP32 persistent kernel occupancy, 0: tuned default */
     uint32_t regeneration_threshold; /* FP32: dead lanes per wave before they take queued new photons, 0: tuned */
@@ -229,7 +229,7 @@ typedef struct {
 /* dxmc_run_cfg.flags */
 #define DXMC_RUN_COUNTERS 1u /* collect step/event counters */
 #define DXMC_RUN_AUTOTUNE 2u /* fill zero tuning fields from the autotuner (tuned once per world/tables/precision/L and kept in the context) */
-#define DXMC_RUN_EXACT_STEPS 4u /* FP32: evaluate every Woodcock step from the voxel record and the full attenuation, without the bounds that settle most steps (same results, for checks) */
+#define DXMC_RUN_EXACT_STEPS 4u /* evaluate every Woodcock step from the voxel and the full attenuation (in the run's precision), without the bounds that settle most steps (same results, for checks) */
 
 typedef struct {
     uint64_t histories; /* histories started */
