@@ -16,9 +16,14 @@ enum : uint32_t { DEAD = 0, FLYING = 1, PENDING = 2 };
 //   WORLD_CODES8    1-byte bounded-density codes (and their block codes
 //                   when the run uses them), 8-byte records, the
 //                   attenuation bounds table, 24-bit index (CT-sized worlds)
-//   WORLD_PALETTE8  1-byte palette indices, no codes, 24-bit index
+//   WORLD_PALETTE8  1-byte palette indices, no codes, no measurement flags,
+//                   24-bit index
+//   WORLD_PALETTE8_MEASURED  the same with measurement flags (forced events)
 //   WORLD_ANY       every other world (branches at run time)
-enum : uint32_t { WORLD_ANY = 0, WORLD_CODES8 = 1, WORLD_PALETTE8 = 2 };
+enum : uint32_t { WORLD_ANY = 0, WORLD_CODES8 = 1, WORLD_PALETTE8 = 2, WORLD_PALETTE8_MEASURED = 3 };
+// kinds whose voxels may carry a measurement flag
+__host__ __device__ constexpr bool kindForces(uint32_t kind) { return kind == WORLD_ANY || kind == WORLD_PALETTE8_MEASURED; }
+__host__ __device__ constexpr bool kindPalette8(uint32_t kind) { return kind == WORLD_PALETTE8 || kind == WORLD_PALETTE8_MEASURED; }
 
 __device__ inline uint32_t rankBelow(uint64_t mask)
 {
@@ -171,5 +176,46 @@ __device__ inline bool claimHistories(unsigned long long* next, uint32_t pool, u
     poolNext = hBegin + base;
     poolEnd = hBegin + (base + pool < span ? base + pool : span);
     return true;
+}
+
+// Adds one score per lane that has one to the tally; the whole wave calls it.
+// Atomics cost a request per cache line, so the scores are packed into the
+// wave's first lanes (one permutation) and added 16 at a time, the four lanes
+// of a group to the dose, the variance and the event count of one voxel.
+// wide: voxel indices may exceed 32 bits.
+template <typename T>
+__device__ inline void scoreWave(const Tally& tally, bool has, uint64_t idx, T e, bool wide)
+{
+    const uint64_t mask = __ballot(has);
+    const uint32_t n = __popcll(mask);
+    if (n == 0)
+        return;
+    const uint32_t lane = __lane_id();
+    const int to = static_cast<int>(4 * (has ? rankBelow(mask) : n + rankBelow(~mask)));
+    auto move = [&](uint32_t v) { return __builtin_amdgcn_ds_permute(to, static_cast<int>(v)); };
+    const int lo = move(static_cast<uint32_t>(idx));
+    const int hi = wide ? move(static_cast<uint32_t>(idx >> 32)) : 0;
+    int e0, e1 = 0;
+    if constexpr (sizeof(T) == 4) {
+        e0 = move(__float_as_uint(e));
+    } else {
+        e0 = move(static_cast<uint32_t>(__double2loint(e)));
+        e1 = move(static_cast<uint32_t>(__double2hiint(e)));
+    }
+    const uint32_t field = lane & 3u;
+    for (uint32_t base = 0; base < n; base += 16) {
+        const uint32_t slot = base + lane / 4;
+        const int from = static_cast<int>(4 * slot);
+        const uint32_t vLo = static_cast<uint32_t>(__builtin_amdgcn_ds_bpermute(from, lo));
+        const uint32_t vHi = wide ? static_cast<uint32_t>(__builtin_amdgcn_ds_bpermute(from, hi)) : 0u;
+        double v;
+        if constexpr (sizeof(T) == 4)
+            v = static_cast<double>(__uint_as_float(static_cast<uint32_t>(__builtin_amdgcn_ds_bpermute(from, e0))));
+        else
+            v = __hiloint2double(__builtin_amdgcn_ds_bpermute(from, e1), __builtin_amdgcn_ds_bpermute(from, e0));
+        const double add = field == 0 ? v : field == 1 ? v * v : 1.0;
+        if (slot < n && field < 3)
+            unsafeAtomicAdd(reinterpret_cast<double*>(tally.voxels + (static_cast<uint64_t>(vHi) << 32 | vLo)) + field, add);
+    }
 }
 }

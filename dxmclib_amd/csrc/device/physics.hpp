@@ -176,16 +176,18 @@ constexpr uint32_t MIXED_CODE = 255; // the 1-byte code kept for mixed blocks
 constexpr uint16_t BLOCK_MIXED = MIXED_CODE; // smallest code 255, largest 0
 constexpr uint32_t CODE_MUL_SHIFT = 20;
 
-// One voxel's accumulators in 32 aligned bytes: the three atomics of a
-// scoring event land in one cache line (separate arrays cost three random
-// lines per event). Normalisation and download write the per-voxel arrays
-// of Result from these.
+// One voxel's accumulators in 32 aligned bytes. Atomics cost one request per
+// cache line a wave instruction touches, not one per lane (measured: 2.4e10
+// requests/s, whether a request carries one double or four adjacent ones), so
+// the event count is a double too (exact below 2^53): one instruction adds a
+// score's three sums through adjacent lanes (scoreWave). As three atomics a
+// score cost three requests. Normalisation and download write the per-voxel
+// arrays of Result from these.
 struct alignas(32) VoxelScore {
     double dose; // energy imparted, eV x weight
     double variance; // sum of squares of the same
-    uint32_t events;
-    uint32_t pad0;
-    uint64_t pad1;
+    double events; // whole number
+    double pad;
 };
 static_assert(sizeof(VoxelScore) == 32, "one voxel score is 32 bytes");
 
@@ -193,10 +195,20 @@ struct Tally {
     VoxelScore* voxels;
 };
 
-// tally plus this thread's event counter
-struct Scorer {
-    Tally tally;
-    uint32_t events;
+// energies imparted by one interaction of a photon (two when forced: the
+// virtual photoabsorption and a Compton event), added to the tally afterwards
+template <typename T>
+struct Deposits {
+    T first = 0, second = 0;
+    uint32_t n = 0;
+    __device__ inline void add(T e)
+    {
+        if (n == 0)
+            first = e;
+        else
+            second = e;
+        ++n;
+    }
 };
 
 struct Counters {
@@ -538,14 +550,13 @@ __device__ inline bool transportToWorld(const World<T>& w, Particle<T>& p)
     return false;
 }
 
-// safeValueAdd x3 (transport.hpp:208-214): hardware FP64 / u32 atomics
-__device__ inline void score(Scorer& sc, uint64_t idx, double e)
+// one score (safeValueAdd x3, transport.hpp:208-214): hardware FP64 atomics
+__device__ inline void score(const Tally& tally, uint64_t idx, double e)
 {
-    VoxelScore* v = sc.tally.voxels + idx;
+    VoxelScore* v = tally.voxels + idx;
     unsafeAtomicAdd(&v->dose, e);
-    atomicAdd(&v->events, 1u);
     unsafeAtomicAdd(&v->variance, e * e);
-    ++sc.events;
+    unsafeAtomicAdd(&v->events, 1.0);
 }
 
 // -------------------------------------------------------------- interactions
@@ -823,37 +834,33 @@ __device__ inline void rayleighScatter(const Tables<T>& t, Particle<T>& p, uint3
 // Energy imparted by an event, with the 1 keV cutoff: below it the photon is
 // absorbed and its remaining energy is added (transport.hpp:596-611).
 template <typename T>
-__device__ inline bool depositAfterEvent(Scorer& sc, uint64_t idx, Particle<T>& p, T e, bool& updateMajorant)
+__device__ inline bool depositAfterEvent(Deposits<T>& d, Particle<T>& p, T e, bool& updateMajorant)
 {
     if (p.energy < T(1)) {
-        const T ei = (e + p.energy) * p.weight;
-        score(sc, idx, static_cast<double>(ei));
+        d.add((e + p.energy) * p.weight);
         p.energy = 0;
         return false;
     }
-    const T ei = e * p.weight;
-    score(sc, idx, static_cast<double>(ei));
+    d.add(e * p.weight);
     updateMajorant = true;
     return true;
 }
 
 template <typename T, int L>
-__device__ inline bool computeInteractions(const Tables<T>& t, const T att[3], Particle<T>& p, uint32_t mat, Scorer& sc, uint64_t idx,
+__device__ inline bool computeInteractions(const Tables<T>& t, const T att[3], Particle<T>& p, uint32_t mat, Deposits<T>& d,
     Rng& rng, bool& updateMajorant)
 {
     const T total = (att[0] + att[1]) + att[2];
     const T r3 = rng.uniform<T>(total);
-    // one scoring call site for photoabsorption and Compton (a wave whose
-    // lanes hold both runs the atomics once)
     const bool photo = r3 < att[0];
     const bool compton = !photo && r3 < (att[0] + att[1]);
     const T e = photo ? photoAbsorption<T, L>(t, p, mat, rng) : scatterEvent<T, L>(t, p, mat, rng, compton);
-    return (photo || compton) ? depositAfterEvent(sc, idx, p, e, updateMajorant) : true;
+    return (photo || compton) ? depositAfterEvent(d, p, e, updateMajorant) : true;
 }
 
 template <typename T, int L>
 __device__ inline bool computeInteractionsForced(const Tables<T>& t, T eventProbability, const T att[3], Particle<T>& p, uint32_t mat,
-    Scorer& sc, uint64_t idx, Rng& rng, bool& updateMajorant)
+    Deposits<T>& d, Rng& rng, bool& updateMajorant)
 {
     const T total = (att[0] + att[1]) + att[2];
     const T photoProbability = att[0] / total;
@@ -866,14 +873,14 @@ __device__ inline bool computeInteractionsForced(const Tables<T>& t, T eventProb
             ei = (ef + pf.energy) * pf.weight * weightCorrection;
         else
             ei = ef * pf.weight * weightCorrection;
-        score(sc, idx, static_cast<double>(ei));
+        d.add(ei);
     }
     const T r1 = rng.uniform<T>();
     if (r1 < eventProbability * (1 - photoProbability)) {
         const T r2 = rng.uniform<T>(att[1] + att[2]);
         const bool compton = r2 < att[1];
         const T e = scatterEvent<T, L>(t, p, mat, rng, compton);
-        if (compton && !depositAfterEvent(sc, idx, p, e, updateMajorant))
+        if (compton && !depositAfterEvent(d, p, e, updateMajorant))
             return false;
     }
     p.weight *= (1 - weightCorrection);

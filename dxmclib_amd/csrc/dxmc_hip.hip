@@ -74,7 +74,7 @@ __global__ void interact(Tables<T> t, int kind, uint64_t n, const uint32_t* mat,
     p.weight = static_cast<T>(q[7]);
     T e = 0;
     int alive = 1;
-    Scorer sc { tally, 0 };
+    Deposits<T> deposits;
     bool update = false;
     if (kind == 0)
         e = photoAbsorption<T, L>(t, p, mat[i], rng);
@@ -86,10 +86,14 @@ __global__ void interact(Tables<T> t, int kind, uint64_t n, const uint32_t* mat,
         T att[3];
         attenuation(t, mat[i], p.energy, att);
         if (kind == 3)
-            alive = computeInteractions<T, L>(t, att, p, mat[i], sc, i, rng, update) ? 1 : 0;
+            alive = computeInteractions<T, L>(t, att, p, mat[i], deposits, rng, update) ? 1 : 0;
         else
-            alive = computeInteractionsForced<T, L>(t, static_cast<T>(forcedProbability), att, p, mat[i], sc, i, rng, update) ? 1 : 0;
+            alive = computeInteractionsForced<T, L>(t, static_cast<T>(forcedProbability), att, p, mat[i], deposits, rng, update) ? 1 : 0;
     }
+    if (deposits.n > 0)
+        score(tally, i, static_cast<double>(deposits.first));
+    if (deposits.n > 1)
+        score(tally, i, static_cast<double>(deposits.second));
     for (int k = 0; k < 3; ++k) {
         q[k] = static_cast<double>(p.pos[k]);
         q[3 + k] = static_cast<double>(p.dir[k]);
@@ -129,7 +133,7 @@ __global__ void normalizeTally(const VoxelScore* __restrict__ scores, double* __
     if (i >= n)
         return;
     const VoxelScore v = scores[i];
-    events[i] = v.events;
+    events[i] = static_cast<uint32_t>(static_cast<uint64_t>(v.events));
     if (mode < 0) {
         dose[i] = v.dose;
         variance[i] = v.variance;

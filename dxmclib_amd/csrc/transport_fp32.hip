@@ -98,7 +98,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(W, 8))) voi
     uint64_t poolNext = 0, poolEnd = 0;
     uint32_t poolExp = 0;
     bool claimedAll = span == 0;
-    Scorer sc { tally, 0 };
+    uint32_t events = 0; // scoring events of the lane's interactions
     // in-world steps of the lane's finished histories, and of its current one
     // (added to 'steps' when the lane takes its next photon or at the end)
     uint32_t steps = 0;
@@ -113,8 +113,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(W, 8))) voi
     LutPoint<float> lp { 0, 0.0f };
     const float inv[3] = { 1.0f / w.spacing[0], 1.0f / w.spacing[1], 1.0f / w.spacing[2] };
     // the world's layout, fixed by K where it can be
-    const uint32_t codeBytes = K == WORLD_CODES8 ? 1u : K == WORLD_PALETTE8 ? 0u : w.codeBytes;
-    const uint32_t voxelBytes = K == WORLD_PALETTE8 ? 1u : K == WORLD_CODES8 ? 8u : w.voxelBytes;
+    const uint32_t codeBytes = K == WORLD_CODES8 ? 1u : kindPalette8(K) ? 0u : w.codeBytes;
+    const uint32_t voxelBytes = kindPalette8(K) ? 1u : K == WORLD_CODES8 ? 8u : w.voxelBytes;
     const bool index24 = K != WORLD_ANY || w.index24 != 0;
     const bool sumBounds = K == WORLD_CODES8 || (K == WORLD_ANY && t.lutSumBound != nullptr);
     // global index of the launch's first history (PCG increments of queued photons)
@@ -123,7 +123,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(W, 8))) voi
 
     // the wave's queue of new photons, already in the world (LDS, SoA)
     // (fixed at 48 on palette worlds, where a run-time capacity cost DX 2 %)
-    const uint32_t QUEUE_CAP = W < 7 ? 64u : K == WORLD_PALETTE8 ? 48u : queueCapacity;
+    const uint32_t QUEUE_CAP = W < 7 ? 64u : kindPalette8(K) ? 48u : queueCapacity;
     float* q = reinterpret_cast<float*>(lds + ldsBytes(tg, S, L) + (threadIdx.x / 64) * queueBytes(QUEUE_CAP));
     uint32_t queued = 0;
 
@@ -219,16 +219,17 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(W, 8))) voi
         }
         const uint32_t nPend = __popcll(pend);
         if (nPend != 0 && (nPend >= interactThreshold || fly == 0)) {
+            Deposits<float> deposits;
             if (phase == PENDING) {
                 const uint32_t mat = matMeas & 0xffu;
                 float att[3];
                 attenuationAt(t, mat, lp, att);
                 bool alive;
-                if (matMeas > 0xffffffu) { // forced event (measurement voxel)
+                if (kindForces(K) && matMeas > 0xffffffu) { // forced event (measurement voxel)
                     const float prob = ((att[0] + att[1]) + att[2]) * density * majInv;
-                    alive = computeInteractionsForced<float, L>(t, prob, att, p, mat, sc, idx, rng, update);
+                    alive = computeInteractionsForced<float, L>(t, prob, att, p, mat, deposits, rng, update);
                 } else {
-                    alive = computeInteractions<float, L>(t, att, p, mat, sc, idx, rng, update);
+                    alive = computeInteractions<float, L>(t, att, p, mat, deposits, rng, update);
                 }
                 if (alive)
                     alive = roulette(p, rng);
@@ -239,6 +240,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(W, 8))) voi
                 }
                 phase = alive ? FLYING : DEAD;
             }
+            events += deposits.n;
+            scoreWave(tally, deposits.n > 0, idx, deposits.first, !index24);
+            if (kindForces(K) && __ballot(deposits.n > 1) != 0) // forced events with a Compton event
+                scoreWave(tally, deposits.n > 1, idx, deposits.second, !index24);
         } else {
             // Woodcock flights of the FLYING lanes, one after the other
             // while no lane needs the outer loop: it ends when interactions
@@ -330,9 +335,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(W, 8))) voi
                             prob = ((att[0] + att[1]) + att[2]) * density * majInv;
                         }
                     }
-                    const bool measured = matMeas > 0xffffffu;
-                    const bool drawn = in & !measured;
-                    rng.s = drawn ? r2.s : rng.s;
+                    const bool measured = kindForces(K) && matMeas > 0xffffffu;
+                    // a photon outside is gone, whatever its stream's state
+                    rng.s = measured ? rng.s : r2.s;
                     const bool real = measured | (u2 < prob);
                     uint32_t next = in ? (real ? PENDING : FLYING) : DEAD;
                     if (next == FLYING && p.energy * p.weight < 5.0f) { // Russian roulette
@@ -354,7 +359,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(W, 8))) voi
         }
     }
     if (ctr)
-        dxmc_backend::accumulateCounters(ctr, steps + historySteps, sc.events);
+        dxmc_backend::accumulateCounters(ctr, steps + historySteps, events);
 }
 
 }
@@ -389,7 +394,9 @@ template <int L>
 KernelFn variant(uint32_t waves, uint32_t stage, uint32_t kind)
 {
     return kind == WORLD_CODES8 ? variant<L, WORLD_CODES8>(waves, stage)
-        : kind == WORLD_PALETTE8 ? variant<L, WORLD_PALETTE8>(waves, stage) : variant<L, WORLD_ANY>(waves, stage);
+        : kind == WORLD_PALETTE8          ? variant<L, WORLD_PALETTE8>(waves, stage)
+        : kind == WORLD_PALETTE8_MEASURED ? variant<L, WORLD_PALETTE8_MEASURED>(waves, stage)
+                                          : variant<L, WORLD_ANY>(waves, stage);
 }
 
 KernelFn kernelFor(int L, uint32_t waves, uint32_t stage, uint32_t kind)
@@ -406,7 +413,7 @@ uint32_t worldKind(const World<float>& w, const Tables<float>& t)
     if (w.codeBytes == 1 && w.voxelBytes == 8 && t.lutSumBound)
         return WORLD_CODES8;
     if (w.codeBytes == 0 && w.voxelBytes == 1 && !t.lutSumBound)
-        return WORLD_PALETTE8;
+        return w.measurement ? WORLD_PALETTE8_MEASURED : WORLD_PALETTE8;
     return WORLD_ANY;
 }
 
@@ -450,7 +457,7 @@ uint32_t queueCapFp32(int L, uint32_t waves, uint32_t tablesBytes, uint32_t kind
 {
     if (waves < 7)
         return 64;
-    if (kind == WORLD_PALETTE8)
+    if (kindPalette8(kind))
         return 48;
     for (uint32_t cap : { 48u, 40u, 32u })
         if (residentBlocksFp32(L, waves, tablesBytes + WAVES_PER_BLOCK * queueBytes(cap), kind) >= 7)

@@ -112,7 +112,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 8))) voi
     uint64_t poolNext = 0, poolEnd = 0;
     uint32_t poolExp = 0;
     bool claimedAll = span == 0;
-    Scorer sc { args.tally, 0 };
+    uint32_t events = 0; // scoring events of the lane's interactions
     uint32_t steps = 0;
     uint32_t historySteps = 0;
     uint64_t idx = 0;
@@ -226,17 +226,18 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 8))) voi
         }
         const uint32_t nPend = __popcll(pend);
         if (nPend != 0 && (nPend >= args.interactThreshold || fly == 0)) {
+            Deposits<double> deposits;
             if (phase == PENDING) {
                 const Args64& a = loopArgs();
                 const uint32_t mat = matMeas & 0xffu;
                 double att[3];
                 attenuationAt(t, mat, lp, att);
                 bool alive;
-                if (matMeas > 0xffffffu) { // forced event (measurement voxel)
+                if (K != WORLD_CODES8 && matMeas > 0xffffffu) { // forced event (measurement voxel)
                     const double prob = ((att[0] + att[1]) + att[2]) * a.w.density[idx] * majInv;
-                    alive = computeInteractionsForced<double, L>(t, prob, att, p, mat, sc, idx, rng, update);
+                    alive = computeInteractionsForced<double, L>(t, prob, att, p, mat, deposits, rng, update);
                 } else {
-                    alive = computeInteractions<double, L>(t, att, p, mat, sc, idx, rng, update);
+                    alive = computeInteractions<double, L>(t, att, p, mat, deposits, rng, update);
                 }
                 if (alive && p.energy * p.weight < 5.0) { // Russian roulette
                     if (rng.uniform<double>() < 0.8)
@@ -253,6 +254,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 8))) voi
                 }
                 phase = alive && historySteps < MAX_STEPS ? FLYING : DEAD;
             }
+            events += deposits.n;
+            const bool wide = K != WORLD_CODES8 && args.w.index24 == 0;
+            scoreWave(args.tally, deposits.n > 0, idx, deposits.first, wide);
+            if (K != WORLD_CODES8 && __ballot(deposits.n > 1) != 0) // forced events with a Compton event
+                scoreWave(args.tally, deposits.n > 1, idx, deposits.second, wide);
         } else {
             // Woodcock flights of the FLYING lanes until the outer loop is needed
             for (;;) {
@@ -336,7 +342,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 8))) voi
         }
     }
     if (args.ctr)
-        dxmc_backend::accumulateCounters(args.ctr, steps + historySteps, sc.events);
+        dxmc_backend::accumulateCounters(args.ctr, steps + historySteps, events);
 }
 
 __global__ void clearCounter(unsigned long long* counter) { *counter = 0; }
