@@ -107,20 +107,15 @@ int autotune(dxmc_ctx* c, const dxmc_world* w, const dxmc_tables* t, const dxmc_
     double bestRate = st ? -1 : tr.rate(cfg, st);
     if (!st) {
         if (cfg.precision == DXMC_PRECISION_FP32) {
-            st = searchField(tr, cfg, &dxmc_run_cfg::waves_per_simd, { 5, 6, 7 }, bestRate);
+            st = searchField(tr, cfg, &dxmc_run_cfg::waves_per_simd, { 4, 6 }, bestRate);
             if (!st)
                 st = searchField(tr, cfg, &dxmc_run_cfg::lds_tables, { 1, 2, 3 }, bestRate);
             if (!st && w->blocks)
                 st = searchField(tr, cfg, &dxmc_run_cfg::block_bounds, { 1, 2 }, bestRate);
-            const uint32_t resident = residentBlocksFp32(cfg.low_energy_correction, wavesFp32(cfg.waves_per_simd, cfg.low_energy_correction, 0), 0);
-            std::vector<uint32_t> perCU;
-            for (uint32_t b : { resident > 1 ? resident - 1 : 1u, std::max(1u, resident / 2) })
-                if (b != resident && std::find(perCU.begin(), perCU.end(), b) == perCU.end())
-                    perCU.push_back(b);
-            if (!st && !(st = searchField(tr, cfg, &dxmc_run_cfg::regeneration_threshold, { 1, 2, 8, 16 }, bestRate))
-                && !(st = searchField(tr, cfg, &dxmc_run_cfg::interaction_threshold, { 1, 8, 16, 24, 32, 40, 48 }, bestRate))
+            if (!st && !(st = searchField(tr, cfg, &dxmc_run_cfg::regeneration_threshold, { 4, 6, 10, 12, 16 }, bestRate))
+                && !(st = searchField(tr, cfg, &dxmc_run_cfg::interaction_threshold, { 24, 32, 40, 44 }, bestRate))
                 && !(st = searchField(tr, cfg, &dxmc_run_cfg::queue_depth, { 128, 256, 512, 1024, 2048, 4096 }, bestRate)))
-                st = searchField(tr, cfg, &dxmc_run_cfg::blocks_per_cu, perCU, bestRate);
+                st = searchField(tr, cfg, &dxmc_run_cfg::blocks_per_cu, { 1 }, bestRate);
         } else {
             st = searchField(tr, cfg, &dxmc_run_cfg::block_size, { 64, 128, 256 }, bestRate);
         }

@@ -25,6 +25,7 @@
 // equal to the last CDF node) are clamped to the last valid element.
 #pragma once
 #include "rng.hpp"
+#include <cmath>
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -168,7 +169,21 @@ struct World {
     const uint16_t* blocks;
     uint32_t bnx, bnxy, blockShift;
     uint32_t codeMul; // 1-byte codes: material of a code by multiply and shift
+    // FP32: 1 when some position inside the extent has a coordinate that
+    // rounds to the grid size (its index is then clamped)
+    uint32_t facesRound;
 };
+
+// Whether (pos - lower) * inv, truncated, may reach n for some float pos
+// inside (lower, upper): subtraction and product round monotonically, so the
+// largest such position decides. The device's reciprocal may be an ulp or two
+// off the host's; four ulp are allowed for.
+inline bool coordinateReaches(float lower, float upper, float inv, uint32_t n)
+{
+    const float d = std::nextafter(upper, lower) - lower;
+    const float q = d * (inv * (1.0f + 4 * 1.1920929e-7f));
+    return !(q < static_cast<float>(n)) || static_cast<uint32_t>(q) >= n;
+}
 
 constexpr uint32_t BLOCK_SHIFT_MIN = 3, BLOCK_SHIFT_MAX = 6; // 8 to 64 voxels per block edge
 constexpr uint64_t BLOCK_TABLE_BYTES = 64 * 1024; // a block-code table above this size takes the next block edge

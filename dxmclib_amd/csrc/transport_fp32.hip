@@ -1,28 +1,33 @@
-// FP32 photon transport: persistent kernel with wave-level regeneration and
-// interaction compaction.
+// FP32 photon transport: persistent kernel with per-wave photon pools.
 //
-// Each lane carries one photon (position, direction, energy, weight,
-// majorant, PCG state) in registers and is in one of three phases:
-//   DEAD     no photon: waits for regeneration
-//   FLYING   advances one Woodcock flight per loop iteration (distance under
-//            the majorant, voxel gather, real-or-virtual decision, roulette
-//            after virtual collisions)
-//   PENDING  a real interaction is due in the voxel just reached
-// Per iteration the wave does one of two things, decided from ballots:
-//   - when at least 'interaction_threshold' lanes are PENDING (or none is
-//     FLYING) it runs the interaction code for the pending lanes only,
-//   - otherwise it advances the FLYING lanes.
-// So the long, branchy interaction samplers (Compton/Rayleigh rejection
-// loops, fluorescence) run with many lanes active instead of with the few
-// lanes that happen to interact in a given flight, while the cheap flights
-// run nearly full. New photons are sampled by the whole wave at once (up to
-// the queue's 64 or 48 histories from a wave-private pool of history
-// indices, which one lane refills with a single atomic on the global
-// counter) into a per-wave queue in LDS; dead lanes take photons from that
-// queue once at least
-// 'regeneration_threshold' of them wait, each by its rank among the dead
-// lanes (ballot + mbcnt). So the costly source sampling runs with all lanes
-// active and a lane is refilled with a few LDS reads.
+// Each lane flies one photon (position, direction, energy, weight, majorant,
+// PCG state) in registers; a wave keeps further photons in a pool in LDS,
+// some ready to fly, others with an interaction due. The wave runs three
+// kinds of work, each with many lanes:
+//   flights       Woodcock flights of the lanes (distance under the majorant,
+//                 real-or-virtual decision from density and attenuation
+//                 bounds, roulette), until 'regeneration_threshold' lanes
+//                 have lost their photon or are due to interact; due photons
+//                 then go to the pool and ready ones take their lanes
+//   interactions  once 'interaction_threshold' photons are due, they come to
+//                 the lanes, in exchange for the photons flying there, and
+//                 run the samplers (Compton/Rayleigh rejection loops,
+//                 fluorescence) together; the survivors fly on
+//   sampling      when too few photons are ready, the whole wave samples new
+//                 histories into the pool (from a wave-private range of
+//                 history indices, which one lane refills with an atomic on
+//                 the launch's counter)
+// Without the pool, due photons waited on their lanes: 51 of 64 lanes flew
+// and 21 interacted (126 vector instructions a history on the CT spiral
+// workload, 91 with it).
+//
+// What bounds it: the latency of a flight's chain (block code from L2, then
+// intervals and segment bounds from LDS) and vector issue (75 % busy before
+// the bounds moved to LDS). CT spiral 512x512x300, 1e9 histories: 228 ms
+// with due photons on their lanes and 7 waves a SIMD, 197 with pools and 6
+// waves, 180 with density intervals and attenuation bounds in LDS; axial
+// 1024x1024x128, 4e8: 77, 69, 60 ms; impulse approximation, 401x333x151,
+// 1.5e8: 48.4, 42.7, 38.9 ms (4 waves).
 //
 // Each history keeps its own PCG stream and consumes it in the reference's
 // order (flight, decision, interaction, roulette), so delaying an interaction
@@ -33,7 +38,7 @@
 // by multiplication with the reciprocal spacing, FP32 denormals flushed);
 // each scoring event is added to the FP64 tallies with hardware FP64
 // atomics. The kernel is compiled per low-energy model, register budget
-// (5, 6 or 7 waves per SIMD), LDS staging level and world kind.
+// (4 or 6 waves per SIMD), LDS staging level and world kind.
 #include "device/persistent.hpp"
 #include "internal.hpp"
 
@@ -41,28 +46,50 @@ using namespace dxmc_dev;
 
 namespace {
 
-// voxel coordinates with the reciprocal spacing (FP32 path), kept inside the
-// grid (the float-to-unsigned conversion clamps negative values to 0)
+// voxel coordinates, with the reciprocal spacing, of a position inside the
+// extent. Kept inside the grid where rounding can reach its far end
+// (facesRound, known per world).
 __device__ inline uint3 voxelCoordsFast(const World<float>& w, const float* pos, const float* inv)
 {
-    return make_uint3(min(static_cast<uint32_t>((pos[0] - w.extent[0]) * inv[0]), w.nx - 1),
-        min(static_cast<uint32_t>((pos[1] - w.extent[2]) * inv[1]), w.ny - 1), min(static_cast<uint32_t>((pos[2] - w.extent[4]) * inv[2]), w.nz - 1));
+    uint3 v = make_uint3(static_cast<uint32_t>((pos[0] - w.extent[0]) * inv[0]), static_cast<uint32_t>((pos[1] - w.extent[2]) * inv[1]),
+        static_cast<uint32_t>((pos[2] - w.extent[4]) * inv[2]));
+    if (w.facesRound) {
+        v.x = min(v.x, w.nx - 1);
+        v.y = min(v.y, w.ny - 1);
+        v.z = min(v.z, w.nz - 1);
+    }
+    return v;
 }
 
 constexpr float LN2F = 0.693147180559945309f;
 
-// per-wave queue of sampled photons in LDS: position, direction, energy,
-// weight, PCG state, the history's offset in the launch (its PCG increment
-// is 2 (first history + launch begin + offset) + 1) and the LUT segment of
-// the energy, found while the whole wave samples (the segment search has
-// loops; a lane that takes the photon only adds the segment offset and the
-// majorant)
-constexpr int QUEUE_FIELDS = 12;
-// photons a wave's queue holds: 64 (the whole wave samples at once), or in
-// the 7-wave kernels, whose LDS must fit 7 blocks per CU, a capacity the
-// launch passes (48, or less where the staged tables are larger)
-__host__ __device__ constexpr uint32_t queueBytes(uint32_t capacity) { return QUEUE_FIELDS * capacity * 4; }
-constexpr uint32_t WAVES_PER_BLOCK = 4;
+// A wave's pool of photons in LDS: a ring of slots whose first 'ready' ones
+// hold photons to fly and the next 'pending' ones photons with an interaction
+// due. One record of 13 words a photon (an odd stride: lanes reading the same
+// word of consecutive slots hit different banks): position, direction,
+// energy, weight, PCG state, the history's offset in the launch (its PCG
+// increment is 2 (first history + launch begin + offset) + 1), LUT segment |
+// material << 20 | measurement flag << 28, and the history's steps so far.
+// What follows from these (the LUT offset, the majorant, the voxel) is
+// computed again when a lane takes the photon.
+constexpr uint32_t SLOT_WORDS = 13;
+constexpr uint32_t SLOT_BYTES = SLOT_WORDS * 4;
+constexpr uint32_t POOL_RESERVE = 16; // slots that sampling leaves for photons that become pending
+constexpr uint32_t POOL_MAX = 128; // most slots a wave uses
+constexpr uint32_t POOL_MIN = 48;
+constexpr uint32_t FLIGHTS_PER_LOOP = 64; // most flights before the outer loop runs
+
+// LDS of the density intervals and attenuation bounds a staged code world
+// adds: a flight reads them after the block code (and the voxel code); from
+// LDS instead of L1 they took the CT spiral from 201 to 180 ms
+__host__ __device__ inline uint32_t boundsBytes(const Tables<float>& t)
+{
+    return ldsAlign(uint64_t(t.nMaterials) * t.lutNodes * sizeof(float2)) + 256 * sizeof(float2);
+}
+
+// Waves of a block: two blocks fill a CU's 4 W waves, so the staged tables
+// are held twice a CU and the LDS left is the waves' pools.
+__host__ __device__ constexpr uint32_t blockWaves(uint32_t W) { return 2 * W; }
 
 // Russian roulette after a step that left the photon alive (transport.hpp:684-694)
 __device__ inline bool roulette(Particle<float>& p, Rng& rng)
@@ -75,40 +102,47 @@ __device__ inline bool roulette(Particle<float>& p, Rng& rng)
     return true;
 }
 
-// W: minimum resident waves per SIMD the register allocation must allow
-// (1: unconstrained, 5 waves; 6: at most 80 VGPRs, spill-free at L = 0, 1;
-// 7: at most 72 VGPRs, spill-free for the two fixed world kinds at L = 0, 1,
-// with a 48-photon queue). S: LDS staging level. K: world kind. The
-// autotuner picks among the register budgets and staging levels.
+// W: resident waves per SIMD the register allocation must allow, 6 (at most 80
+// VGPRs, spill-free at L = 0, 1 but for few lanes' values of kind any) or 4
+// (128 VGPRs; CT spiral 206 ms, 6: 180). Blocks of 10 or 14 waves load the
+// SIMDs unevenly, so that a CU holds one instead of two (340 ms); 16 waves
+// with 64 VGPRs spill (282 ms).
+// S: LDS staging level. K: world kind. The autotuner picks among the register
+// budgets and staging levels.
 template <int L, int W, uint32_t S, uint32_t K>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(W, 8))) void transportPersistent(World<float> w, Tables<float> tg, const Exposure<float>* exps, const uint64_t* expStart,
+__global__ __launch_bounds__(64 * blockWaves(W)) __attribute__((amdgpu_waves_per_eu(W, 8))) void transportPersistent(World<float> w, Tables<float> tg, const Exposure<float>* exps, const uint64_t* expStart,
     uint32_t nExp, uint64_t hBegin, uint64_t hEnd, uint64_t seed, uint64_t firstHistory, Tally tally, Counters* ctr, unsigned long long* next,
-    uint32_t regenThreshold, uint32_t interactThreshold, uint32_t poolSize, uint32_t queueCapacity)
+    uint32_t refillThreshold, uint32_t interactThreshold, uint32_t poolSize, uint32_t slots)
 {
     extern __shared__ __align__(16) unsigned char lds[];
     Tables<float> t = tg;
     stageTables<float, S, L>(t, lds);
+    const float2* bounds = nullptr; // CODES8, staged: density interval of each code
+    constexpr bool BOUNDS_LDS = K == WORLD_CODES8 && S >= STAGE_SMALL;
+    if constexpr (BOUNDS_LDS) {
+        unsigned char* c = lds + ldsBytes(tg, S, L);
+        t.lutSumBound = stageArray(t.lutSumBound, uint64_t(t.nMaterials) * t.lutNodes, c);
+        float2* d = reinterpret_cast<float2*>(c);
+        for (uint32_t i = threadIdx.x; i < 256; i += blockDim.x)
+            d[i] = make_float2(w.bounds[i].lo, w.bounds[i].hi);
+        bounds = d;
+        __syncthreads();
+    }
     Particle<float> p;
     Rng rng { 0, 1 };
     float majInv = 0;
-    bool update = true;
-    uint32_t phase = DEAD;
-    // the wave's pool of claimed, not yet started histories [poolNext, poolEnd)
+    bool flying = false, due = false; // neither: the lane holds no photon
+    // the wave's claimed, not yet started histories [poolNext, poolEnd)
     const uint64_t span = hEnd - hBegin;
     uint64_t poolNext = 0, poolEnd = 0;
     uint32_t poolExp = 0;
     bool claimedAll = span == 0;
     uint32_t events = 0; // scoring events of the lane's interactions
-    // in-world steps of the lane's finished histories, and of its current one
-    // (added to 'steps' when the lane takes its next photon or at the end)
-    uint32_t steps = 0;
-    uint32_t historySteps = 0;
-    // the pending interaction
-    uint64_t idx = 0;
+    uint32_t steps = 0; // in-world steps of the histories that ended on this lane
+    uint32_t historySteps = 0; // of its current one
     // material | measurement flag << 24 of the voxel reached (one register;
     // the LUT row products are 24-bit and ignore the flag)
     uint32_t matMeas = 0;
-    float density = 0;
     // the photon's place in the LUT; changes only with its energy
     LutPoint<float> lp { 0, 0.0f };
     const float inv[3] = { 1.0f / w.spacing[0], 1.0f / w.spacing[1], 1.0f / w.spacing[2] };
@@ -117,26 +151,141 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(W, 8))) voi
     const uint32_t voxelBytes = kindPalette8(K) ? 1u : K == WORLD_CODES8 ? 8u : w.voxelBytes;
     const bool index24 = K != WORLD_ANY || w.index24 != 0;
     const bool sumBounds = K == WORLD_CODES8 || (K == WORLD_ANY && t.lutSumBound != nullptr);
-    // global index of the launch's first history (PCG increments of queued photons)
+    // global index of the launch's first history (PCG increments of pooled photons)
     const uint64_t launchFirst = firstHistory + hBegin;
     const uint32_t lane = __lane_id();
 
-    // the wave's queue of new photons, already in the world (LDS, SoA)
-    // (fixed at 48 on palette worlds, where a run-time capacity cost DX 2 %)
-    const uint32_t QUEUE_CAP = W < 7 ? 64u : kindPalette8(K) ? 48u : queueCapacity;
-    float* q = reinterpret_cast<float*>(lds + ldsBytes(tg, S, L) + (threadIdx.x / 64) * queueBytes(QUEUE_CAP));
-    uint32_t queued = 0;
+    uint32_t* pool = reinterpret_cast<uint32_t*>(lds + ldsBytes(tg, S, L) + (BOUNDS_LDS ? boundsBytes(tg) : 0u) + (threadIdx.x / 64) * (slots * SLOT_BYTES));
+    uint32_t first = 0, ready = 0, pending = 0; // the ring's window (wave-uniform)
+    // slot 'offset' from the start of the window
+    auto slotAt = [&](uint32_t offset) {
+        const uint32_t k = first + offset;
+        return pool + (k >= slots ? k - slots : k) * SLOT_WORDS;
+    };
+    auto packSegment = [&]() { return lp.k | (matMeas & 0xffu) << 20 | (kindForces(K) ? (matMeas >> 24 != 0 ? 1u << 28 : 0u) : 0u); };
+    auto store = [&](uint32_t* q) {
+        for (int i = 0; i < 3; ++i) {
+            q[i] = __float_as_uint(p.pos[i]);
+            q[3 + i] = __float_as_uint(p.dir[i]);
+        }
+        q[6] = __float_as_uint(p.energy);
+        q[7] = __float_as_uint(p.weight);
+        q[8] = static_cast<uint32_t>(rng.s);
+        q[9] = static_cast<uint32_t>(rng.s >> 32);
+        q[10] = static_cast<uint32_t>(rng.inc >> 1) - static_cast<uint32_t>(launchFirst);
+        q[11] = packSegment();
+        q[12] = historySteps;
+    };
+    // takes the photon out of a slot; what it leaves out is set by derive()
+    auto load = [&](const uint32_t* q) {
+        for (int i = 0; i < 3; ++i) {
+            p.pos[i] = __uint_as_float(q[i]);
+            p.dir[i] = __uint_as_float(q[3 + i]);
+        }
+        p.energy = __uint_as_float(q[6]);
+        p.weight = __uint_as_float(q[7]);
+        rng.s = static_cast<uint64_t>(q[9]) << 32 | q[8];
+        rng.inc = 2 * (launchFirst + q[10]) + 1;
+        const uint32_t segment = q[11];
+        lp.k = segment & 0xfffffu;
+        matMeas = (segment >> 20 & 0xffu) | (kindForces(K) ? segment >> 28 << 24 : 0u);
+        historySteps = q[12];
+    };
+    // the LUT point lutPoint() gives, from the known segment, and the majorant
+    auto derive = [&]() {
+        lp.x = __builtin_amdgcn_logf(p.energy) - t.lutAnchor[lp.k];
+        majInv = majorantInverseAt(t, lp);
+    };
 
     for (;;) {
-        uint64_t dead = __ballot(phase == DEAD);
-        uint32_t nDead = __popcll(dead);
+        const uint64_t dueMask = __ballot(due);
+        uint64_t flyMask = __ballot(flying);
+        const uint32_t nDue = __popcll(dueMask);
+        const uint32_t nFly = __popcll(flyMask);
+        const uint32_t room = slots - ready - pending;
         const bool work = poolNext < poolEnd || !claimedAll;
-        if (work && queued < nDead) {
+        const bool canSample = work && room > POOL_RESERVE;
+        // Interactions run once enough photons wait for one (on lanes and in
+        // the pool), when the pool cannot take the lanes' due photons, or when
+        // there is little else left to do.
+        const uint32_t waiting = nDue + pending;
+        if (waiting != 0
+            && (waiting >= interactThreshold || nDue > room || (!work && ready == 0 && waiting >= nFly) || (nFly == 0 && ready == 0 && !canSample))) {
+            // The pool's pending photons come to the lanes: to lanes without
+            // a photon from the end of the window, and to flying lanes from
+            // its front in exchange for their photon, whose slot then joins
+            // the ready ones.
+            const uint64_t emptyMask = ~(dueMask | flyMask);
+            const uint32_t back = min(64u - nDue - nFly, pending);
+            const uint32_t front = min(nFly, pending - back);
+            const bool taken = !due && !flying && rankBelow(emptyMask) < back;
+            const bool exchanged = flying && rankBelow(flyMask) < front;
+            if (taken || exchanged) {
+                uint32_t* q = slotAt(taken ? ready + pending - 1 - rankBelow(emptyMask) : ready + rankBelow(flyMask));
+                if (exchanged) {
+                    uint32_t v[SLOT_WORDS];
+                    for (uint32_t f = 0; f < SLOT_WORDS; ++f)
+                        v[f] = q[f];
+                    store(q);
+                    load(v);
+                } else {
+                    steps += historySteps;
+                    load(q);
+                }
+                derive();
+                due = true;
+                flying = false;
+            }
+            pending -= back + front;
+            ready += front;
+            Deposits<float> deposits;
+            uint64_t idx = 0;
+            if (due) {
+                const uint32_t mat = matMeas & 0xffu;
+                idx = voxelIndexFast(w, voxelCoordsFast(w, p.pos, inv), index24); // the voxel the flight ended in
+                bool update = false;
+                float att[3];
+                attenuationAt(t, mat, lp, att);
+                bool alive;
+                if (kindForces(K) && matMeas > 0xffffffu) { // forced event (measurement voxel)
+                    float density;
+                    uint32_t tag;
+                    readVoxelPacked(w, voxelBytes, idx, tag, density);
+                    const float prob = ((att[0] + att[1]) + att[2]) * density * majInv;
+                    alive = computeInteractionsForced<float, L>(t, prob, att, p, mat, deposits, rng, update);
+                } else {
+                    alive = computeInteractions<float, L>(t, att, p, mat, deposits, rng, update);
+                }
+                if (alive)
+                    alive = roulette(p, rng);
+                if (alive && update) { // new energy: its LUT segment and majorant
+                    lp = lutPoint(t, p.energy);
+                    majInv = majorantInverseAt(t, lp);
+                }
+                flying = alive;
+                due = false;
+            }
+            events += deposits.n;
+            scoreWave(tally, deposits.n > 0, idx, deposits.first, !index24);
+            if (kindForces(K) && __ballot(deposits.n > 1) != 0) // forced events with a Compton event
+                scoreWave(tally, deposits.n > 1, idx, deposits.second, !index24);
+        } else if (nDue != 0) {
+            // photons with an interaction due wait in the pool
+            if (due) {
+                store(slotAt(ready + pending + rankBelow(dueMask)));
+                historySteps = 0;
+                due = false;
+            }
+            pending += nDue;
+        }
+        flyMask = __ballot(flying);
+        const uint32_t nEmpty = 64u - __popcll(flyMask);
+        if (work && ready < nEmpty && slots - ready - pending > POOL_RESERVE) {
             // sample new histories with the whole wave: lanes 0 .. want-1
             // take the next histories of the wave's pool (refilled from the
             // global counter as needed), photons that enter the world join
-            // the queue
-            const uint32_t want = QUEUE_CAP - queued;
+            // the ready ones
+            const uint32_t want = min(64u, slots - ready - pending - POOL_RESERVE);
             uint32_t assigned = 0;
             bool sampled = false;
             Particle<float> np;
@@ -170,100 +319,64 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(W, 8))) voi
                 assigned += take;
             }
             const uint64_t entered = __ballot(sampled);
+            const uint32_t n = __popcll(entered);
+            first = first >= n ? first - n : first + slots - n; // ahead of the ready ones
+            ready += n;
             if (sampled) {
-                const uint32_t slot = queued + rankBelow(entered);
-                const float v[QUEUE_FIELDS] = { np.pos[0], np.pos[1], np.pos[2], np.dir[0], np.dir[1], np.dir[2], np.energy, np.weight,
-                    __uint_as_float(static_cast<uint32_t>(nr.s)), __uint_as_float(static_cast<uint32_t>(nr.s >> 32)), __uint_as_float(nOffset),
-                    __uint_as_float(lutPoint(t, np.energy).k) };
-                for (int f = 0; f < QUEUE_FIELDS; ++f)
-                    q[f * QUEUE_CAP + slot] = v[f];
-            }
-            queued += __popcll(entered);
-        }
-        // dead lanes take photons from the queue (last in, first out)
-        if (nDead >= regenThreshold || (nDead > 0 && !work)) {
-            const uint32_t take = nDead < queued ? nDead : queued;
-            if (phase == DEAD) {
-                const uint32_t r = rankBelow(dead);
-                if (r < take) {
-                    const uint32_t slot = queued - 1 - r;
-                    float v[QUEUE_FIELDS];
-                    for (int f = 0; f < QUEUE_FIELDS; ++f)
-                        v[f] = q[f * QUEUE_CAP + slot];
-                    for (int i = 0; i < 3; ++i) {
-                        p.pos[i] = v[i];
-                        p.dir[i] = v[3 + i];
-                    }
-                    p.energy = v[6];
-                    p.weight = v[7];
-                    rng.s = static_cast<uint64_t>(__float_as_uint(v[9])) << 32 | __float_as_uint(v[8]);
-                    rng.inc = 2 * (launchFirst + __float_as_uint(v[10])) + 1;
-                    // the LUT point lutPoint() gives, from the queued segment
-                    lp.k = __float_as_uint(v[11]);
-                    lp.x = __builtin_amdgcn_logf(p.energy) - t.lutAnchor[lp.k];
-                    majInv = majorantInverseAt(t, lp);
-                    update = false;
-                    steps += historySteps;
-                    historySteps = 0;
-                    phase = FLYING;
+                uint32_t* q = slotAt(rankBelow(entered));
+                for (int i = 0; i < 3; ++i) {
+                    q[i] = __float_as_uint(np.pos[i]);
+                    q[3 + i] = __float_as_uint(np.dir[i]);
                 }
+                q[6] = __float_as_uint(np.energy);
+                q[7] = __float_as_uint(np.weight);
+                q[8] = static_cast<uint32_t>(nr.s);
+                q[9] = static_cast<uint32_t>(nr.s >> 32);
+                q[10] = nOffset;
+                q[11] = lutPoint(t, np.energy).k;
+                q[12] = 0;
             }
-            queued -= take;
         }
-        const uint64_t pend = __ballot(phase == PENDING);
-        const uint64_t fly = __ballot(phase == FLYING);
-        if ((pend | fly) == 0) {
-            if (poolNext >= poolEnd && claimedAll && queued == 0)
+        // lanes without a photon take ready ones from the front of the window
+        const uint32_t take = min(nEmpty, ready);
+        if (take != 0) {
+            const uint32_t r = rankBelow(~flyMask);
+            if (!flying && r < take) {
+                steps += historySteps;
+                load(slotAt(r));
+                derive();
+                flying = true;
+            }
+            first += take;
+            first = first >= slots ? first - slots : first;
+            ready -= take;
+        }
+        const bool more = poolNext < poolEnd || !claimedAll || ready != 0;
+        if (__ballot(flying) == 0) {
+            if (!more && pending == 0)
                 break;
             continue;
         }
-        const uint32_t nPend = __popcll(pend);
-        if (nPend != 0 && (nPend >= interactThreshold || fly == 0)) {
-            Deposits<float> deposits;
-            if (phase == PENDING) {
-                const uint32_t mat = matMeas & 0xffu;
-                float att[3];
-                attenuationAt(t, mat, lp, att);
-                bool alive;
-                if (kindForces(K) && matMeas > 0xffffffu) { // forced event (measurement voxel)
-                    const float prob = ((att[0] + att[1]) + att[2]) * density * majInv;
-                    alive = computeInteractionsForced<float, L>(t, prob, att, p, mat, deposits, rng, update);
-                } else {
-                    alive = computeInteractions<float, L>(t, att, p, mat, deposits, rng, update);
-                }
-                if (alive)
-                    alive = roulette(p, rng);
-                if (alive && update) { // new energy: its LUT segment and majorant
-                    lp = lutPoint(t, p.energy);
-                    majInv = majorantInverseAt(t, lp);
-                    update = false;
-                }
-                phase = alive ? FLYING : DEAD;
-            }
-            events += deposits.n;
-            scoreWave(tally, deposits.n > 0, idx, deposits.first, !index24);
-            if (kindForces(K) && __ballot(deposits.n > 1) != 0) // forced events with a Compton event
-                scoreWave(tally, deposits.n > 1, idx, deposits.second, !index24);
-        } else {
-            // Woodcock flights of the FLYING lanes, one after the other
-            // while no lane needs the outer loop: it ends when interactions
-            // are due (interaction_threshold pending lanes, or none flying)
-            // or dead lanes wait (for a refill of the queue while histories
-            // remain, or for regeneration). Only the flight's own values are
-            // live in this loop, so they stay in registers.
-            for (;;) {
-                if (phase == FLYING) {
-                    // one Woodcock flight (woodcockParticleTracking, transport.hpp:
-                    // 650-699), written without branches apart from the rare
-                    // roulette: the random draws the reference makes only inside
-                    // the world (decision) are drawn and kept by selection
-                    const float u1 = rng.uniform<float>();
-                    const float step = -__builtin_amdgcn_logf(u1) * (LN2F * 10.0f) * majInv; // cm -> mm
-                    for (int i = 0; i < 3; ++i)
-                        p.pos[i] += p.dir[i] * step;
-                    const bool in = insideFast(w, p.pos);
-                    const uint3 vc = voxelCoordsFast(w, p.pos, inv); // clamped: a valid voxel also outside
-                    idx = voxelIndexFast(w, vc, index24);
+        // Woodcock flights of the flying lanes until enough lanes wait for
+        // another photon (or, near the end, for interactions). Only the
+        // flight's own values are live in this loop. Lanes whose photon may be
+        // below the roulette limit (a flight only raises a weight) or within
+        // the loop's flights of the step cap are known as wave masks, so that
+        // the other flights test neither.
+        const uint32_t limit = more ? refillThreshold : 64u;
+        const uint64_t faintMask = __ballot(p.energy * p.weight < 5.0f);
+        const bool nearCap = __ballot(flying && historySteps >= MAX_STEPS - FLIGHTS_PER_LOOP) != 0;
+        for (uint32_t n = 0; n < FLIGHTS_PER_LOOP; ++n) {
+            if (flying) {
+                // one Woodcock flight (woodcockParticleTracking, transport.hpp:
+                // 650-699)
+                const float u1 = rng.uniform<float>();
+                const float step = -__builtin_amdgcn_logf(u1) * (LN2F * 10.0f) * majInv; // cm -> mm
+                for (int i = 0; i < 3; ++i)
+                    p.pos[i] += p.dir[i] * step;
+                flying = insideFast(w, p.pos);
+                if (flying) {
+                    const uint3 vc = voxelCoordsFast(w, p.pos, inv);
                     Rng r2 = rng;
                     const float u2 = r2.uniform<float>();
                     // The acceptance probability (Σμ·ρ)·(1/μ̂) is monotone in Σμ and
@@ -284,27 +397,33 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(W, 8))) voi
                         // the material from the largest code by arithmetic, so
                         // the intervals and the segment bounds load together
                         const uint32_t bm = __umul24(bc >> 8, w.codeMul) >> CODE_MUL_SHIFT;
-                        const float bLo = w.bounds[bc & 0xffu].lo;
-                        const float bHi = w.bounds[bc >> 8].hi;
-                        const float2 sb = loadAt(t.lutSumBound, __umul24(bm, t.lutNodes) + lp.k);
+                        const float bLo = BOUNDS_LDS ? bounds[bc & 0xffu].x : w.bounds[bc & 0xffu].lo;
+                        const float bHi = BOUNDS_LDS ? bounds[bc >> 8].y : w.bounds[bc >> 8].hi;
+                        const float2 sb = BOUNDS_LDS ? t.lutSumBound[__umul24(bm, t.lutNodes) + lp.k] : loadAt(t.lutSumBound, __umul24(bm, t.lutNodes) + lp.k);
                         const float lo = sb.x * bLo * majInv;
                         const float hi = sb.y * bHi * majInv;
                         settled = (bc != BLOCK_MIXED) & ((u2 < lo) | (u2 >= hi));
                         matMeas = bm;
-                        density = bLo;
                         prob = lo;
                     }
                     if (!settled) {
-                        float dLo, dHi;
+                        const uint64_t idx = voxelIndexFast(w, vc, index24);
+                        float density, dLo, dHi;
                         if (K == WORLD_CODES8) {
                             // material by arithmetic, interval and segment bounds
                             // loaded together (code worlds carry no measurement flags)
                             // (1-byte codes: below 2^32 voxels, a 32-bit offset)
                             const uint32_t code = loadAt(static_cast<const uint8_t*>(w.codes), static_cast<uint32_t>(idx));
                             matMeas = __umul24(code, w.codeMul) >> CODE_MUL_SHIFT;
-                            const uint2 b = *reinterpret_cast<const uint2*>(w.bounds + code);
-                            dLo = __uint_as_float(b.x);
-                            dHi = __uint_as_float(b.y);
+                            if constexpr (BOUNDS_LDS) {
+                                const float2 b = bounds[code];
+                                dLo = b.x;
+                                dHi = b.y;
+                            } else {
+                                const uint2 b = *reinterpret_cast<const uint2*>(w.bounds + code);
+                                dLo = __uint_as_float(b.x);
+                                dHi = __uint_as_float(b.y);
+                            }
                             density = dLo;
                         } else if (codeBytes != 0) {
                             const uint32_t code = codeBytes == 1 ? static_cast<const uint8_t*>(w.codes)[idx] : static_cast<const uint16_t*>(w.codes)[idx];
@@ -321,7 +440,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(W, 8))) voi
                             dHi = density;
                         }
                         if (sumBounds) {
-                            const float2 sb = loadAt(t.lutSumBound, __umul24(matMeas, t.lutNodes) + lp.k);
+                            const float2 sb = BOUNDS_LDS ? t.lutSumBound[__umul24(matMeas, t.lutNodes) + lp.k] : loadAt(t.lutSumBound, __umul24(matMeas, t.lutNodes) + lp.k);
                             const float lo = sb.x * dLo * majInv;
                             const float hi = sb.y * dHi * majInv;
                             settled = (u2 < lo) | (u2 >= hi);
@@ -335,27 +454,23 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(W, 8))) voi
                             prob = ((att[0] + att[1]) + att[2]) * density * majInv;
                         }
                     }
+                    // a forced event draws no decision
                     const bool measured = kindForces(K) && matMeas > 0xffffffu;
-                    // a photon outside is gone, whatever its stream's state
                     rng.s = measured ? rng.s : r2.s;
-                    const bool real = measured | (u2 < prob);
-                    uint32_t next = in ? (real ? PENDING : FLYING) : DEAD;
-                    if (next == FLYING && p.energy * p.weight < 5.0f) { // Russian roulette
-                        if (rng.uniform<float>() < 0.8f)
-                            next = DEAD;
-                        else
-                            p.weight *= 1.0f / (1.0f - 0.8f);
+                    due = measured | (u2 < prob);
+                    flying = !due;
+                    if (flying & __builtin_amdgcn_inverse_ballot_w64(faintMask))
+                        flying = roulette(p, rng);
+                    ++historySteps;
+                    if (nearCap && historySteps >= MAX_STEPS) {
+                        flying = false;
+                        due = false;
                     }
-                    historySteps += in ? 1u : 0u;
-                    phase = (next != DEAD && historySteps >= MAX_STEPS) ? DEAD : next;
                 }
-                const uint64_t flyNow = __ballot(phase == FLYING);
-                const uint32_t nPendNow = __popcll(__ballot(phase == PENDING));
-                const uint32_t nDeadNow = __popcll(__ballot(phase == DEAD));
-                if (flyNow == 0 || nPendNow >= interactThreshold || nDeadNow >= regenThreshold || (work && nDeadNow > queued)
-                    || (!work && nDeadNow > 0 && queued > 0))
-                    break;
             }
+            const uint32_t flyNow = __popcll(__ballot(flying));
+            if (flyNow == 0 || 64u - flyNow >= limit || (!more && __popcll(__ballot(due)) + pending >= flyNow))
+                break;
         }
     }
     if (ctr)
@@ -373,15 +488,11 @@ __global__ void clearCounter(unsigned long long* counter) { *counter = 0; }
 using KernelFn = void (*)(World<float>, Tables<float>, const Exposure<float>*, const uint64_t*, uint32_t, uint64_t, uint64_t, uint64_t, uint64_t,
     Tally, Counters*, unsigned long long*, uint32_t, uint32_t, uint32_t, uint32_t);
 
-// waves: resolved by wavesFp32 (5, 6 or 7); the 7-wave kernel (72 VGPRs)
-// exists for the two fixed world kinds at L = 0, 1
+// waves: resolved by wavesFp32
 template <int L, uint32_t S, uint32_t K>
 KernelFn variant(uint32_t waves)
 {
-    if constexpr (K != WORLD_ANY && L < 2)
-        if (waves >= 7)
-            return transportPersistent<L, 7, S, K>;
-    return waves >= 6 ? transportPersistent<L, 6, S, K> : transportPersistent<L, 1, S, K>;
+    return waves >= 6 ? transportPersistent<L, 6, S, K> : transportPersistent<L, 4, S, K>;
 }
 
 template <int L, uint32_t K>
@@ -419,82 +530,32 @@ uint32_t worldKind(const World<float>& w, const Tables<float>& t)
 
 }
 
-// Resident waves per SIMD of a run: the requested 5, 6 or 7, or by default
-// 6 where that fits 80 VGPRs without spills (L = 0, 1: CT spiral 3.55e9 vs
-// 3.34e9, DX 4.13e9 vs 3.90e9 histories/s with 5), 7 for the two fixed
-// world kinds (palette: DX 4.50e9 vs 4.39e9; 1-byte codes with block codes:
-// CT spiral 3.95e9 vs 3.86e9, whole body 1.69e9 vs 1.59e9, their flights
-// being bound by gather latency more than by VALU issue; the 72-VGPR code
-// kernel keeps one lane counter in scratch, touched once per history);
-// L = 2 would spill at 6 and keeps 5.
-uint32_t wavesFp32(uint32_t requested, int L, uint32_t kind)
+// Resident waves per SIMD of a run: 6, or 4 at L = 2, whose interaction
+// samplers spill at 80 VGPRs (1.5e8 histories of the impulse approximation:
+// 47.5 ms with 6, 38.9 with 4)
+uint32_t wavesFp32(uint32_t requested, int L)
 {
-    if (requested == 0)
-        return L == 2 ? 5u : kind != WORLD_ANY ? 7u : 6u;
-    if (requested >= 7)
-        return kind != WORLD_ANY && L < 2 ? 7u : 6u;
-    return requested >= 6 ? 6u : 5u;
+    return requested == 0 ? (L == 2 ? 4u : 6u) : requested >= 6 ? 6u : 4u;
 }
 
-uint32_t residentBlocksFp32(int L, uint32_t waves, uint32_t ldsPerBlock, uint32_t kind)
+// slots of a wave's pool in blocks of 'blockOf' waves beside the staged
+// tables (half a CU's 160 KiB less an allocation granule)
+uint32_t poolSlots(const Tables<float>& t, uint32_t stage, int L, uint32_t blockOf, uint32_t kind)
 {
-    int resident = 0;
-    const uint32_t stage = ldsPerBlock ? STAGE_SMALL : STAGE_NONE;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&resident, reinterpret_cast<const void*>(kernelFor(L, waves, stage, kind)), 256, ldsPerBlock)
-            != hipSuccess
-        || resident <= 0) {
-        hipGetLastError();
-        resident = 1;
-    }
-    return static_cast<uint32_t>(resident);
+    const uint32_t tables = ldsBytes(t, stage, L) + (kind == WORLD_CODES8 && stage >= STAGE_SMALL ? boundsBytes(t) : 0u), block = 80 * 1024 - 1280;
+    return tables >= block ? 0u : std::min(POOL_MAX, (block - tables) / blockOf / SLOT_BYTES);
 }
 
-// queue capacity of a run's kernel: 64, and in the 7-wave kernels the
-// largest of 48, 40 and 32 photons with which 7 blocks stay resident on a
-// CU beside the staged tables (48 when none does, and always 48 on palette
-// worlds; whole body, 8 materials: 40, 1.87e9 -> 1.94e9 histories/s)
-uint32_t queueCapFp32(int L, uint32_t waves, uint32_t tablesBytes, uint32_t kind)
+// staging level of a run: the requested one, or by default the sampling
+// tables, lowered while the tables leave a wave's pool too few slots. The
+// attenuation coefficients are staged on request only: they are read once an
+// interaction, and the pool slots they would take are worth more.
+uint32_t stageLevelFp32(const dxmc_run_cfg& cfg, const Tables<float>& t, uint32_t W, uint32_t kind)
 {
-    if (waves < 7)
-        return 64;
-    if (kindPalette8(kind))
-        return 48;
-    for (uint32_t cap : { 48u, 40u, 32u })
-        if (residentBlocksFp32(L, waves, tablesBytes + WAVES_PER_BLOCK * queueBytes(cap), kind) >= 7)
-            return cap;
-    return 48;
-}
-
-// staging level of a run: the requested one (lowered until it fits), or by
-// default the attenuation coefficients too when they cost no resident block,
-// else the sampling tables when they cost at most one, else none
-uint32_t stageLevelFp32(const dxmc_run_cfg& cfg, const Tables<float>& t, uint32_t waves, uint32_t kind)
-{
-    // a block gets at most 64 KiB of dynamic LDS
-    constexpr uint32_t ldsPerBlock = 64 * 1024;
-    auto bytes = [&](uint32_t level) {
-        const uint32_t tb = ldsBytes(t, level, cfg.low_energy_correction);
-        return uint64_t(tb) + WAVES_PER_BLOCK * queueBytes(queueCapFp32(cfg.low_energy_correction, waves, tb, kind));
-    };
-    auto fits = [&](uint32_t level) { return bytes(level) <= ldsPerBlock; };
-    if (cfg.lds_tables >= STAGE_NONE && cfg.lds_tables <= STAGE_ALL) {
-        uint32_t level = cfg.lds_tables;
-        while (level > STAGE_NONE && !fits(level))
-            --level;
-        return level;
-    }
-    // The sampling tables are worth a resident block (whole body, 8
-    // materials: 1.04e9 histories/s with them and 4 blocks per CU against
-    // 0.98e9 without and 5); the attenuation coefficients are not worth two
-    // (CT spiral 2.84e9 vs 2.50e9, DX 4.07e9 vs 3.32e9 with 5 and 3 blocks)
-    // and are staged only when they cost none.
-    const uint32_t best = residentBlocksFp32(cfg.low_energy_correction, waves, bytes(STAGE_NONE), kind);
-    auto resident = [&](uint32_t level) { return residentBlocksFp32(cfg.low_energy_correction, waves, static_cast<uint32_t>(bytes(level)), kind); };
-    if (fits(STAGE_ALL) && resident(STAGE_ALL) >= best)
-        return STAGE_ALL;
-    if (fits(STAGE_SMALL) && resident(STAGE_SMALL) + 1 >= best)
-        return STAGE_SMALL;
-    return STAGE_NONE;
+    uint32_t level = cfg.lds_tables >= STAGE_NONE && cfg.lds_tables <= STAGE_ALL ? cfg.lds_tables : STAGE_SMALL;
+    while (level > STAGE_NONE && poolSlots(t, level, cfg.low_energy_correction, blockWaves(W), kind) < POOL_MIN)
+        --level;
+    return level;
 }
 
 void launchFp32(dxmc_ctx* c, const dxmc_run_cfg& cfg, const World<float>& w, const Tables<float>& t, const Exposure<float>* exps,
@@ -504,7 +565,6 @@ void launchFp32(dxmc_ctx* c, const dxmc_run_cfg& cfg, const World<float>& w, con
     // sequence stays valid under stream capture
     auto* nx = historyCounter;
     hipLaunchKernelGGL(clearCounter, dim3(1), dim3(1), 0, c->stream, nx);
-    const uint32_t block = 256;
     World<float> world = w;
     Tables<float> tables = t;
     // the attenuation bounds pay where they also spare the record read
@@ -530,25 +590,25 @@ void launchFp32(dxmc_ctx* c, const dxmc_run_cfg& cfg, const World<float>& w, con
     uint32_t kind = worldKind(world, tables);
     if (kind == WORLD_CODES8 && !world.blocks && cfg.low_energy_correction < 2)
         kind = WORLD_ANY;
-    const uint32_t waves = wavesFp32(cfg.waves_per_simd, cfg.low_energy_correction, kind);
+    const uint32_t waves = wavesFp32(cfg.waves_per_simd, cfg.low_energy_correction);
+    // launches with too few histories for full blocks on every CU get blocks
+    // of fewer waves, spread over the CUs
+    const uint64_t wavesNeeded = (he - hb + 63) / 64;
+    const uint32_t wavesPerBlock = static_cast<uint32_t>(std::clamp<uint64_t>((wavesNeeded + c->numCU - 1) / c->numCU, 1, blockWaves(waves)));
     const uint32_t stage = stageLevelFp32(cfg, tables, waves, kind);
-    const uint32_t tablesBytes = ldsBytes(tables, stage, cfg.low_energy_correction);
-    const uint32_t cap = queueCapFp32(cfg.low_energy_correction, waves, tablesBytes, kind);
-    const uint32_t lds = tablesBytes + WAVES_PER_BLOCK * queueBytes(cap);
-    // default: as many blocks as stay resident on a CU (registers and LDS)
-    const uint32_t perCU = cfg.blocks_per_cu ? cfg.blocks_per_cu : residentBlocksFp32(cfg.low_energy_correction, waves, lds, kind);
-    const uint32_t regen = cfg.regeneration_threshold ? std::min<uint32_t>(cfg.regeneration_threshold, 64u) : 4u;
-    // pending lanes before an interaction pass: at L = 2 a pass costs more
-    // (the impulse-approximation sampler), so it waits for more lanes (CT
-    // spiral 2.39e9 at 20, 2.49e9 at 28, 2.52e9 at 32, 2.45e9 at 40; at
-    // L = 1, 32 cost 3 % and 24 0.5 %)
-    const uint32_t interact = cfg.interaction_threshold ? std::min<uint32_t>(cfg.interaction_threshold, 64u) : cfg.low_energy_correction == 2 ? 32u : 20u;
-    uint64_t grid = static_cast<uint64_t>(c->numCU) * perCU;
-    const uint64_t lanesNeeded = (he - hb + 63) / 64 * 64;
-    grid = std::max<uint64_t>(1, std::min<uint64_t>(grid, (lanesNeeded + block - 1) / block));
+    const uint32_t slots = poolSlots(tables, stage, cfg.low_energy_correction, wavesPerBlock, kind);
+    const uint32_t lds = ldsBytes(tables, stage, cfg.low_energy_correction) + (kind == WORLD_CODES8 && stage >= STAGE_SMALL ? boundsBytes(tables) : 0u) + wavesPerBlock * slots * SLOT_BYTES;
+    const uint32_t perCU = cfg.blocks_per_cu ? cfg.blocks_per_cu : 2u;
+    // lanes without a photon before they are refilled (CT spiral, ms: 8 185,
+    // 12 180; 16 and 20 within 1 % of 12 before the bounds were in LDS)
+    const uint32_t refill = cfg.regeneration_threshold ? std::min<uint32_t>(cfg.regeneration_threshold, 64u) : 12u;
+    // photons due before they interact, at most half the pool (CT spiral,
+    // ms: 32 207, 40 202.4, 48 199.4, 56 198.7 before the bounds were in LDS)
+    const uint32_t interact = std::min<uint32_t>(cfg.interaction_threshold ? std::min<uint32_t>(cfg.interaction_threshold, 64u) : 48u, slots / 2);
+    const uint64_t grid = std::clamp<uint64_t>((wavesNeeded + wavesPerBlock - 1) / wavesPerBlock, 1, static_cast<uint64_t>(c->numCU) * perCU);
     // histories a wave claims per atomic on the global counter
     const uint32_t pool = cfg.queue_depth ? std::clamp<uint32_t>(cfg.queue_depth, 64u, 1u << 16) : 512u;
-    hipLaunchKernelGGL(kernelFor(cfg.low_energy_correction, waves, stage, kind), dim3(static_cast<uint32_t>(grid)), dim3(block), lds, c->stream, world, tables,
-        exps, expStart, nExp, hb, he, cfg.seed, cfg.first_history, tally, ctr, nx, regen, interact, pool, cap);
+    hipLaunchKernelGGL(kernelFor(cfg.low_energy_correction, waves, stage, kind), dim3(static_cast<uint32_t>(grid)), dim3(64 * wavesPerBlock), lds, c->stream,
+        world, tables, exps, expStart, nExp, hb, he, cfg.seed, cfg.first_history, tally, ctr, nx, refill, interact, pool, slots);
 }
 }

@@ -212,13 +212,12 @@ typedef struct {
     uint64_t histories_per_launch; /* 0: automatic; bounds cancel/progress latency; at most 2^32 */
     uint32_t block_size; /* 0: tuned default */
     uint32_t blocks_per_cu; /* FP32 persistent kernel occupancy, 0: tuned default */
-    uint32_t regeneration_threshold; /* FP32: dead lanes per wave before they take queued new photons, 0: tuned */
+    uint32_t regeneration_threshold; /* FP32, FP64: lanes of a wave without a photon to fly before they are refilled, 0: tuned */
     uint32_t flags; /* DXMC_RUN_* bits */
-    uint32_t interaction_threshold; /* FP32: pending interactions per wave before they run, 0: tuned */
-    uint32_t queue_depth; /* FP32: histories a wave claims per refill of its pool, 0: tuned */
-    uint32_t waves_per_simd; /* FP32: kernel variant by register budget, 5, 6 or 7 resident waves per SIMD
-                              * (7 only at L = 0, 1 on worlds of 1-byte codes or palette indices, else 6);
-                              * 0: 7 on those worlds and 6 on others for L = 0, 1, 5 for L = 2 */
+    uint32_t interaction_threshold; /* FP32, FP64: photons of a wave with an interaction due before they run, 0: tuned */
+    uint32_t queue_depth; /* FP32, FP64: histories a wave claims at a time, 0: tuned */
+    uint32_t waves_per_simd; /* FP32: kernel variant by register budget, 6 resident waves per SIMD (6 or more asked
+                              * for) or 4 (fewer); 0: 6 for L = 0, 1, 4 for L = 2 */
     uint32_t lds_tables; /* FP32: sampling tables in LDS, 1 none, 2 all but the attenuation coefficients, 3 all (0: tuned) */
     uint32_t block_bounds; /* FP32 on worlds with 1-byte codes: 1 settle Woodcock decisions from the code range of the
                             * voxel's 8x8x8 block before its own code, 2 from the voxel's code only (same results);
