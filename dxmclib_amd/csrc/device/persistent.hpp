@@ -14,8 +14,8 @@ enum : uint32_t { DEAD = 0, FLYING = 1, PENDING = 2 };
 // get their code width, record width, 24-bit index and bounds table fixed at
 // compile time, so a flight carries no branches on them
 //   WORLD_CODES8    1-byte bounded-density codes (and their block codes
-//                   when the run uses them), 8-byte records, the
-//                   attenuation bounds table, 24-bit index (CT-sized worlds)
+//                   when the run uses them), records of any width, the
+//                   attenuation bounds table, 24-bit index
 //   WORLD_PALETTE8  1-byte palette indices, no codes, no measurement flags,
 //                   24-bit index
 //   WORLD_PALETTE8_MEASURED  the same with measurement flags (forced events)

@@ -854,7 +854,7 @@ int runTransport(dxmc_ctx* c, const dxmc_world* w, const dxmc_tables* t, const d
     DXMC_CHECK(c, hipSetDevice(c->device));
     RunBuffers rb(c);
     int st = uploadExposures(c, x, nExp, rb);
-    if (st)
+    if (st || (st = preparePaletteCodes(c, w, rb.totalHistories)))
         return st;
     const bool counters = (cfg.flags & 1u) != 0 || stats;
     const RunInputs in { static_cast<const Exposure<double>*>(rb.exp64.p), static_cast<const Exposure<float>*>(rb.exp32.p),

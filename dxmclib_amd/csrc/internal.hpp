@@ -214,19 +214,22 @@ struct dxmc_world {
     void* palette = nullptr; // uint2[nPalette] FP32 records, null for 8-byte voxels
     uint32_t voxelBytes = 8;
     uint32_t nPalette = 0;
-    // 8-byte-record worlds: bounded-density code per voxel (u8/u16) and the
-    // interval of each code (DensityBound[nCodes]); codeBytes 0: none
-    void* codes = nullptr;
-    void* bounds = nullptr;
-    uint32_t codeBytes = 0;
-    uint32_t nCodes = 0;
-    // 1-byte code worlds: a 2-byte code per block of 8x8x8 voxels (smallest
-    // | largest code << 8 of a one-material block, else BLOCK_MIXED)
-    void* blocks = nullptr;
-    uint32_t blockDims[3] = { 0, 0, 0 };
-    uint32_t blockShift = 0; // block edge 2^blockShift voxels
-    uint32_t codeMul = 0; // 1-byte codes: (code * codeMul) >> CODE_MUL_SHIFT is the code's material
-    uint64_t bytes = 0;
+    // Bounded-density code per voxel (u8/u16) and the interval of each code
+    // (DensityBound[nCodes]); codeBytes 0: none. 8-byte-record worlds get
+    // them at upload, palette worlds by their first large run (under the
+    // context's lock, hence mutable).
+    mutable void* codes = nullptr;
+    mutable void* bounds = nullptr;
+    mutable uint32_t codeBytes = 0;
+    mutable uint32_t nCodes = 0;
+    mutable bool codesTried = false; // palette worlds: the run-time build was done (or failed)
+    // 1-byte code worlds: a 2-byte code per block of voxels (smallest |
+    // largest code << 8 of a one-material block, else BLOCK_MIXED)
+    mutable void* blocks = nullptr;
+    mutable uint32_t blockDims[3] = { 0, 0, 0 };
+    mutable uint32_t blockShift = 0; // block edge 2^blockShift voxels
+    mutable uint32_t codeMul = 0; // 1-byte codes: (code * codeMul) >> CODE_MUL_SHIFT is the code's material
+    mutable uint64_t bytes = 0;
 };
 
 struct dxmc_tables {
@@ -300,6 +303,13 @@ struct RunBuffers {
     }
 };
 
+// the linear voxel index fits 24-bit products (World::index24)
+inline bool hasIndex24(const dxmc_world* w)
+{
+    const uint64_t slice = uint64_t(w->dims[0]) * w->dims[1];
+    return slice < (uint64_t(1) << 24) && w->dims[2] < (uint32_t(1) << 24) && slice * w->dims[2] < (uint64_t(1) << 32);
+}
+
 template <typename T>
 inline dxmc_dev::World<T> deviceWorld(const dxmc_world* w)
 {
@@ -331,7 +341,7 @@ inline dxmc_dev::World<T> deviceWorld(const dxmc_world* w)
     d.codes = w->codes;
     d.bounds = static_cast<const dxmc_dev::DensityBound*>(w->bounds);
     d.codeBytes = w->codeBytes;
-    d.index24 = uint64_t(d.nx) * d.ny < (uint64_t(1) << 24) && d.nz < (uint32_t(1) << 24) && uint64_t(d.nx) * d.ny * d.nz < (uint64_t(1) << 32);
+    d.index24 = hasIndex24(w);
     d.nxy = d.index24 ? d.nx * d.ny : 0;
     d.blocks = static_cast<const uint16_t*>(w->blocks);
     d.bnx = w->blockDims[0];
@@ -380,6 +390,8 @@ inline std::tuple<const void*, const void*, int, int> tuneKey(const dxmc_world* 
 // autotune.hip
 int autotune(dxmc_ctx* c, const dxmc_world* w, const dxmc_tables* t, const dxmc_exposure* x, uint64_t nExp, const dxmc_run_cfg& base,
     uint64_t trialHistories, dxmc_run_cfg& best, dxmc_tune_report* report);
+// codes of a palette world, for a run of so many histories (world.hip)
+int preparePaletteCodes(dxmc_ctx* c, const dxmc_world* w, uint64_t histories);
 int runTransport(dxmc_ctx* c, const dxmc_world* w, const dxmc_tables* t, const dxmc_exposure* x, uint64_t nExp, const dxmc_run_cfg& cfg,
     dxmc_tally* tally, const dxmc_run_monitor* monitor, dxmc_run_stats* stats);
 // device inputs of a run's launches: exposure records of both precisions,

@@ -148,7 +148,7 @@ __global__ __launch_bounds__(64 * blockWaves(W)) __attribute__((amdgpu_waves_per
     const float inv[3] = { 1.0f / w.spacing[0], 1.0f / w.spacing[1], 1.0f / w.spacing[2] };
     // the world's layout, fixed by K where it can be
     const uint32_t codeBytes = K == WORLD_CODES8 ? 1u : kindPalette8(K) ? 0u : w.codeBytes;
-    const uint32_t voxelBytes = kindPalette8(K) ? 1u : K == WORLD_CODES8 ? 8u : w.voxelBytes;
+    const uint32_t voxelBytes = kindPalette8(K) ? 1u : w.voxelBytes; // (kinds without codes)
     const bool index24 = K != WORLD_ANY || w.index24 != 0;
     const bool sumBounds = K == WORLD_CODES8 || (K == WORLD_ANY && t.lutSumBound != nullptr);
     // global index of the launch's first history (PCG increments of pooled photons)
@@ -447,8 +447,11 @@ __global__ __launch_bounds__(64 * blockWaves(W)) __attribute__((amdgpu_waves_per
                             prob = lo;
                         }
                         if (!settled) {
-                            if (codeBytes != 0)
-                                density = __uint_as_float(static_cast<const uint2*>(w.voxels)[idx].x);
+                            // the record's density, from the FP64 array it was
+                            // rounded from (one layout for all code worlds); a
+                            // code of one density names it
+                            if (codeBytes != 0 && dLo != dHi)
+                                density = static_cast<float>(w.density[idx]);
                             float att[3];
                             attenuationAt(t, matMeas, lp, att); // 24-bit row product: flag ignored
                             prob = ((att[0] + att[1]) + att[2]) * density * majInv;
@@ -521,7 +524,7 @@ uint32_t worldKind(const World<float>& w, const Tables<float>& t)
 {
     if (!w.index24)
         return WORLD_ANY;
-    if (w.codeBytes == 1 && w.voxelBytes == 8 && t.lutSumBound)
+    if (w.codeBytes == 1 && t.lutSumBound)
         return WORLD_CODES8;
     if (w.codeBytes == 0 && w.voxelBytes == 1 && !t.lutSumBound)
         return w.measurement ? WORLD_PALETTE8_MEASURED : WORLD_PALETTE8;
@@ -574,13 +577,12 @@ void launchFp32(dxmc_ctx* c, const dxmc_run_cfg& cfg, const World<float>& w, con
         world.codeBytes = 0;
         tables.lutSumBound = nullptr;
     }
-    // the block code ranges spare most steps the code gather, and pay
-    // wherever that gather misses the caches or 7 waves per SIMD hide the
-    // block entry's loads (measured: CT spiral +3 % at L = 1, whole body
-    // +39 %); at L = 2, with 5 waves per SIMD, the longer chain of a step
-    // whose draw falls in the block's band costs more than a code gather
-    // from the Infinity Cache saves (CT spiral -6.5 %, its 79 MB codes
-    // cached; whole body +13 %, its 629 MB not)
+    // the block code ranges spare most steps the code gather (CT spiral 180
+    // ms against 277 without, CT-number world 34.6 against 46.8, DX 19.6
+    // against 25.8); at L = 2, with 4 waves per SIMD, the longer chain of a
+    // step whose draw falls in the block's band costs more than a code gather
+    // from the Infinity Cache saves (401x333x151: 41.1 ms against 39.4), but
+    // not more than one from HBM
     constexpr uint64_t INFINITY_CACHE_BYTES = uint64_t(256) << 20;
     const uint64_t codeArrayBytes = uint64_t(world.nx) * world.ny * world.nz * world.codeBytes;
     const bool blocksOn = world.codeBytes == 1 && world.blocks
@@ -599,9 +601,10 @@ void launchFp32(dxmc_ctx* c, const dxmc_run_cfg& cfg, const World<float>& w, con
     const uint32_t slots = poolSlots(tables, stage, cfg.low_energy_correction, wavesPerBlock, kind);
     const uint32_t lds = ldsBytes(tables, stage, cfg.low_energy_correction) + (kind == WORLD_CODES8 && stage >= STAGE_SMALL ? boundsBytes(tables) : 0u) + wavesPerBlock * slots * SLOT_BYTES;
     const uint32_t perCU = cfg.blocks_per_cu ? cfg.blocks_per_cu : 2u;
-    // lanes without a photon before they are refilled (CT spiral, ms: 8 185,
-    // 12 180; 16 and 20 within 1 % of 12 before the bounds were in LDS)
-    const uint32_t refill = cfg.regeneration_threshold ? std::min<uint32_t>(cfg.regeneration_threshold, 64u) : 12u;
+    // lanes without a photon before they are refilled (ms: CT spiral 8 185,
+    // 12 180.5, 16 178.8, 20 181; DX 12 19.6, 16 19.3; impulse approximation
+    // 12 40.9, 16 39.4, 20 38.3, 24 38.7)
+    const uint32_t refill = cfg.regeneration_threshold ? std::min<uint32_t>(cfg.regeneration_threshold, 64u) : cfg.low_energy_correction == 2 ? 20u : 16u;
     // photons due before they interact, at most half the pool (CT spiral,
     // ms: 32 207, 40 202.4, 48 199.4, 56 198.7 before the bounds were in LDS)
     const uint32_t interact = std::min<uint32_t>(cfg.interaction_threshold ? std::min<uint32_t>(cfg.interaction_threshold, 64u) : 48u, slots / 2);

@@ -308,7 +308,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 8))) voi
                             settled = (f2 < lo) | (f2 > hi);
                             real = f2 < lo;
                             if (!settled)
-                                evaluate(__uint_as_float(static_cast<const uint2*>(w.voxels)[idx].x));
+                                evaluate(static_cast<float>(w.density[idx]));
                         }
                     } else {
                         float density;

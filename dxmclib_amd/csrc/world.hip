@@ -17,6 +17,8 @@
 //   boundCodes<I>   for those worlds, a 1- or 2-byte code per voxel naming
 //                   its material and a density interval (Woodcock decisions
 //                   settled from the interval at most steps)
+//   paletteBounds, paletteCodes  the same codes for worlds of palette
+//                   indices, made by the first large FP32 or FP64 run
 //   blockCodes      with 1-byte codes, the code range of every block of
 //                   8^3 to 64^3 voxels that holds one material (decisions
 //                   settled from the block's interval without reading the
@@ -270,6 +272,73 @@ __global__ __launch_bounds__(SCAN_BLOCK) void boundCodes(const uint2* __restrict
     }
 }
 
+// Codes of a palette world's records, as boundCodes gives them: each
+// material's density range (of its records) in 'bins' equal parts. A code's
+// interval is that of the records in it, so a code with one density names it
+// exactly. One workgroup; a record that is not a number widens every interval
+// to all numbers, which settles nothing.
+__global__ __launch_bounds__(1024) void paletteBounds(const uint2* __restrict__ palette, uint32_t n, uint32_t bins, uint8_t* __restrict__ codeOf,
+    dxmc_dev::DensityBound* __restrict__ bounds)
+{
+    __shared__ unsigned int low[256], high[256], codeLow[256], codeHigh[256], notNumber;
+    // order-preserving image of a float
+    auto key = [](float v) {
+        const uint32_t b = __float_as_uint(v);
+        return (b >> 31) ? ~b : (b | 0x80000000u);
+    };
+    auto value = [](uint32_t k) { return __uint_as_float((k >> 31) ? (k & 0x7fffffffu) : ~k); };
+    if (threadIdx.x < 256) {
+        low[threadIdx.x] = codeLow[threadIdx.x] = 0xffffffffu;
+        high[threadIdx.x] = codeHigh[threadIdx.x] = 0u;
+    }
+    if (threadIdx.x == 0)
+        notNumber = 0;
+    __syncthreads();
+    for (uint32_t i = threadIdx.x; i < n; i += 1024) {
+        const float d = __uint_as_float(palette[i].x);
+        if (d == d) {
+            atomicMin(&low[palette[i].y & 0xffu], key(d));
+            atomicMax(&high[palette[i].y & 0xffu], key(d));
+        } else {
+            atomicOr(&notNumber, 1u);
+        }
+    }
+    __syncthreads();
+    for (uint32_t i = threadIdx.x; i < n; i += 1024) {
+        const float d = __uint_as_float(palette[i].x);
+        const uint32_t m = palette[i].y & 0xffu;
+        const float a = value(low[m]), b = value(high[m]);
+        // not decreasing with d, so a material's codes are in density order
+        const double x = b > a && d == d ? (static_cast<double>(d) - a) * (bins / (static_cast<double>(b) - a)) : 0.0;
+        const uint32_t code = m * bins + static_cast<uint32_t>(min(max(x, 0.0), static_cast<double>(bins - 1)));
+        codeOf[i] = static_cast<uint8_t>(code);
+        if (d == d) {
+            atomicMin(&codeLow[code], key(d));
+            atomicMax(&codeHigh[code], key(d));
+        }
+    }
+    __syncthreads();
+    if (threadIdx.x < 256) {
+        dxmc_dev::DensityBound e { 1.0f, 0.0f, threadIdx.x / bins, 0u };
+        if (codeHigh[threadIdx.x] != 0)
+            e = { value(codeLow[threadIdx.x]), value(codeHigh[threadIdx.x]), threadIdx.x / bins, 0u };
+        if (notNumber)
+            e = { -HUGE_VALF, HUGE_VALF, threadIdx.x / bins, 0u };
+        if (threadIdx.x == dxmc_dev::MIXED_CODE)
+            e = { 0.0f, 0.0f, 0u, 0u };
+        bounds[threadIdx.x] = e;
+    }
+}
+
+template <typename I>
+__global__ __launch_bounds__(SCAN_BLOCK) void paletteCodes(const I* __restrict__ voxels, const uint8_t* __restrict__ codeOf, uint64_t n,
+    uint8_t* __restrict__ codes)
+{
+    const uint64_t stride = static_cast<uint64_t>(gridDim.x) * SCAN_BLOCK;
+    for (uint64_t i = static_cast<uint64_t>(blockIdx.x) * SCAN_BLOCK + threadIdx.x; i < n; i += stride)
+        codes[i] = codeOf[voxels[i]];
+}
+
 // Block code of every block of 2^shift voxels per edge of a 1-byte code
 // world (the blocks of the last row, column and slice clipped to the grid),
 // one workgroup per block: smallest code | largest code << 8 when every
@@ -336,6 +405,41 @@ float floatAbove(double v)
     if (static_cast<double>(f) < v)
         f = std::nextafter(f, HUGE_VALF);
     return f;
+}
+
+// Block codes of a world with 1-byte codes of 'bins' a material, and the
+// multiplier that gives a code's material.
+int buildBlockCodes(dxmc_ctx* c, const dxmc_world* w, uint32_t bins)
+{
+    const auto* bnd = static_cast<const dxmc_dev::DensityBound*>(w->bounds);
+    // (code * codeMul) >> CODE_MUL_SHIFT = code / bins for every code below
+    // 256: codeMul exceeds 2^20 / bins by less than 1, which adds less than
+    // 256 / 2^20 to a quotient whose fraction is at most 1 - 1/bins
+    w->codeMul = ((uint32_t(1) << dxmc_dev::CODE_MUL_SHIFT) + bins - 1) / bins;
+    // block edge: the smallest of 8, 16, 32 and 64 voxels whose table fits
+    // 64 KiB, so that it stays in the caches (CT spiral, 512x512x300: 16,
+    // 39 KB, 4.27e9 -> 4.44e9 histories/s against 8; whole body,
+    // 1024x1024x600: 32, 39 KB, 1.95e9 -> 2.09e9; a larger block is more
+    // often mixed, but its entry is far more often cached)
+    uint32_t shift = dxmc_dev::BLOCK_SHIFT_MIN, bd[3];
+    for (;; ++shift) {
+        const uint32_t E = 1u << shift;
+        for (int i = 0; i < 3; ++i)
+            bd[i] = (w->dims[i] + E - 1) / E;
+        if (uint64_t(bd[0]) * bd[1] * bd[2] * sizeof(uint16_t) <= dxmc_dev::BLOCK_TABLE_BYTES || shift == dxmc_dev::BLOCK_SHIFT_MAX)
+            break;
+    }
+    const uint64_t nBlocks = uint64_t(bd[0]) * bd[1] * bd[2];
+    if (int st = c->alloc(&w->blocks, nBlocks * sizeof(uint16_t)))
+        return st;
+    hipLaunchKernelGGL(blockCodes, dim3(gridFor(nBlocks, 1, SCAN_GRID * 4)), dim3(SCAN_BLOCK), 0, c->stream, static_cast<const uint8_t*>(w->codes), bnd,
+        w->dims[0], w->dims[1], w->dims[2], shift, bd[0], bd[1], nBlocks, static_cast<uint16_t*>(w->blocks));
+    if (int st = c->check(hipGetLastError()))
+        return st;
+    for (int i = 0; i < 3; ++i)
+        w->blockDims[i] = bd[i];
+    w->blockShift = shift;
+    return DXMC_OK;
 }
 
 // Bounded-density codes of an 8-byte-record world without measurement
@@ -408,34 +512,7 @@ int buildBoundCodes(dxmc_ctx* c, dxmc_world* w, ScanResult* dev, const ScanResul
     w->nCodes = nCodes;
     if (codeBytes != 1)
         return DXMC_OK;
-    // (code * codeMul) >> CODE_MUL_SHIFT = code / bins for every code below
-    // 256: codeMul exceeds 2^20 / bins by less than 1, which adds less than
-    // 256 / 2^20 to a quotient whose fraction is at most 1 - 1/bins
-    w->codeMul = ((uint32_t(1) << dxmc_dev::CODE_MUL_SHIFT) + bins - 1) / bins;
-    // block edge: the smallest of 8, 16, 32 and 64 voxels whose table fits
-    // 64 KiB, so that it stays in the caches (CT spiral, 512x512x300: 16,
-    // 39 KB, 4.27e9 -> 4.44e9 histories/s against 8; whole body,
-    // 1024x1024x600: 32, 39 KB, 1.95e9 -> 2.09e9; a larger block is more
-    // often mixed, but its entry is far more often cached)
-    uint32_t shift = dxmc_dev::BLOCK_SHIFT_MIN, bd[3];
-    for (;; ++shift) {
-        const uint32_t E = 1u << shift;
-        for (int i = 0; i < 3; ++i)
-            bd[i] = (w->dims[i] + E - 1) / E;
-        if (uint64_t(bd[0]) * bd[1] * bd[2] * sizeof(uint16_t) <= dxmc_dev::BLOCK_TABLE_BYTES || shift == dxmc_dev::BLOCK_SHIFT_MAX)
-            break;
-    }
-    const uint64_t nBlocks = uint64_t(bd[0]) * bd[1] * bd[2];
-    if ((st = c->alloc(&w->blocks, nBlocks * sizeof(uint16_t))))
-        return st;
-    hipLaunchKernelGGL(blockCodes, dim3(gridFor(nBlocks, 1, SCAN_GRID * 4)), block, 0, c->stream, static_cast<const uint8_t*>(w->codes), bnd,
-        w->dims[0], w->dims[1], w->dims[2], shift, bd[0], bd[1], nBlocks, static_cast<uint16_t*>(w->blocks));
-    if ((st = c->check(hipGetLastError())))
-        return st;
-    for (int i = 0; i < 3; ++i)
-        w->blockDims[i] = bd[i];
-    w->blockShift = shift;
-    return DXMC_OK;
+    return buildBlockCodes(c, w, bins);
 }
 
 int fillVoxelRecords(dxmc_ctx* c, dxmc_world* w, ScanResult* dev, ScanResult& host)
@@ -484,6 +561,50 @@ int fillVoxelRecords(dxmc_ctx* c, dxmc_world* w, ScanResult* dev, ScanResult& ho
 }
 
 } // namespace
+
+namespace dxmc_backend {
+
+// Gives a palette world the 1-byte codes and block codes that settle most
+// Woodcock decisions without its voxels' records. Made by the first run of
+// 2^22 histories or more rather than at upload: three launches and a byte a
+// voxel, about 60 us with its allocations, which a run of a millisecond
+// repays and a small one does not. Worlds with measurement flags, more than
+// 64 materials or no 24-bit index keep their records.
+int preparePaletteCodes(dxmc_ctx* c, const dxmc_world* w, uint64_t histories)
+{
+    if (histories < (uint64_t(1) << 22) || w->codesTried || w->voxelBytes > 2 || w->hasMeasurement || w->nMaterials > 64 || !hasIndex24(w))
+        return DXMC_OK;
+    w->codesTried = true;
+    const uint32_t bins = 255 / w->nMaterials;
+    DeviceBuffer codeOf(c);
+    auto drop = [&](int st) {
+        c->release(w->codes);
+        c->release(w->bounds);
+        w->codes = w->bounds = nullptr;
+        return st == DXMC_ERR_MEMORY ? DXMC_OK : st; // no room for them: the run reads the records
+    };
+    int st = DXMC_OK;
+    if ((st = codeOf.alloc(w->nPalette)) || (st = c->alloc(&w->bounds, 256 * sizeof(dxmc_dev::DensityBound))) || (st = c->alloc(&w->codes, w->n)))
+        return drop(st);
+    auto* of = static_cast<uint8_t*>(codeOf.p);
+    hipLaunchKernelGGL(paletteBounds, dim3(1), dim3(1024), 0, c->stream, static_cast<const uint2*>(w->palette), w->nPalette, bins, of,
+        static_cast<dxmc_dev::DensityBound*>(w->bounds));
+    const dim3 grid(gridFor(w->n, SCAN_BLOCK, SCAN_GRID)), block(SCAN_BLOCK);
+    if (w->voxelBytes == 1)
+        hipLaunchKernelGGL(paletteCodes<uint8_t>, grid, block, 0, c->stream, static_cast<const uint8_t*>(w->voxels), of, w->n,
+            static_cast<uint8_t*>(w->codes));
+    else
+        hipLaunchKernelGGL(paletteCodes<uint16_t>, grid, block, 0, c->stream, static_cast<const uint16_t*>(w->voxels), of, w->n,
+            static_cast<uint8_t*>(w->codes));
+    if ((st = c->check(hipGetLastError())) || (st = buildBlockCodes(c, w, bins)))
+        return drop(st);
+    w->nCodes = 256;
+    w->codeBytes = 1; // the codes are complete on the stream before any kernel of the run
+    w->bytes += w->n + 256 * sizeof(dxmc_dev::DensityBound) + uint64_t(w->blockDims[0]) * w->blockDims[1] * w->blockDims[2] * sizeof(uint16_t);
+    return DXMC_OK;
+}
+
+}
 
 extern "C" {
 
