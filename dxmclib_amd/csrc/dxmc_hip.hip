@@ -284,6 +284,9 @@ int dxmc_hip_ctx_create(int device, dxmc_ctx** out)
         uint64_t keep = UINT64_MAX;
         hipMemPoolSetAttribute(pool, hipMemPoolAttrReleaseThreshold, &keep);
     }
+    // page-locked ring of the small transfers (without it they go direct)
+    if (hipHostMalloc(reinterpret_cast<void**>(&c->ring), dxmc_ctx::RING_BYTES, hipHostMallocDefault) != hipSuccess)
+        c->ring = nullptr;
     hipGetLastError();
     hipDeviceProp_t prop;
     if (hipGetDeviceProperties(&prop, device) == hipSuccess) {
@@ -306,6 +309,8 @@ int dxmc_hip_ctx_destroy(dxmc_ctx* c)
     hipEventDestroy(c->ev0);
     hipEventDestroy(c->ev1);
     c->releaseStaging();
+    if (c->ring)
+        hipHostFree(c->ring);
     hipFree(c->historyCounter);
     hipStreamDestroy(c->stream);
     threadErrors().erase(c);
@@ -481,14 +486,11 @@ int dxmc_hip_tally_download(dxmc_ctx* c, const dxmc_tally* t, double* dose, uint
         if (int st = launchNormalize(c, t, nullptr, -1, 0, 0.0))
             return st;
     }
-    // through the context's page-locked staging chunks (a direct copy into
-    // pageable memory ran at about 7 GB/s), or direct into page-locked memory
-    int st = DXMC_OK;
-    if (dose && (st = c->download(dose, t->dose, t->n * sizeof(double))))
-        return st;
-    if (nEvents && (st = c->download(nEvents, t->nEvents, t->n * sizeof(uint32_t))))
-        return st;
-    if (variance && (st = c->download(variance, t->variance, t->n * sizeof(double))))
+    // through the context's page-locked memory (a direct copy into pageable
+    // memory ran at about 7 GB/s), or direct into page-locked memory
+    const dxmc_ctx::Fetch list[3] = { { dose, t->dose, dose ? t->n * sizeof(double) : 0 }, { nEvents, t->nEvents, nEvents ? t->n * sizeof(uint32_t) : 0 },
+        { variance, t->variance, variance ? t->n * sizeof(double) : 0 } };
+    if (int st = c->download(list, 3))
         return st;
     DXMC_CHECK(c, hipStreamSynchronize(c->stream));
     return DXMC_OK;
@@ -729,24 +731,26 @@ int dxmc_hip_sample_particles(dxmc_ctx* c, const dxmc_world* w, const dxmc_table
 
 namespace dxmc_backend {
 
-// exposures -> device records of both precisions + history prefix sums
-int uploadExposures(dxmc_ctx* c, const dxmc_exposure* x, uint64_t nExp, RunBuffers& rb)
+// exposures -> device records of the run's precision, history prefix sums and
+// cleared counters, as one block in one transfer
+int uploadExposures(dxmc_ctx* c, const dxmc_exposure* x, uint64_t nExp, int precision, RunBuffers& rb)
 {
-    std::vector<Exposure<double>> e64(nExp);
-    std::vector<Exposure<float>> e32(nExp);
-    std::vector<uint64_t> start(nExp + 1, 0);
+    const auto aligned = [](size_t b) { return (b + 63) & ~size_t { 63 }; };
+    const size_t record = precision == DXMC_PRECISION_FP64 ? sizeof(Exposure<double>) : sizeof(Exposure<float>);
+    rb.startAt = aligned(nExp * record);
+    rb.countersAt = rb.startAt + aligned((nExp + 1) * sizeof(uint64_t));
+    std::vector<unsigned char> host(rb.countersAt + sizeof(Counters)); // zero: the counters'
+    rb.start.assign(nExp + 1, 0);
     for (uint64_t i = 0; i < nExp; ++i) {
-        e64[i] = toDevice<double>(x[i]);
-        e32[i] = toDevice<float>(x[i]);
-        start[i + 1] = start[i] + x[i].n_histories;
+        if (precision == DXMC_PRECISION_FP64)
+            reinterpret_cast<Exposure<double>*>(host.data())[i] = toDevice<double>(x[i]);
+        else
+            reinterpret_cast<Exposure<float>*>(host.data())[i] = toDevice<float>(x[i]);
+        rb.start[i + 1] = rb.start[i] + x[i].n_histories;
     }
-    rb.totalHistories = start[nExp];
-    rb.start = start;
-    int st;
-    if ((st = rb.exp64.upload(e64.data(), nExp * sizeof(Exposure<double>))) || (st = rb.exp32.upload(e32.data(), nExp * sizeof(Exposure<float>)))
-        || (st = rb.startDev.upload(start.data(), (nExp + 1) * sizeof(uint64_t))) || (st = rb.counters.zeros(sizeof(Counters))))
-        return st;
-    return DXMC_OK;
+    std::memcpy(host.data() + rb.startAt, rb.start.data(), (nExp + 1) * sizeof(uint64_t));
+    rb.totalHistories = rb.start[nExp];
+    return rb.block.upload(host.data(), host.size());
 }
 
 int launchTallyMip(dxmc_ctx* c, const dxmc_tally* tally, const dxmc_world* w, int axis, float* image, uint64_t& width, uint64_t& height)
@@ -853,12 +857,14 @@ int runTransport(dxmc_ctx* c, const dxmc_world* w, const dxmc_tables* t, const d
 {
     DXMC_CHECK(c, hipSetDevice(c->device));
     RunBuffers rb(c);
-    int st = uploadExposures(c, x, nExp, rb);
+    int st = uploadExposures(c, x, nExp, cfg.precision, rb);
     if (st || (st = preparePaletteCodes(c, w, rb.totalHistories)))
         return st;
     const bool counters = (cfg.flags & 1u) != 0 || stats;
-    const RunInputs in { static_cast<const Exposure<double>*>(rb.exp64.p), static_cast<const Exposure<float>*>(rb.exp32.p),
-        static_cast<const uint64_t*>(rb.startDev.p), rb.start.data(), rb.totalHistories, counters ? static_cast<Counters*>(rb.counters.p) : nullptr,
+    const bool fp64 = cfg.precision == DXMC_PRECISION_FP64;
+    auto* counterBlock = rb.at<Counters>(rb.countersAt);
+    const RunInputs in { fp64 ? rb.at<const Exposure<double>>(0) : nullptr, fp64 ? nullptr : rb.at<const Exposure<float>>(0),
+        rb.at<const uint64_t>(rb.startAt), rb.start.data(), rb.totalHistories, counters ? counterBlock : nullptr,
         static_cast<unsigned long long*>(c->historyCounter) };
     double kernelMs = 0;
     uint64_t launches = 0;
@@ -866,7 +872,7 @@ int runTransport(dxmc_ctx* c, const dxmc_world* w, const dxmc_tables* t, const d
         return st;
     if (stats) {
         Counters h {};
-        if (int e = c->download(&h, rb.counters.p, sizeof(Counters)))
+        if (int e = c->download(&h, counterBlock, sizeof(Counters)))
             return e;
         stats->histories = in.total;
         stats->steps = h.steps;

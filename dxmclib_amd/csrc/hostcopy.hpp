@@ -1,10 +1,12 @@
 // Host-side copies of the staged transfers, free of HIP so that they build
 // and are tested on any host.
 //
-// CopyHelpers: three persistent helper threads that copy parts of one block
-// while the calling thread copies the first part. One core copies 27-30 GB/s
-// out of page-locked memory on the MI355X host, four 80-100 GB/s, while the
-// device-to-host DMA of a staging chunk runs at 53-57 GB/s. A context starts
+// CopyHelpers: persistent helper threads that copy parts of one block while
+// the calling thread copies the first part. One core copies 27-30 GB/s out of
+// page-locked memory on the MI355X host, four 80-100 GB/s, while the
+// device-to-host DMA of a staging chunk runs at 53-57 GB/s; but result arrays
+// are mostly fresh memory, whose pages are cleared at the first touch, and
+// four threads then keep up with 31 GB/s, eight with 44. A context starts
 // its helpers with its staging chunks and stops them with them; its lock
 // keeps one copy at a time. When the threads cannot start, every copy runs
 // on the calling thread.
@@ -21,9 +23,9 @@ namespace dxmc_backend {
 
 class CopyHelpers {
 public:
-    static constexpr int PARTS = 4;
+    static constexpr int PARTS = 8;
     // blocks below this are copied by the calling thread alone
-    static constexpr std::size_t PART_MIN = std::size_t { 1 } << 22;
+    static constexpr std::size_t PART_MIN = std::size_t { 1 } << 19;
 
     CopyHelpers() = default;
     CopyHelpers(const CopyHelpers&) = delete;
