@@ -9,8 +9,8 @@
 //                   :52-58), whether any measurement flag is set, and the
 //                   FP64 density copy the normalisation reads
 //   paletteInsert   distinct FP32 voxel records (density bits, material |
-//                   measurement << 24) into an open-addressing hash table
-//   paletteCompact  palette index of each distinct record
+//                   measurement << 24) into an open-addressing hash table,
+//                   with a palette index each
 //   paletteIndex<I> 1- or 2-byte palette index of every voxel
 //   packVoxels      8-byte records when there are more than 65536
 //                   distinct records
@@ -45,7 +45,6 @@ constexpr uint32_t PALETTE_LIMIT = 65536;
 constexpr uint32_t HASH_BITS = 20;
 constexpr uint32_t HASH_SLOTS = 1u << HASH_BITS;
 constexpr uint32_t HASH_PROBES = 256; // longer probe sequences fall back to 8-byte records
-constexpr uint32_t COMPACT_BLOCK = 1024;
 constexpr unsigned long long EMPTY = ~0ull; // not a record key: a tag is at most 0xff0000ff
 
 uint32_t gridFor(uint64_t n, uint32_t block, uint32_t cap) { return static_cast<uint32_t>(std::min<uint64_t>((n + block - 1) / block, cap)); }
@@ -139,75 +138,79 @@ __global__ __launch_bounds__(SCAN_BLOCK) void scanWorld(const uint8_t* __restric
     }
 }
 
-// state[0]: distinct records inserted; state[1]: overflow (too many
-// records, or a probe sequence longer than HASH_PROBES). Every thread stops
-// at its next voxel once state[1] is set.
+// Distinct records into the hash table; the thread that places a record gives
+// it the next palette index. state[0]: distinct records placed; state[1]:
+// overflow (too many records, or a probe sequence longer than HASH_PROBES):
+// every thread stops at its next record that its block has not met.
+// A block remembers records it has placed or found, one per slot of 'seen',
+// and lanes that meet the same new record leave it to one of them: worlds have
+// far fewer records than voxels, and looking each voxel's up in the table made
+// all CUs read and swap the same few lines past L1 (3 M voxels of 7 records:
+// 1.08 ms, with 'seen' 0.68, with one lane a record 0.027; a separate kernel
+// that numbered the records took 0.58).
 __global__ __launch_bounds__(SCAN_BLOCK) void paletteInsert(const uint8_t* __restrict__ mat, const double* __restrict__ dens,
-    const uint8_t* __restrict__ meas, uint64_t n, unsigned long long* keys, unsigned int* state)
+    const uint8_t* __restrict__ meas, uint64_t n, unsigned long long* keys, uint32_t* __restrict__ rank, uint2* __restrict__ palette,
+    unsigned int* state)
 {
+    constexpr uint32_t SEEN = 2048;
+    __shared__ unsigned long long seen[SEEN];
+    for (uint32_t i = threadIdx.x; i < SEEN; i += SCAN_BLOCK)
+        seen[i] = EMPTY;
+    __syncthreads();
+    // false: no room for k (overflow flagged)
+    auto place = [&](unsigned long long k) {
+        uint32_t h = hashSlot(k);
+        unsigned long long* mine = &seen[h % SEEN];
+        for (uint32_t p = 0; p < HASH_PROBES; ++p, h = (h + 1) & (HASH_SLOTS - 1)) {
+            unsigned long long cur = __hip_atomic_load(&keys[h], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (cur == EMPTY) {
+                cur = atomicCAS(&keys[h], EMPTY, k);
+                if (cur == EMPTY) {
+                    const uint32_t r = atomicAdd(&state[0], 1u);
+                    if (r >= PALETTE_LIMIT) {
+                        atomicOr(&state[1], 1u);
+                        return false;
+                    }
+                    rank[h] = r;
+                    palette[r] = make_uint2(static_cast<uint32_t>(k), static_cast<uint32_t>(k >> 32));
+                    cur = k;
+                }
+            }
+            if (cur == k) {
+                __hip_atomic_store(mine, k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                return true;
+            }
+        }
+        atomicOr(&state[1], 1u);
+        return false;
+    };
     unsigned long long last = EMPTY;
     const uint64_t stride = static_cast<uint64_t>(gridDim.x) * SCAN_BLOCK;
     for (uint64_t i = static_cast<uint64_t>(blockIdx.x) * SCAN_BLOCK + threadIdx.x; i < n; i += stride) {
+        const unsigned long long k = recordKey(mat, dens, meas, i);
+        bool fresh = k != last && __hip_atomic_load(&seen[hashSlot(k) % SEEN], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) != k;
+        last = k;
+        if (!fresh)
+            continue;
         if (__hip_atomic_load(&state[1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
             return;
-        const unsigned long long k = recordKey(mat, dens, meas, i);
-        if (k == last)
-            continue;
-        last = k;
-        uint32_t h = hashSlot(k);
-        bool placed = false;
-        for (uint32_t p = 0; p < HASH_PROBES; ++p, h = (h + 1) & (HASH_SLOTS - 1)) {
-            const unsigned long long cur = __hip_atomic_load(&keys[h], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            if (cur == k) {
-                placed = true;
+        // a few records shared by lanes, then each lane its own
+        bool full = false;
+        for (int round = 0; round < 4; ++round) {
+            const uint64_t mask = __ballot(fresh);
+            if (mask == 0)
                 break;
-            }
-            if (cur != EMPTY)
-                continue;
-            const unsigned long long prev = atomicCAS(&keys[h], EMPTY, k);
-            if (prev == EMPTY) {
-                if (atomicAdd(&state[0], 1u) >= PALETTE_LIMIT)
-                    atomicOr(&state[1], 1u);
-                placed = true;
-                break;
-            }
-            if (prev == k) {
-                placed = true;
-                break;
+            const int leader = __ffsll(static_cast<unsigned long long>(mask)) - 1;
+            if (fresh && k == __shfl(k, leader)) {
+                fresh = false;
+                if (static_cast<int>(__lane_id()) == leader)
+                    full = !place(k);
             }
         }
-        if (!placed) {
-            atomicOr(&state[1], 1u);
+        if (fresh)
+            full = !place(k);
+        if (full)
             return;
-        }
-    }
-}
-
-// One block: thread t owns slots t, t + 1024, ...; ranks follow (t, slot).
-__global__ __launch_bounds__(COMPACT_BLOCK) void paletteCompact(const unsigned long long* __restrict__ keys, uint32_t* __restrict__ rank,
-    uint2* __restrict__ palette)
-{
-    __shared__ uint32_t count[COMPACT_BLOCK];
-    const uint32_t t = threadIdx.x;
-    uint32_t c = 0;
-    for (uint32_t j = t; j < HASH_SLOTS; j += COMPACT_BLOCK)
-        c += keys[j] != EMPTY;
-    count[t] = c;
-    __syncthreads();
-    for (uint32_t off = 1; off < COMPACT_BLOCK; off <<= 1) {
-        const uint32_t v = t >= off ? count[t - off] : 0u;
-        __syncthreads();
-        count[t] += v;
-        __syncthreads();
-    }
-    uint32_t r = count[t] - c;
-    for (uint32_t j = t; j < HASH_SLOTS; j += COMPACT_BLOCK) {
-        const unsigned long long k = keys[j];
-        if (k != EMPTY) {
-            rank[j] = r;
-            palette[r] = make_uint2(static_cast<uint32_t>(k), static_cast<uint32_t>(k >> 32));
-            ++r;
-        }
     }
 }
 
@@ -521,23 +524,25 @@ int fillVoxelRecords(dxmc_ctx* c, dxmc_world* w, ScanResult* dev, ScanResult& ho
     const auto* mat = static_cast<const uint8_t*>(w->material);
     const auto* dens = static_cast<const double*>(w->density);
     const auto* meas = static_cast<const uint8_t*>(w->measurement);
-    DeviceBuffer keys(c), rank(c);
+    DeviceBuffer keys(c), rank(c), records(c);
     int st = DXMC_OK;
     if ((st = keys.alloc(HASH_SLOTS * sizeof(unsigned long long))) || (st = rank.zeros(HASH_SLOTS * sizeof(uint32_t)))
+        || (st = records.alloc(PALETTE_LIMIT * sizeof(uint2)))
         || (st = c->check(hipMemsetAsync(keys.p, 0xff, HASH_SLOTS * sizeof(unsigned long long), c->stream))))
         return st;
     auto* k = static_cast<unsigned long long*>(keys.p);
-    hipLaunchKernelGGL(paletteInsert, dim3(gridFor(n, SCAN_BLOCK, INSERT_GRID)), dim3(SCAN_BLOCK), 0, c->stream, mat, dens, meas, n, k, dev->palette);
+    auto* r = static_cast<uint32_t*>(rank.p);
+    hipLaunchKernelGGL(paletteInsert, dim3(gridFor(n, SCAN_BLOCK, INSERT_GRID)), dim3(SCAN_BLOCK), 0, c->stream, mat, dens, meas, n, k, r,
+        static_cast<uint2*>(records.p), dev->palette);
     if ((st = c->check(hipGetLastError())) || (st = c->download(host.palette, dev->palette, sizeof(host.palette))))
         return st;
     const uint32_t distinct = host.palette[0];
     if (host.palette[1] == 0 && distinct <= PALETTE_LIMIT) {
         w->voxelBytes = distinct <= 256 ? 1u : 2u;
         w->nPalette = distinct;
-        if ((st = c->alloc(&w->palette, distinct * sizeof(uint2))) || (st = c->alloc(&w->voxels, n * w->voxelBytes)))
+        if ((st = c->alloc(&w->palette, distinct * sizeof(uint2))) || (st = c->alloc(&w->voxels, n * w->voxelBytes))
+            || (st = c->check(hipMemcpyAsync(w->palette, records.p, distinct * sizeof(uint2), hipMemcpyDeviceToDevice, c->stream))))
             return st;
-        auto* r = static_cast<uint32_t*>(rank.p);
-        hipLaunchKernelGGL(paletteCompact, dim3(1), dim3(COMPACT_BLOCK), 0, c->stream, k, r, static_cast<uint2*>(w->palette));
         if (w->voxelBytes == 1)
             hipLaunchKernelGGL(paletteIndex<uint8_t>, dim3(gridFor(n, SCAN_BLOCK, SCAN_GRID)), dim3(SCAN_BLOCK), 0, c->stream, mat, dens, meas, n, k, r,
                 static_cast<uint8_t*>(w->voxels));
