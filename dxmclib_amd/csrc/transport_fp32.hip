@@ -79,14 +79,6 @@ constexpr uint32_t POOL_MAX = 128; // most slots a wave uses
 constexpr uint32_t POOL_MIN = 48;
 constexpr uint32_t FLIGHTS_PER_LOOP = 64; // most flights before the outer loop runs
 
-// LDS of the density intervals and attenuation bounds a staged code world
-// adds: a flight reads them after the block code (and the voxel code); from
-// LDS instead of L1 they took the CT spiral from 201 to 180 ms
-__host__ __device__ inline uint32_t boundsBytes(const Tables<float>& t)
-{
-    return ldsAlign(uint64_t(t.nMaterials) * t.lutNodes * sizeof(float2)) + 256 * sizeof(float2);
-}
-
 // Waves of a block: two blocks fill a CU's 4 W waves, so the staged tables
 // are held twice a CU and the LDS left is the waves' pools.
 __host__ __device__ constexpr uint32_t blockWaves(uint32_t W) { return 2 * W; }

@@ -1,8 +1,8 @@
 // FP64 photon transport: the plain method's histories on a persistent kernel.
 //
 // Same scheme as the FP32 kernel (transport_fp32.hip): one photon per lane in
-// registers, flights advanced together, interactions run when enough lanes
-// are due, new photons sampled by whole waves into an LDS queue. Every value
+// registers, a pool of further ones in LDS, and flights, interactions and
+// sampling each run with most of a wave's lanes. Every value
 // that decides a history (position, direction, energy, weight, attenuation,
 // majorant) is computed in FP64 by the code the plain method uses
 // (device/physics.hpp, compiled without FMA contraction), so histories round
@@ -37,13 +37,18 @@ constexpr double LOG2_10 = 3.321928094887362347870319429489390175864831393;
 // products are each below 1e-6 for ordinary tables.
 constexpr float FILTER_MARGIN = 1e-4f;
 
-// per-wave queue of sampled photons (SoA of 4-byte words): position,
-// direction, energy, weight, log10 E and 1 / majorant as 11 pairs of words
-// (low, high), PCG state (2), the history's offset in the launch and the LUT
-// segment
-constexpr uint32_t QUEUE_DOUBLES = 10;
-constexpr uint32_t QUEUE_WORDS = 2 * QUEUE_DOUBLES + 4;
-__host__ __device__ constexpr uint32_t queueBytes(uint32_t capacity) { return QUEUE_WORDS * capacity * 4; }
+// A slot of a wave's photon pool (the ring of the FP32 kernel): ten doubles
+// (position, direction, energy, weight, log10 E, 1 / majorant) as pairs of
+// words, PCG state, the history's offset in the launch, LUT segment |
+// material << 20 | measurement flag << 28, and the history's steps so far. 25
+// words, an odd stride (see the FP32 kernel).
+constexpr uint32_t SLOT_DOUBLES = 10;
+constexpr uint32_t SLOT_WORDS = 2 * SLOT_DOUBLES + 5;
+constexpr uint32_t SLOT_BYTES = SLOT_WORDS * 4;
+constexpr uint32_t POOL_RESERVE = 16; // slots that sampling leaves for photons that become pending
+constexpr uint32_t POOL_MAX = 128, POOL_MIN = 48;
+constexpr uint32_t FLIGHTS_PER_LOOP = 64; // most flights before the outer loop runs
+constexpr uint32_t WAVES_PER_CU = 8; // 2 a SIMD
 
 // voxel coordinate (uint32_t)((pos - lower) / spacing) of the plain method,
 // clamped to the grid: the product q with the reciprocal differs from the
@@ -81,7 +86,7 @@ struct Args64 {
     Tally tally;
     Counters* ctr;
     unsigned long long* next;
-    uint32_t nExp, regenThreshold, interactThreshold, poolSize, queueCapacity, exactSteps;
+    uint32_t nExp, refillThreshold, interactThreshold, poolSize, slots, exactSteps;
 };
 
 __device__ inline const Args64& loopArgs()
@@ -92,30 +97,42 @@ __device__ inline const Args64& loopArgs()
 }
 
 // K: world kind (WORLD_CODES8 with block codes, or WORLD_ANY: palette or
-// 8-byte records). S: LDS staging level. Three waves per SIMD (168 VGPRs):
-// the FP64 samplers' temporaries spill, and fewer waves with fewer spills won
-// (CT spiral 384x384x200, 4e7 histories: 148 ms for the plain form, one
-// thread a history; here 50.5 ms with 5 waves, 33.7 with 4, 28.4 with 3,
-// 30.1 with 2; CTDI phantom, 2e7 histories: 19.9 ms plain, 8.7 with 3).
+// 8-byte records). S: LDS staging level. Two waves per SIMD (256 VGPRs): the
+// FP64 samplers' temporaries spill with less. CT spiral 384x384x200, 4e7
+// histories: 148 ms for the plain form (one thread a history); without pools
+// 50.5 ms with 5 waves, 33.7 with 4, 28.4 with 3; with pools 31.6 with 4, 22.4
+// with 3, 21.8 with 2 (181 wave instructions a history, vector issue 59 %
+// busy). CTDI phantom, 2e7 histories: 19.9 ms plain, 8.7 without pools, 6.8.
 template <int L, uint32_t S, uint32_t K>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 8))) void transportPersistent64(Args64 args)
+__global__ __launch_bounds__(64 * WAVES_PER_CU) __attribute__((amdgpu_waves_per_eu(2, 8))) void transportPersistent64(Args64 args)
 {
     extern __shared__ __align__(16) unsigned char lds[];
     Tables<double> t = args.t;
     stageTables<double, S, L>(t, lds);
+    // density intervals and attenuation bounds of code worlds
+    constexpr bool BOUNDS_LDS = K == WORLD_CODES8 && S >= STAGE_SMALL;
+    const float2* sumBound = args.sumBound;
+    const float2* bounds = nullptr;
+    uint32_t poolAt = ldsBytes(args.t, S, L);
+    if constexpr (BOUNDS_LDS) {
+        unsigned char* c = lds + poolAt;
+        sumBound = stageArray(args.sumBound, uint64_t(t.nMaterials) * t.lutNodes, c);
+        float2* d = reinterpret_cast<float2*>(c);
+        for (uint32_t i = threadIdx.x; i < 256; i += blockDim.x)
+            d[i] = make_float2(args.w.bounds[i].lo, args.w.bounds[i].hi);
+        bounds = d;
+        poolAt += boundsBytes(args.t);
+        __syncthreads();
+    }
     Particle<double> p;
     Rng rng { 0, 1 };
     double majInv = 0;
-    bool update = true;
-    uint32_t phase = DEAD;
+    bool flying = false, due = false; // neither: the lane holds no photon
     const uint64_t span = args.hEnd - args.hBegin;
     uint64_t poolNext = 0, poolEnd = 0;
     uint32_t poolExp = 0;
     bool claimedAll = span == 0;
-    uint32_t events = 0; // scoring events of the lane's interactions
-    uint32_t steps = 0;
-    uint32_t historySteps = 0;
-    uint64_t idx = 0;
+    uint32_t events = 0, steps = 0, historySteps = 0;
     uint32_t matMeas = 0; // material | measurement flag << 24 of the voxel reached
     // the photon's place in the LUT (x = log10 E), and the FP32 filter's
     // copies: log2 E above the segment's node, 1 / majorant
@@ -123,19 +140,159 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 8))) voi
     float x32 = 0, maj32 = 0;
     const uint32_t lane = __lane_id();
 
-    const uint32_t cap = args.queueCapacity;
-    uint32_t* q = reinterpret_cast<uint32_t*>(lds + ldsBytes(args.t, S, L) + (threadIdx.x / 64) * queueBytes(cap));
-    uint32_t queued = 0;
+    const uint32_t slots = args.slots;
+    uint32_t* pool = reinterpret_cast<uint32_t*>(lds + poolAt + (threadIdx.x / 64) * (slots * SLOT_BYTES));
+    uint32_t first = 0, ready = 0, pending = 0; // the ring's window (wave-uniform)
+    auto slotAt = [&](uint32_t offset) {
+        const uint32_t k = first + offset;
+        return pool + (k >= slots ? k - slots : k) * SLOT_WORDS;
+    };
+    auto put = [](uint32_t* q, uint32_t f, double v) {
+        q[2 * f] = static_cast<uint32_t>(__double2loint(v));
+        q[2 * f + 1] = static_cast<uint32_t>(__double2hiint(v));
+    };
+    auto get = [](const uint32_t* q, uint32_t f) { return __hiloint2double(static_cast<int>(q[2 * f + 1]), static_cast<int>(q[2 * f])); };
+    auto storeWords = [&](uint32_t* q, uint64_t launchFirst) {
+        q[20] = static_cast<uint32_t>(rng.s);
+        q[21] = static_cast<uint32_t>(rng.s >> 32);
+        q[22] = static_cast<uint32_t>(rng.inc >> 1) - static_cast<uint32_t>(launchFirst);
+        q[23] = lp.k | (matMeas & 0xffu) << 20 | (K != WORLD_CODES8 && matMeas >> 24 != 0 ? 1u << 28 : 0u);
+        q[24] = historySteps;
+    };
+    auto store = [&](uint32_t* q, uint64_t launchFirst) {
+        for (uint32_t i = 0; i < 3; ++i) {
+            put(q, i, p.pos[i]);
+            put(q, 3 + i, p.dir[i]);
+        }
+        put(q, 6, p.energy);
+        put(q, 7, p.weight);
+        put(q, 8, lp.x);
+        put(q, 9, majInv);
+        storeWords(q, launchFirst);
+    };
+    auto filter = [&]() { // the FP32 filter's copies
+        x32 = static_cast<float>((lp.x - t.lutGrid[lp.k]) * LOG2_10);
+        maj32 = static_cast<float>(majInv);
+    };
+    auto loadWords = [&](const uint32_t* v, uint64_t launchFirst) {
+        rng.s = static_cast<uint64_t>(v[1]) << 32 | v[0];
+        rng.inc = 2 * (launchFirst + v[2]) + 1;
+        lp.k = v[3] & 0xfffffu;
+        matMeas = (v[3] >> 20 & 0xffu) | (K != WORLD_CODES8 ? v[3] >> 28 << 24 : 0u);
+        historySteps = v[4];
+        filter();
+    };
+    auto load = [&](const uint32_t* q, uint64_t launchFirst) {
+        for (uint32_t i = 0; i < 3; ++i) {
+            p.pos[i] = get(q, i);
+            p.dir[i] = get(q, 3 + i);
+        }
+        p.energy = get(q, 6);
+        p.weight = get(q, 7);
+        lp.x = get(q, 8);
+        majInv = get(q, 9);
+        loadWords(q + 20, launchFirst);
+    };
 
     for (;;) {
-        const uint64_t dead = __ballot(phase == DEAD);
-        const uint32_t nDead = __popcll(dead);
+        const uint64_t dueMask = __ballot(due);
+        uint64_t flyMask = __ballot(flying);
+        const uint32_t nDue = __popcll(dueMask);
+        const uint32_t nFly = __popcll(flyMask);
+        const uint32_t room = slots - ready - pending;
         const bool work = poolNext < poolEnd || !claimedAll;
-        if (work && queued < nDead) {
+        const bool canSample = work && room > POOL_RESERVE;
+        // when interactions run, and how their photons come to the lanes: as
+        // in the FP32 kernel
+        const uint32_t waiting = nDue + pending;
+        if (waiting != 0
+            && (waiting >= args.interactThreshold || nDue > room || (!work && ready == 0 && waiting >= nFly)
+                || (nFly == 0 && ready == 0 && !canSample))) {
             const Args64& a = loopArgs();
+            const uint64_t launchFirst = a.firstHistory + a.hBegin;
+            const uint64_t emptyMask = ~(dueMask | flyMask);
+            const uint32_t back = min(64u - nDue - nFly, pending);
+            const uint32_t front = min(nFly, pending - back);
+            const bool taken = !due && !flying && rankBelow(emptyMask) < back;
+            const bool exchanged = flying && rankBelow(flyMask) < front;
+            if (taken || exchanged) {
+                uint32_t* q = slotAt(taken ? ready + pending - 1 - rankBelow(emptyMask) : ready + rankBelow(flyMask));
+                if (exchanged) { // field by field: few values live twice
+                    auto swap = [&](uint32_t f, double& x) {
+                        const double v = get(q, f);
+                        put(q, f, x);
+                        x = v;
+                    };
+                    for (uint32_t i = 0; i < 3; ++i) {
+                        swap(i, p.pos[i]);
+                        swap(3 + i, p.dir[i]);
+                    }
+                    swap(6, p.energy);
+                    swap(7, p.weight);
+                    swap(8, lp.x);
+                    swap(9, majInv);
+                    const uint32_t v[5] = { q[20], q[21], q[22], q[23], q[24] };
+                    storeWords(q, launchFirst);
+                    loadWords(v, launchFirst);
+                } else {
+                    steps += historySteps;
+                    load(q, launchFirst);
+                }
+                due = true;
+                flying = false;
+            }
+            pending -= back + front;
+            ready += front;
+            Deposits<double> deposits;
+            uint64_t idx = 0;
+            const bool wide = K != WORLD_CODES8 && a.w.index24 == 0;
+            if (due) {
+                const uint32_t mat = matMeas & 0xffu;
+                idx = voxelIndexFast(a.w, voxelCoords64(a.w, p.pos, a.inv), !wide); // the voxel the flight ended in
+                bool update = false;
+                double att[3];
+                attenuationAt(t, mat, lp, att);
+                bool alive;
+                if (K != WORLD_CODES8 && matMeas > 0xffffffu) { // forced event (measurement voxel)
+                    const double prob = ((att[0] + att[1]) + att[2]) * a.w.density[idx] * majInv;
+                    alive = computeInteractionsForced<double, L>(t, prob, att, p, mat, deposits, rng, update);
+                } else {
+                    alive = computeInteractions<double, L>(t, att, p, mat, deposits, rng, update);
+                }
+                if (alive && p.energy * p.weight < 5.0) { // Russian roulette
+                    if (rng.uniform<double>() < 0.8)
+                        alive = false;
+                    else
+                        p.weight *= 1.0 / (1.0 - 0.8);
+                }
+                if (alive && update) { // new energy: its LUT point and majorant
+                    lp = lutPoint(t, p.energy);
+                    majInv = majorantInverseAt(t, lp);
+                    filter();
+                }
+                flying = alive && historySteps < MAX_STEPS;
+                due = false;
+            }
+            events += deposits.n;
+            scoreWave(a.tally, deposits.n > 0, idx, deposits.first, wide);
+            if (K != WORLD_CODES8 && __ballot(deposits.n > 1) != 0) // forced events with a Compton event
+                scoreWave(a.tally, deposits.n > 1, idx, deposits.second, wide);
+        } else if (nDue != 0) {
+            // photons with an interaction due wait in the pool
+            if (due) {
+                store(slotAt(ready + pending + rankBelow(dueMask)), args.firstHistory + args.hBegin);
+                historySteps = 0;
+                due = false;
+            }
+            pending += nDue;
+        }
+        flyMask = __ballot(flying);
+        const uint32_t nEmpty = 64u - __popcll(flyMask);
+        if (work && ready < nEmpty && slots - ready - pending > POOL_RESERVE) {
             // sample with the whole wave: the next histories of the wave's
-            // pool, those that enter the world join the queue
-            const uint32_t want = cap - queued;
+            // range, those that enter the world join the ready ones
+            const Args64& a = loopArgs();
+            const uint32_t want = min(64u, slots - ready - pending - POOL_RESERVE);
             uint32_t assigned = 0;
             bool sampled = false;
             Particle<double> np;
@@ -169,109 +326,62 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 8))) voi
                 assigned += take;
             }
             const uint64_t entered = __ballot(sampled);
+            const uint32_t n = __popcll(entered);
+            first = first >= n ? first - n : first + slots - n; // ahead of the ready ones
+            ready += n;
             if (sampled) {
-                const uint32_t slot = queued + rankBelow(entered);
+                uint32_t* q = slotAt(rankBelow(entered));
                 const LutPoint<double> np0 = lutPoint(t, np.energy);
-                const double v[QUEUE_DOUBLES] = { np.pos[0], np.pos[1], np.pos[2], np.dir[0], np.dir[1], np.dir[2], np.energy, np.weight, np0.x,
-                    majorantInverseAt(t, np0) };
-                for (uint32_t f = 0; f < QUEUE_DOUBLES; ++f) {
-                    q[2 * f * cap + slot] = static_cast<uint32_t>(__double2loint(v[f]));
-                    q[(2 * f + 1) * cap + slot] = static_cast<uint32_t>(__double2hiint(v[f]));
+                for (uint32_t i = 0; i < 3; ++i) {
+                    put(q, i, np.pos[i]);
+                    put(q, 3 + i, np.dir[i]);
                 }
-                q[(2 * QUEUE_DOUBLES) * cap + slot] = static_cast<uint32_t>(nr.s);
-                q[(2 * QUEUE_DOUBLES + 1) * cap + slot] = static_cast<uint32_t>(nr.s >> 32);
-                q[(2 * QUEUE_DOUBLES + 2) * cap + slot] = nOffset;
-                q[(2 * QUEUE_DOUBLES + 3) * cap + slot] = np0.k;
+                put(q, 6, np.energy);
+                put(q, 7, np.weight);
+                put(q, 8, np0.x);
+                put(q, 9, majorantInverseAt(t, np0));
+                q[20] = static_cast<uint32_t>(nr.s);
+                q[21] = static_cast<uint32_t>(nr.s >> 32);
+                q[22] = nOffset;
+                q[23] = np0.k;
+                q[24] = 0;
             }
-            queued += __popcll(entered);
         }
-        // dead lanes take photons from the queue (last in, first out)
-        if (nDead >= args.regenThreshold || (nDead > 0 && !work)) {
-            const Args64& a = loopArgs();
-            const uint32_t take = nDead < queued ? nDead : queued;
-            if (phase == DEAD) {
-                const uint32_t r = rankBelow(dead);
-                if (r < take) {
-                    const uint32_t slot = queued - 1 - r;
-                    double v[QUEUE_DOUBLES];
-                    for (uint32_t f = 0; f < QUEUE_DOUBLES; ++f)
-                        v[f] = __hiloint2double(static_cast<int>(q[(2 * f + 1) * cap + slot]), static_cast<int>(q[2 * f * cap + slot]));
-                    for (int i = 0; i < 3; ++i) {
-                        p.pos[i] = v[i];
-                        p.dir[i] = v[3 + i];
-                    }
-                    p.energy = v[6];
-                    p.weight = v[7];
-                    rng.s = static_cast<uint64_t>(q[(2 * QUEUE_DOUBLES + 1) * cap + slot]) << 32 | q[(2 * QUEUE_DOUBLES) * cap + slot];
-                    rng.inc = 2 * (a.firstHistory + a.hBegin + q[(2 * QUEUE_DOUBLES + 2) * cap + slot]) + 1;
-                    lp.k = q[(2 * QUEUE_DOUBLES + 3) * cap + slot];
-                    lp.x = v[8];
-                    majInv = v[9];
-                    x32 = static_cast<float>((lp.x - t.lutGrid[lp.k]) * LOG2_10);
-                    maj32 = static_cast<float>(majInv);
-                    update = false;
-                    steps += historySteps;
-                    historySteps = 0;
-                    phase = FLYING;
-                }
+        // lanes without a photon take ready ones from the front of the window
+        const uint32_t take = min(nEmpty, ready);
+        if (take != 0) {
+            const uint32_t r = rankBelow(~flyMask);
+            if (!flying && r < take) {
+                steps += historySteps;
+                load(slotAt(r), args.firstHistory + args.hBegin);
+                flying = true;
             }
-            queued -= take;
+            first += take;
+            first = first >= slots ? first - slots : first;
+            ready -= take;
         }
-        const uint64_t pend = __ballot(phase == PENDING);
-        const uint64_t fly = __ballot(phase == FLYING);
-        if ((pend | fly) == 0) {
-            if (poolNext >= poolEnd && claimedAll && queued == 0)
+        const bool more = poolNext < poolEnd || !claimedAll || ready != 0;
+        if (__ballot(flying) == 0) {
+            if (!more && pending == 0)
                 break;
             continue;
         }
-        const uint32_t nPend = __popcll(pend);
-        if (nPend != 0 && (nPend >= args.interactThreshold || fly == 0)) {
-            Deposits<double> deposits;
-            if (phase == PENDING) {
+        // Woodcock flights of the flying lanes until the outer loop is needed
+        const uint32_t limit = more ? args.refillThreshold : 64u;
+        const uint64_t faintMask = __ballot(p.energy * p.weight < 5.0);
+        const bool nearCap = __ballot(flying && historySteps >= MAX_STEPS - FLIGHTS_PER_LOOP) != 0;
+        for (uint32_t n = 0; n < FLIGHTS_PER_LOOP; ++n) {
+            if (flying) {
                 const Args64& a = loopArgs();
-                const uint32_t mat = matMeas & 0xffu;
-                double att[3];
-                attenuationAt(t, mat, lp, att);
-                bool alive;
-                if (K != WORLD_CODES8 && matMeas > 0xffffffu) { // forced event (measurement voxel)
-                    const double prob = ((att[0] + att[1]) + att[2]) * a.w.density[idx] * majInv;
-                    alive = computeInteractionsForced<double, L>(t, prob, att, p, mat, deposits, rng, update);
-                } else {
-                    alive = computeInteractions<double, L>(t, att, p, mat, deposits, rng, update);
-                }
-                if (alive && p.energy * p.weight < 5.0) { // Russian roulette
-                    if (rng.uniform<double>() < 0.8)
-                        alive = false;
-                    else
-                        p.weight *= 1.0 / (1.0 - 0.8);
-                }
-                if (alive && update) { // new energy: its LUT point and majorant
-                    lp = lutPoint(t, p.energy);
-                    majInv = majorantInverseAt(t, lp);
-                    x32 = static_cast<float>((lp.x - t.lutGrid[lp.k]) * LOG2_10);
-                    maj32 = static_cast<float>(majInv);
-                    update = false;
-                }
-                phase = alive && historySteps < MAX_STEPS ? FLYING : DEAD;
-            }
-            events += deposits.n;
-            const bool wide = K != WORLD_CODES8 && args.w.index24 == 0;
-            scoreWave(args.tally, deposits.n > 0, idx, deposits.first, wide);
-            if (K != WORLD_CODES8 && __ballot(deposits.n > 1) != 0) // forced events with a Compton event
-                scoreWave(args.tally, deposits.n > 1, idx, deposits.second, wide);
-        } else {
-            // Woodcock flights of the FLYING lanes until the outer loop is needed
-            for (;;) {
-                if (phase == FLYING) {
-                    const Args64& a = loopArgs();
-                    const World<double>& w = a.w;
-                    const double u1 = rng.uniform<double>();
-                    const double step = -log(u1) * majInv * 10.0; // cm -> mm
-                    for (int i = 0; i < 3; ++i)
-                        p.pos[i] += p.dir[i] * step;
-                    const bool in = insideFast(w, p.pos);
-                    const uint3 vc = voxelCoords64(w, p.pos, a.inv); // clamped: a valid voxel also outside
-                    idx = voxelIndexFast(w, vc, K == WORLD_CODES8 || w.index24 != 0);
+                const World<double>& w = a.w;
+                const double u1 = rng.uniform<double>();
+                const double step = -log(u1) * majInv * 10.0; // cm -> mm
+                for (int i = 0; i < 3; ++i)
+                    p.pos[i] += p.dir[i] * step;
+                flying = insideFast(w, p.pos);
+                if (flying) {
+                    const uint3 vc = voxelCoords64(w, p.pos, a.inv);
+                    const uint64_t idx = voxelIndexFast(w, vc, K == WORLD_CODES8 || w.index24 != 0);
                     Rng r2 = rng;
                     const uint32_t n2 = r2.next();
                     const double u2 = static_cast<double>(n2) * 2.32830643653869628906e-010;
@@ -289,24 +399,27 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 8))) voi
                         real = f2 < prob;
                     };
                     if constexpr (K == WORLD_CODES8) {
+                        auto bracket = [&](float dLo, float dHi) {
+                            const uint32_t row = __umul24(matMeas, t.lutNodes) + lp.k;
+                            const float2 sb = BOUNDS_LDS ? sumBound[row] : loadAt(a.sumBound, row);
+                            const float lo = sb.x * dLo * maj32, hi = sb.y * dHi * maj32;
+                            settled = (f2 < lo) | (f2 > hi);
+                            real = f2 < lo;
+                        };
                         const uint32_t bc = loadAt(w.blocks, blockIndexFast(w, vc));
                         matMeas = __umul24(bc >> 8, w.codeMul) >> CODE_MUL_SHIFT;
-                        {
-                            const float bLo = w.bounds[bc & 0xffu].lo;
-                            const float bHi = w.bounds[bc >> 8].hi;
-                            const float2 sb = loadAt(a.sumBound, __umul24(matMeas, t.lutNodes) + lp.k);
-                            const float lo = sb.x * bLo * maj32, hi = sb.y * bHi * maj32;
-                            settled = (bc != BLOCK_MIXED) & ((f2 < lo) | (f2 > hi));
-                            real = f2 < lo;
-                        }
+                        if constexpr (BOUNDS_LDS)
+                            bracket(bounds[bc & 0xffu].x, bounds[bc >> 8].y);
+                        else
+                            bracket(w.bounds[bc & 0xffu].lo, w.bounds[bc >> 8].hi);
+                        settled &= bc != BLOCK_MIXED;
                         if (!settled) {
                             const uint32_t code = loadAt(static_cast<const uint8_t*>(w.codes), static_cast<uint32_t>(idx));
                             matMeas = __umul24(code, w.codeMul) >> CODE_MUL_SHIFT;
-                            const uint2 b = *reinterpret_cast<const uint2*>(w.bounds + code);
-                            const float2 sb = loadAt(a.sumBound, __umul24(matMeas, t.lutNodes) + lp.k);
-                            const float lo = sb.x * __uint_as_float(b.x) * maj32, hi = sb.y * __uint_as_float(b.y) * maj32;
-                            settled = (f2 < lo) | (f2 > hi);
-                            real = f2 < lo;
+                            if constexpr (BOUNDS_LDS)
+                                bracket(bounds[code].x, bounds[code].y);
+                            else
+                                bracket(w.bounds[code].lo, w.bounds[code].hi);
                             if (!settled)
                                 evaluate(static_cast<float>(w.density[idx]));
                         }
@@ -320,25 +433,26 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 8))) voi
                         attenuationAt(t, matMeas, lp, att);
                         real = u2 < ((att[0] + att[1]) + att[2]) * w.density[idx] * majInv;
                     }
-                    const bool measured = matMeas > 0xffffffu; // (code worlds carry no flags)
-                    rng.s = (in & !measured) ? r2.s : rng.s;
-                    uint32_t now = in ? ((measured | real) ? PENDING : FLYING) : DEAD;
-                    if (now == FLYING && p.energy * p.weight < 5.0) { // Russian roulette
-                        if (rng.uniform<double>() < 0.8)
-                            now = DEAD;
-                        else
-                            p.weight *= 1.0 / (1.0 - 0.8);
-                    }
-                    historySteps += in ? 1u : 0u;
-                    phase = (now == FLYING && historySteps >= MAX_STEPS) ? DEAD : now;
+                    // a forced event draws no decision (code worlds carry no flags)
+                    const bool measured = K != WORLD_CODES8 && matMeas > 0xffffffu;
+                    rng.s = measured ? rng.s : r2.s;
+                    due = measured | real;
+                    flying = !due;
+                    if (flying & __builtin_amdgcn_inverse_ballot_w64(faintMask)) // Russian roulette
+                        if (p.energy * p.weight < 5.0) {
+                            if (rng.uniform<double>() < 0.8)
+                                flying = false;
+                            else
+                                p.weight *= 1.0 / (1.0 - 0.8);
+                        }
+                    ++historySteps;
+                    if (nearCap && historySteps >= MAX_STEPS) // an interaction due is still run
+                        flying = false;
                 }
-                const uint64_t flyNow = __ballot(phase == FLYING);
-                const uint32_t nPendNow = __popcll(__ballot(phase == PENDING));
-                const uint32_t nDeadNow = __popcll(__ballot(phase == DEAD));
-                if (flyNow == 0 || nPendNow >= args.interactThreshold || nDeadNow >= args.regenThreshold || (work && nDeadNow > queued)
-                    || (!work && nDeadNow > 0 && queued > 0))
-                    break;
             }
+            const uint32_t flyNow = __popcll(__ballot(flying));
+            if (flyNow == 0 || 64u - flyNow >= limit || (!more && __popcll(__ballot(due)) + pending >= flyNow))
+                break;
         }
     }
     if (args.ctr)
@@ -374,46 +488,33 @@ void launchFp64(dxmc_ctx* c, const dxmc_run_cfg& cfg, const World<double>& w, co
     hipLaunchKernelGGL(clearCounter, dim3(1), dim3(1), 0, c->stream, historyCounter);
     const int L = cfg.low_energy_correction;
     const uint32_t kind = w.index24 && w.codeBytes == 1 && w.blocks && t32.lutSumBound ? WORLD_CODES8 : WORLD_ANY;
-    // queue capacity and staging with the most resident blocks, the staged
-    // tables and the larger queue first among equals (CT spiral with 7
-    // materials: 25 KB of tables and 64 photons fit 3 blocks, which is what
-    // the registers allow)
-    const uint32_t block = cfg.block_size ? cfg.block_size : 256;
-    constexpr uint32_t LDS_PER_BLOCK = 64 * 1024;
-    uint32_t cap = 64, lds = 0, perCU = 0;
-    bool staged = true;
-    for (const bool st : { true, false })
-        for (const uint32_t q : { 64u, 48u, 32u }) {
-            const uint64_t bytes = uint64_t(ldsBytes(t, st ? STAGE_SMALL : STAGE_NONE, L)) + block / 64 * queueBytes(q);
-            if (bytes > LDS_PER_BLOCK)
-                continue;
-            int blocks = 0;
-            if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, reinterpret_cast<const void*>(kernelFor(L, st, kind)), static_cast<int>(block), bytes)
-                != hipSuccess) {
-                hipGetLastError();
-                blocks = 1;
-            }
-            if (static_cast<uint32_t>(std::max(blocks, 1)) > perCU) {
-                cap = q;
-                lds = static_cast<uint32_t>(bytes);
-                perCU = static_cast<uint32_t>(std::max(blocks, 1));
-                staged = st;
-            }
-        }
-    if (cfg.blocks_per_cu)
-        perCU = cfg.blocks_per_cu;
-    // thresholds on CT spiral, ms: interaction 12 50.1, 20 42.1, 28 38.8, 40
-    // 38.7 (at 4 waves); 28 28.4, 36 28.6, 44 30.7 (at 3); regeneration 1
-    // 45.5, 4 38.8, 8 37.7, 16 39.0 (at 4)
-    const uint32_t regen = cfg.regeneration_threshold ? std::min<uint32_t>(cfg.regeneration_threshold, 64u) : 8u;
-    const uint32_t interact = cfg.interaction_threshold ? std::min<uint32_t>(cfg.interaction_threshold, 64u) : 28u;
-    uint64_t grid = static_cast<uint64_t>(c->numCU) * perCU;
-    grid = std::max<uint64_t>(1, std::min<uint64_t>(grid, (he - hb + block - 1) / block));
+    // one block of 8 waves a CU, so the tables are held once and the rest of
+    // the LDS is the waves' pools; a block size asked for divides them.
+    // Launches with too few histories get blocks of fewer waves.
+    const uint64_t wavesNeeded = (he - hb + 63) / 64;
+    const uint32_t fullBlock = cfg.block_size ? cfg.block_size / 64 : WAVES_PER_CU;
+    const uint32_t perCU = cfg.blocks_per_cu ? cfg.blocks_per_cu : WAVES_PER_CU / fullBlock;
+    const uint32_t wavesPerBlock = static_cast<uint32_t>(std::clamp<uint64_t>((wavesNeeded + c->numCU - 1) / c->numCU, 1, fullBlock));
+    auto tablesBytes = [&](uint32_t stage) {
+        return ldsBytes(t, stage, L) + (kind == WORLD_CODES8 && stage >= STAGE_SMALL ? boundsBytes(t) : 0u);
+    };
+    auto poolSlots = [&](uint32_t stage, uint32_t waves) {
+        const uint32_t block = 160 * 1024 / (WAVES_PER_CU / fullBlock) - 1280, tables = tablesBytes(stage);
+        return tables >= block ? 0u : std::min(POOL_MAX, (block - tables) / waves / SLOT_BYTES);
+    };
+    const bool staged = poolSlots(STAGE_SMALL, fullBlock) >= POOL_MIN;
+    const uint32_t stage = staged ? STAGE_SMALL : STAGE_NONE;
+    const uint32_t slots = poolSlots(stage, wavesPerBlock);
+    const uint32_t lds = tablesBytes(stage) + wavesPerBlock * slots * SLOT_BYTES;
+    // thresholds on CT spiral, ms: interaction 48 22.3, 56 21.8, 64 21.9;
+    // refill 10 22.2, 16 21.9, 20 21.9, 28 22.5
+    const uint32_t refill = cfg.regeneration_threshold ? std::min<uint32_t>(cfg.regeneration_threshold, 64u) : 16u;
+    const uint32_t interact = std::min<uint32_t>(cfg.interaction_threshold ? std::min<uint32_t>(cfg.interaction_threshold, 64u) : 56u, slots / 2);
+    const uint64_t grid = std::clamp<uint64_t>((wavesNeeded + wavesPerBlock - 1) / wavesPerBlock, 1, static_cast<uint64_t>(c->numCU) * perCU);
     // histories a wave claims per atomic on the global counter
     const uint32_t pool = cfg.queue_depth ? std::clamp<uint32_t>(cfg.queue_depth, 64u, 1u << 16) : 512u;
-
     const Args64 args { w, t, { 1.0 / w.spacing[0], 1.0 / w.spacing[1], 1.0 / w.spacing[2] }, t32.lutCoef, t32.lutSumBound, exps, expStart, hb, he,
-        cfg.seed, cfg.first_history, tally, ctr, historyCounter, nExp, regen, interact, pool, cap, (cfg.flags & DXMC_RUN_EXACT_STEPS) != 0 };
-    hipLaunchKernelGGL(kernelFor(L, staged, kind), dim3(static_cast<uint32_t>(grid)), dim3(block), lds, c->stream, args);
+        cfg.seed, cfg.first_history, tally, ctr, historyCounter, nExp, refill, interact, pool, slots, (cfg.flags & DXMC_RUN_EXACT_STEPS) != 0 };
+    hipLaunchKernelGGL(kernelFor(L, staged, kind), dim3(static_cast<uint32_t>(grid)), dim3(64 * wavesPerBlock), lds, c->stream, args);
 }
 }
