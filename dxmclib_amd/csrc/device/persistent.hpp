@@ -227,4 +227,53 @@ __device__ inline void scoreWave(const Tally& tally, bool has, uint64_t idx, T e
             unsafeAtomicAdd(reinterpret_cast<double*>(tally.voxels + (static_cast<uint64_t>(vHi) << 32 | vLo)) + field, add);
     }
 }
+
+// Scores of pencil beams. Their photons interact on one line of voxels, whose
+// cache lines all XCDs then change in turn (95 ns a change of owner against 4
+// ns within an XCD), so a block keeps the sums of up to 256 voxels in LDS,
+// first come, first served, and adds them to the tally once, at its end. Runs
+// of other beams score all over the world and would only fill it.
+constexpr uint32_t SCORE_CACHE_ENTRIES = 256;
+constexpr uint32_t SCORE_CACHE_BYTES = SCORE_CACHE_ENTRIES * (3 * sizeof(double) + sizeof(uint32_t));
+
+struct ScoreCache {
+    static constexpr uint32_t FREE = 0xffffffffu; // no voxel index where indices fit 24-bit products
+    double* sums; // dose, variance, events of each entry
+    uint32_t* voxel;
+
+    // the cache in LDS, empty (all threads of the block call it)
+    __device__ explicit ScoreCache(unsigned char* lds)
+        : sums(reinterpret_cast<double*>(lds))
+        , voxel(reinterpret_cast<uint32_t*>(lds + SCORE_CACHE_ENTRIES * 3 * sizeof(double)))
+    {
+    }
+    __device__ inline void clear() const
+    {
+        for (uint32_t i = threadIdx.x; i < SCORE_CACHE_ENTRIES; i += blockDim.x)
+            voxel[i] = FREE;
+        for (uint32_t i = threadIdx.x; i < 3 * SCORE_CACHE_ENTRIES; i += blockDim.x)
+            sums[i] = 0.0;
+        __syncthreads();
+    }
+    // takes the score of a lane that has one; false when its entry is another voxel's
+    __device__ inline bool add(uint32_t idx, double e) const
+    {
+        const uint32_t k = (idx * 2654435761u) >> 24;
+        const uint32_t was = atomicCAS(&voxel[k], FREE, idx);
+        if (was != FREE && was != idx)
+            return false;
+        const double v[3] = { e, e * e, 1.0 };
+        for (int f = 0; f < 3; ++f)
+            __hip_atomic_fetch_add(&sums[3 * k + f], v[f], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        return true;
+    }
+    // adds the sums to the tally (all threads of the block call it)
+    __device__ inline void flush(const Tally& tally) const
+    {
+        __syncthreads();
+        for (uint32_t i = threadIdx.x; i < 4 * SCORE_CACHE_ENTRIES; i += blockDim.x)
+            if ((i & 3u) < 3 && voxel[i / 4] != FREE)
+                unsafeAtomicAdd(reinterpret_cast<double*>(tally.voxels + voxel[i / 4]) + (i & 3u), sums[3 * (i / 4) + (i & 3u)]);
+    }
+};
 }

@@ -827,9 +827,9 @@ int runLaunches(dxmc_ctx* c, const dxmc_world* w, const dxmc_tables* t, uint64_t
         const uint64_t he = std::min(in.total, hb + chunk);
         DXMC_CHECK(c, hipEventRecord(c->ev0, c->stream));
         if (cfg.precision == DXMC_PRECISION_FP64)
-            launchFp64(c, cfg, w64, t->f64, t->f32, in.exp64, in.startDev, static_cast<uint32_t>(nExp), hb, he, tl, in.ctr, in.historyCounter);
+            launchFp64(c, cfg, w64, t->f64, t->f32, in.exp64, in.startDev, static_cast<uint32_t>(nExp), hb, he, tl, in.ctr, in.historyCounter, in.pencil);
         else
-            launchFp32(c, cfg, w32, t->f32, in.exp32, in.startDev, static_cast<uint32_t>(nExp), hb, he, tl, in.ctr, in.historyCounter);
+            launchFp32(c, cfg, w32, t->f32, in.exp32, in.startDev, static_cast<uint32_t>(nExp), hb, he, tl, in.ctr, in.historyCounter, in.pencil);
         DXMC_CHECK(c, hipGetLastError());
         DXMC_CHECK(c, hipEventRecord(c->ev1, c->stream));
         DXMC_CHECK(c, hipEventSynchronize(c->ev1));
@@ -865,7 +865,7 @@ int runTransport(dxmc_ctx* c, const dxmc_world* w, const dxmc_tables* t, const d
     auto* counterBlock = rb.at<Counters>(rb.countersAt);
     const RunInputs in { fp64 ? rb.at<const Exposure<double>>(0) : nullptr, fp64 ? nullptr : rb.at<const Exposure<float>>(0),
         rb.at<const uint64_t>(rb.startAt), rb.start.data(), rb.totalHistories, counters ? counterBlock : nullptr,
-        static_cast<unsigned long long*>(c->historyCounter) };
+        static_cast<unsigned long long*>(c->historyCounter), pencilBeams(x, nExp) };
     double kernelMs = 0;
     uint64_t launches = 0;
     if ((st = runLaunches(c, w, t, nExp, cfg, tally, in, monitor, kernelMs, launches)))

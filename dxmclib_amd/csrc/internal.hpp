@@ -488,7 +488,16 @@ struct RunInputs {
     uint64_t total;
     dxmc_dev::Counters* ctr;
     unsigned long long* historyCounter;
+    bool pencil; // every exposure is a pencil beam
 };
+// whether every exposure is a pencil beam (one direction)
+inline bool pencilBeams(const dxmc_exposure* x, uint64_t nExp)
+{
+    for (uint64_t i = 0; i < nExp; ++i)
+        if (x[i].collimation_angles[0] != x[i].collimation_angles[1] || x[i].collimation_angles[2] != x[i].collimation_angles[3])
+            return false;
+    return true;
+}
 // the launch loop of a run on prepared inputs (cancel, progress and preview
 // through the monitor, which may be null)
 int runLaunches(dxmc_ctx* c, const dxmc_world* w, const dxmc_tables* t, uint64_t nExp, const dxmc_run_cfg& cfg, dxmc_tally* tally,
@@ -505,12 +514,12 @@ int noallocScratch(int device, void** out);
 // FP32 transport launch (transport_fp32.hip)
 void launchFp32(dxmc_ctx* c, const dxmc_run_cfg& cfg, const dxmc_dev::World<float>& w, const dxmc_dev::Tables<float>& t,
     const dxmc_dev::Exposure<float>* exps, const uint64_t* expStart, uint32_t nExp, uint64_t hb, uint64_t he, const dxmc_dev::Tally& tally,
-    dxmc_dev::Counters* ctr, unsigned long long* historyCounter);
+    dxmc_dev::Counters* ctr, unsigned long long* historyCounter, bool pencilBeam);
 // FP64 transport launch (transport_fp64.hip); t32: the FP32 copy of the tables,
 // whose attenuation bounds and coefficients filter the FP64 decisions
 void launchFp64(dxmc_ctx* c, const dxmc_run_cfg& cfg, const dxmc_dev::World<double>& w, const dxmc_dev::Tables<double>& t,
     const dxmc_dev::Tables<float>& t32, const dxmc_dev::Exposure<double>* exps, const uint64_t* expStart, uint32_t nExp, uint64_t hb, uint64_t he,
-    const dxmc_dev::Tally& tally, dxmc_dev::Counters* ctr, unsigned long long* historyCounter);
+    const dxmc_dev::Tally& tally, dxmc_dev::Counters* ctr, unsigned long long* historyCounter, bool pencilBeam);
 // Histories a wave of a persistent kernel claims per atomic on the launch's
 // counter: 512, less in launches where that leaves waves without work while
 // others run long (two claims a wave; at least a wave's 64 lanes, from 2^18

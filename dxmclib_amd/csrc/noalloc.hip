@@ -152,7 +152,7 @@ extern "C" int dxmc_hip_run_noalloc(dxmc_ctx* c, const dxmc_world* w, const dxmc
     hipLaunchKernelGGL(prepareRun, dim3(static_cast<uint32_t>(std::max<uint64_t>(1, (nExp + 255) / 256))), dim3(256), 0, c->stream, raw, nExp, e64,
         e32, start, historyCounter, ctr);
     DXMC_CHECK(c, hipGetLastError());
-    const RunInputs in { e64, e32, start, nullptr, total, ctr, historyCounter };
+    const RunInputs in { e64, e32, start, nullptr, total, ctr, historyCounter, pencilBeams(exposures, nExp) };
     double kernelMs = 0;
     uint64_t launches = 0;
     if ((st = runLaunches(c, w, t, nExp, run, tally, in, nullptr, kernelMs, launches)))

@@ -104,7 +104,7 @@ __device__ inline bool roulette(Particle<float>& p, Rng& rng)
 template <int L, int W, uint32_t S, uint32_t K>
 __global__ __launch_bounds__(64 * blockWaves(W)) __attribute__((amdgpu_waves_per_eu(W, 8))) void transportPersistent(World<float> w, Tables<float> tg, const Exposure<float>* exps, const uint64_t* expStart,
     uint32_t nExp, uint64_t hBegin, uint64_t hEnd, uint64_t seed, uint64_t firstHistory, Tally tally, Counters* ctr, unsigned long long* next,
-    uint32_t refillThreshold, uint32_t interactThreshold, uint32_t poolSize, uint32_t slots)
+    uint32_t refillThreshold, uint32_t interactThreshold, uint32_t poolSize, uint32_t slots, bool pencil)
 {
     extern __shared__ __align__(16) unsigned char lds[];
     Tables<float> t = tg;
@@ -147,7 +147,13 @@ __global__ __launch_bounds__(64 * blockWaves(W)) __attribute__((amdgpu_waves_per
     const uint64_t launchFirst = firstHistory + hBegin;
     const uint32_t lane = __lane_id();
 
-    uint32_t* pool = reinterpret_cast<uint32_t*>(lds + ldsBytes(tg, S, L) + (BOUNDS_LDS ? boundsBytes(tg) : 0u) + (threadIdx.x / 64) * (slots * SLOT_BYTES));
+    uint32_t poolAt = ldsBytes(tg, S, L) + (BOUNDS_LDS ? boundsBytes(tg) : 0u);
+    const ScoreCache cache(lds + poolAt);
+    if (pencil) {
+        poolAt += SCORE_CACHE_BYTES;
+        cache.clear();
+    }
+    uint32_t* pool = reinterpret_cast<uint32_t*>(lds + poolAt + (threadIdx.x / 64) * (slots * SLOT_BYTES));
     uint32_t first = 0, ready = 0, pending = 0; // the ring's window (wave-uniform)
     // slot 'offset' from the start of the window
     auto slotAt = [&](uint32_t offset) {
@@ -258,7 +264,10 @@ __global__ __launch_bounds__(64 * blockWaves(W)) __attribute__((amdgpu_waves_per
                 due = false;
             }
             events += deposits.n;
-            scoreWave(tally, deposits.n > 0, idx, deposits.first, !index24);
+            bool scores = deposits.n > 0;
+            if (pencil && scores)
+                scores = !cache.add(static_cast<uint32_t>(idx), static_cast<double>(deposits.first));
+            scoreWave(tally, scores, idx, deposits.first, !index24);
             if (kindForces(K) && __ballot(deposits.n > 1) != 0) // forced events with a Compton event
                 scoreWave(tally, deposits.n > 1, idx, deposits.second, !index24);
         } else if (nDue != 0) {
@@ -468,6 +477,8 @@ __global__ __launch_bounds__(64 * blockWaves(W)) __attribute__((amdgpu_waves_per
                 break;
         }
     }
+    if (pencil)
+        cache.flush(tally);
     if (ctr)
         dxmc_backend::accumulateCounters(ctr, steps + historySteps, events);
 }
@@ -481,7 +492,7 @@ namespace {
 __global__ void clearCounter(unsigned long long* counter) { *counter = 0; }
 
 using KernelFn = void (*)(World<float>, Tables<float>, const Exposure<float>*, const uint64_t*, uint32_t, uint64_t, uint64_t, uint64_t, uint64_t,
-    Tally, Counters*, unsigned long long*, uint32_t, uint32_t, uint32_t, uint32_t);
+    Tally, Counters*, unsigned long long*, uint32_t, uint32_t, uint32_t, uint32_t, bool);
 
 // waves: resolved by wavesFp32
 template <int L, uint32_t S, uint32_t K>
@@ -535,9 +546,9 @@ uint32_t wavesFp32(uint32_t requested, int L)
 
 // slots of a wave's pool in blocks of 'blockOf' waves beside the staged
 // tables (half a CU's 160 KiB less an allocation granule)
-uint32_t poolSlots(const Tables<float>& t, uint32_t stage, int L, uint32_t blockOf, uint32_t kind)
+uint32_t poolSlots(const Tables<float>& t, uint32_t stage, int L, uint32_t blockOf, uint32_t kind, bool pencil)
 {
-    const uint32_t tables = ldsBytes(t, stage, L) + (kind == WORLD_CODES8 && stage >= STAGE_SMALL ? boundsBytes(t) : 0u), block = 80 * 1024 - 1280;
+    const uint32_t tables = ldsBytes(t, stage, L) + (pencil ? SCORE_CACHE_BYTES : 0u) + (kind == WORLD_CODES8 && stage >= STAGE_SMALL ? boundsBytes(t) : 0u), block = 80 * 1024 - 1280;
     return tables >= block ? 0u : std::min(POOL_MAX, (block - tables) / blockOf / SLOT_BYTES);
 }
 
@@ -545,17 +556,18 @@ uint32_t poolSlots(const Tables<float>& t, uint32_t stage, int L, uint32_t block
 // tables, lowered while the tables leave a wave's pool too few slots. The
 // attenuation coefficients are staged on request only: they are read once an
 // interaction, and the pool slots they would take are worth more.
-uint32_t stageLevelFp32(const dxmc_run_cfg& cfg, const Tables<float>& t, uint32_t W, uint32_t kind)
+uint32_t stageLevelFp32(const dxmc_run_cfg& cfg, const Tables<float>& t, uint32_t W, uint32_t kind, bool pencil)
 {
     uint32_t level = cfg.lds_tables >= STAGE_NONE && cfg.lds_tables <= STAGE_ALL ? cfg.lds_tables : STAGE_SMALL;
-    while (level > STAGE_NONE && poolSlots(t, level, cfg.low_energy_correction, blockWaves(W), kind) < POOL_MIN)
+    while (level > STAGE_NONE && poolSlots(t, level, cfg.low_energy_correction, blockWaves(W), kind, pencil) < POOL_MIN)
         --level;
     return level;
 }
 
 void launchFp32(dxmc_ctx* c, const dxmc_run_cfg& cfg, const World<float>& w, const Tables<float>& t, const Exposure<float>* exps,
-    const uint64_t* expStart, uint32_t nExp, uint64_t hb, uint64_t he, const Tally& tally, Counters* ctr, unsigned long long* historyCounter)
+    const uint64_t* expStart, uint32_t nExp, uint64_t hb, uint64_t he, const Tally& tally, Counters* ctr, unsigned long long* historyCounter, bool pencilBeam)
 {
+    const bool pencil = pencilBeam && w.index24;
     // the work counter is cleared by a kernel, not a memset, so the launch
     // sequence stays valid under stream capture
     auto* nx = historyCounter;
@@ -589,9 +601,9 @@ void launchFp32(dxmc_ctx* c, const dxmc_run_cfg& cfg, const World<float>& w, con
     // of fewer waves, spread over the CUs
     const uint64_t wavesNeeded = (he - hb + 63) / 64;
     const uint32_t wavesPerBlock = static_cast<uint32_t>(std::clamp<uint64_t>((wavesNeeded + c->numCU - 1) / c->numCU, 1, blockWaves(waves)));
-    const uint32_t stage = stageLevelFp32(cfg, tables, waves, kind);
-    const uint32_t slots = poolSlots(tables, stage, cfg.low_energy_correction, wavesPerBlock, kind);
-    const uint32_t lds = ldsBytes(tables, stage, cfg.low_energy_correction) + (kind == WORLD_CODES8 && stage >= STAGE_SMALL ? boundsBytes(tables) : 0u) + wavesPerBlock * slots * SLOT_BYTES;
+    const uint32_t stage = stageLevelFp32(cfg, tables, waves, kind, pencil);
+    const uint32_t slots = poolSlots(tables, stage, cfg.low_energy_correction, wavesPerBlock, kind, pencil);
+    const uint32_t lds = ldsBytes(tables, stage, cfg.low_energy_correction) + (pencil ? SCORE_CACHE_BYTES : 0u) + (kind == WORLD_CODES8 && stage >= STAGE_SMALL ? boundsBytes(tables) : 0u) + wavesPerBlock * slots * SLOT_BYTES;
     const uint32_t perCU = cfg.blocks_per_cu ? cfg.blocks_per_cu : 2u;
     // lanes without a photon before they are refilled (ms: CT spiral 8 185,
     // 12 180.5, 16 178.8, 20 181; DX 12 19.6, 16 19.3; impulse approximation
@@ -604,6 +616,6 @@ void launchFp32(dxmc_ctx* c, const dxmc_run_cfg& cfg, const World<float>& w, con
     // histories a wave claims per atomic on the global counter
     const uint32_t pool = cfg.queue_depth ? std::clamp<uint32_t>(cfg.queue_depth, 64u, 1u << 16) : historiesPerClaim(he - hb, grid * wavesPerBlock);
     hipLaunchKernelGGL(kernelFor(cfg.low_energy_correction, waves, stage, kind), dim3(static_cast<uint32_t>(grid)), dim3(64 * wavesPerBlock), lds, c->stream,
-        world, tables, exps, expStart, nExp, hb, he, cfg.seed, cfg.first_history, tally, ctr, nx, refill, interact, pool, slots);
+        world, tables, exps, expStart, nExp, hb, he, cfg.seed, cfg.first_history, tally, ctr, nx, refill, interact, pool, slots, pencil);
 }
 }

@@ -86,7 +86,7 @@ struct Args64 {
     Tally tally;
     Counters* ctr;
     unsigned long long* next;
-    uint32_t nExp, refillThreshold, interactThreshold, poolSize, slots, exactSteps;
+    uint32_t nExp, refillThreshold, interactThreshold, poolSize, slots, exactSteps, pencil;
 };
 
 __device__ inline const Args64& loopArgs()
@@ -140,6 +140,11 @@ __global__ __launch_bounds__(64 * WAVES_PER_CU) __attribute__((amdgpu_waves_per_
     float x32 = 0, maj32 = 0;
     const uint32_t lane = __lane_id();
 
+    const ScoreCache cache(lds + poolAt);
+    if (args.pencil) {
+        poolAt += SCORE_CACHE_BYTES;
+        cache.clear();
+    }
     const uint32_t slots = args.slots;
     uint32_t* pool = reinterpret_cast<uint32_t*>(lds + poolAt + (threadIdx.x / 64) * (slots * SLOT_BYTES));
     uint32_t first = 0, ready = 0, pending = 0; // the ring's window (wave-uniform)
@@ -274,7 +279,10 @@ __global__ __launch_bounds__(64 * WAVES_PER_CU) __attribute__((amdgpu_waves_per_
                 due = false;
             }
             events += deposits.n;
-            scoreWave(a.tally, deposits.n > 0, idx, deposits.first, wide);
+            bool scores = deposits.n > 0;
+            if (a.pencil && scores)
+                scores = !cache.add(static_cast<uint32_t>(idx), deposits.first);
+            scoreWave(a.tally, scores, idx, deposits.first, wide);
             if (K != WORLD_CODES8 && __ballot(deposits.n > 1) != 0) // forced events with a Compton event
                 scoreWave(a.tally, deposits.n > 1, idx, deposits.second, wide);
         } else if (nDue != 0) {
@@ -455,6 +463,8 @@ __global__ __launch_bounds__(64 * WAVES_PER_CU) __attribute__((amdgpu_waves_per_
                 break;
         }
     }
+    if (args.pencil)
+        cache.flush(args.tally);
     if (args.ctr)
         dxmc_backend::accumulateCounters(args.ctr, steps + historySteps, events);
 }
@@ -482,8 +492,9 @@ namespace dxmc_backend {
 
 void launchFp64(dxmc_ctx* c, const dxmc_run_cfg& cfg, const World<double>& w, const Tables<double>& t, const Tables<float>& t32,
     const Exposure<double>* exps, const uint64_t* expStart, uint32_t nExp, uint64_t hb, uint64_t he, const Tally& tally, Counters* ctr,
-    unsigned long long* historyCounter)
+    unsigned long long* historyCounter, bool pencilBeam)
 {
+    const bool pencil = pencilBeam && w.index24;
     // cleared by a kernel, not a memset, so the sequence stays valid under capture
     hipLaunchKernelGGL(clearCounter, dim3(1), dim3(1), 0, c->stream, historyCounter);
     const int L = cfg.low_energy_correction;
@@ -496,7 +507,7 @@ void launchFp64(dxmc_ctx* c, const dxmc_run_cfg& cfg, const World<double>& w, co
     const uint32_t perCU = cfg.blocks_per_cu ? cfg.blocks_per_cu : WAVES_PER_CU / fullBlock;
     const uint32_t wavesPerBlock = static_cast<uint32_t>(std::clamp<uint64_t>((wavesNeeded + c->numCU - 1) / c->numCU, 1, fullBlock));
     auto tablesBytes = [&](uint32_t stage) {
-        return ldsBytes(t, stage, L) + (kind == WORLD_CODES8 && stage >= STAGE_SMALL ? boundsBytes(t) : 0u);
+        return ldsBytes(t, stage, L) + (pencil ? SCORE_CACHE_BYTES : 0u) + (kind == WORLD_CODES8 && stage >= STAGE_SMALL ? boundsBytes(t) : 0u);
     };
     auto poolSlots = [&](uint32_t stage, uint32_t waves) {
         const uint32_t block = 160 * 1024 / (WAVES_PER_CU / fullBlock) - 1280, tables = tablesBytes(stage);
@@ -514,7 +525,7 @@ void launchFp64(dxmc_ctx* c, const dxmc_run_cfg& cfg, const World<double>& w, co
     // histories a wave claims per atomic on the global counter
     const uint32_t pool = cfg.queue_depth ? std::clamp<uint32_t>(cfg.queue_depth, 64u, 1u << 16) : historiesPerClaim(he - hb, grid * wavesPerBlock);
     const Args64 args { w, t, { 1.0 / w.spacing[0], 1.0 / w.spacing[1], 1.0 / w.spacing[2] }, t32.lutCoef, t32.lutSumBound, exps, expStart, hb, he,
-        cfg.seed, cfg.first_history, tally, ctr, historyCounter, nExp, refill, interact, pool, slots, (cfg.flags & DXMC_RUN_EXACT_STEPS) != 0 };
+        cfg.seed, cfg.first_history, tally, ctr, historyCounter, nExp, refill, interact, pool, slots, (cfg.flags & DXMC_RUN_EXACT_STEPS) != 0, pencil };
     hipLaunchKernelGGL(kernelFor(L, staged, kind), dim3(static_cast<uint32_t>(grid)), dim3(64 * wavesPerBlock), lds, c->stream, args);
 }
 }
