@@ -8,7 +8,7 @@
 //                           regeneration threshold, interaction threshold,
 //                           queue depth (histories per pool refill), resident
 //                           blocks per CU
-//   FP64 plain kernel:      block size
+//   FP64 kernel:            block size
 // Each candidate is timed twice (best of two) from HIP events on the stream
 // the kernel runs on. The tuning fields only change scheduling: every
 // history keeps its own random stream, so results do not depend on them.

@@ -11,7 +11,8 @@
 //   Compton scatter (KN, scatter factor)    transport.hpp:300-340, interpolation.hpp:169-176
 //   Compton impulse approximation           transport.hpp:342-483
 //   interaction dispatch, forced dispatch   transport.hpp:523-638
-//   Woodcock delta tracking                 transport.hpp:640-700
+//   Woodcock delta tracking                 transport.hpp:640-700 (the loops of transport_fp32.hip and
+//                                           transport_fp64.hip)
 //   direction deflection                    vectormath.hpp:83-99, 197-221
 // For T = double (the plain method) every expression keeps the reference's
 // operation order so the CPU oracle and this code round identically except
