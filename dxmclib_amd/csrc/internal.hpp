@@ -7,6 +7,7 @@
 
 #include <hip/hip_runtime.h>
 #include <algorithm>
+#include <atomic>
 #include <cstring>
 #include <map>
 #include <mutex>
@@ -308,7 +309,9 @@ struct dxmc_world {
     mutable uint32_t blockDims[3] = { 0, 0, 0 };
     mutable uint32_t blockShift = 0; // block edge 2^blockShift voxels
     mutable uint32_t codeMul = 0; // 1-byte codes: (code * codeMul) >> CODE_MUL_SHIFT is the code's material
-    mutable uint64_t bytes = 0;
+    // device bytes; read by dxmc_hip_world_bytes without the lock, while a
+    // run on another thread may add a palette world's codes
+    mutable std::atomic<uint64_t> bytes { 0 };
 };
 
 struct dxmc_tables {

@@ -713,7 +713,7 @@ int dxmc_hip_world_bytes(const dxmc_world* w, uint64_t* bytes)
 {
     if (!w || !bytes)
         return DXMC_ERR_ARGUMENT;
-    *bytes = w->bytes;
+    *bytes = w->bytes.load(std::memory_order_relaxed);
     return DXMC_OK;
 }
 
