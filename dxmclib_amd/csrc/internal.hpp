@@ -181,8 +181,9 @@ struct dxmc_ctx {
         const void* src;
         size_t bytes;
     };
-    // device -> host, complete on return: the arrays as one stream of bytes
-    // (into the caller's page-locked memory each array goes by itself)
+    // device -> host, complete on return. Arrays that fit the ring together go
+    // through it; of others those in the caller's page-locked memory go direct,
+    // each by itself, and the pageable ones as one stream of bytes.
     int download(const Fetch* list, int count)
     {
         size_t total = 0;
@@ -190,30 +191,54 @@ struct dxmc_ctx {
             total += list[k].bytes;
         if (total == 0)
             return DXMC_OK;
-        if (unsigned char* p = ringSpace(total)) {
-            size_t off = 0;
-            for (int k = 0; k < count; off += list[k++].bytes)
-                if (list[k].bytes)
-                    if (int st = check(hipMemcpyAsync(p + off, list[k].src, list[k].bytes, hipMemcpyDeviceToHost, stream)))
-                        return st;
-            if (int st = check(hipStreamSynchronize(stream)))
+        if (unsigned char* p = ringSpace(total))
+            return downloadRing(p, list, count);
+        std::vector<Fetch> pageable;
+        size_t pageableBytes = 0;
+        for (int k = 0; k < count; ++k) {
+            if (list[k].bytes && !dxmc_backend::pinnedHost(list[k].dst, list[k].bytes)) {
+                pageable.push_back(list[k]);
+                pageableBytes += list[k].bytes;
+            } else if (int st = downloadDirect(list[k])) {
                 return st;
-            off = 0;
-            for (int k = 0; k < count; off += list[k++].bytes)
-                if (list[k].bytes)
-                    std::memcpy(list[k].dst, p + off, list[k].bytes);
-            return DXMC_OK;
+            }
         }
-        bool direct = !staging();
-        for (int k = 0; k < count; ++k)
-            direct = direct || dxmc_backend::pinnedHost(list[k].dst, list[k].bytes);
-        if (direct) {
-            for (int k = 0; k < count; ++k)
-                if (list[k].bytes)
-                    if (int st = check(hipMemcpyAsync(list[k].dst, list[k].src, list[k].bytes, hipMemcpyDeviceToHost, stream)))
-                        return st;
-            return check(hipStreamSynchronize(stream));
+        const int left = static_cast<int>(pageable.size());
+        if (unsigned char* p = left ? ringSpace(pageableBytes) : nullptr)
+            return downloadRing(p, pageable.data(), left); // waits for the direct ones too
+        if (left && staging()) {
+            if (int st = downloadChunks(pageable.data(), left))
+                return st;
+        } else {
+            for (const Fetch& f : pageable)
+                if (int st = downloadDirect(f))
+                    return st;
         }
+        return check(hipStreamSynchronize(stream));
+    }
+    // one array straight to its destination (on the stream, without a wait)
+    int downloadDirect(const Fetch& f)
+    {
+        return f.bytes ? check(hipMemcpyAsync(f.dst, f.src, f.bytes, hipMemcpyDeviceToHost, stream)) : DXMC_OK;
+    }
+    // the arrays through 'p' in the ring
+    int downloadRing(unsigned char* p, const Fetch* list, int count)
+    {
+        size_t off = 0;
+        for (int k = 0; k < count; off += list[k++].bytes)
+            if (int st = downloadDirect({ p + off, list[k].src, list[k].bytes }))
+                return st;
+        if (int st = check(hipStreamSynchronize(stream)))
+            return st;
+        off = 0;
+        for (int k = 0; k < count; off += list[k++].bytes)
+            if (list[k].bytes)
+                std::memcpy(list[k].dst, p + off, list[k].bytes);
+        return DXMC_OK;
+    }
+    // the arrays as one stream of bytes through the staging chunks
+    int downloadChunks(const Fetch* list, int count)
+    {
         // chunks across the arrays: a chunk holds the end of one and the
         // start of the next
         struct Part {

@@ -1,8 +1,12 @@
 """Result arrays come to the host as one stream of bytes: through a 1 MiB
 page-locked ring when they fit it together, else through 16 MiB chunks that
 may hold the end of one array and the start of the next. Sizes at the ring's
-and the chunks' ends give the arrays that downloads one by one give."""
+and the chunks' ends give the arrays that downloads one by one give. Arrays in
+page-locked memory go direct, each by itself: beside them pageable ones keep
+the chunks, and without pageable ones a context makes no chunks (and starts no
+copy threads)."""
 import ctypes as C
+import os
 
 import numpy as np
 import pytest
@@ -47,3 +51,56 @@ def test_arrays_together_and_alone(device, dims):
         device.destroy_tables(t)
         device.destroy_world(w)
     assert int(together[1].sum()) == stats.events > 0
+
+
+HELPERS = 7  # copy threads a context starts with its chunks
+
+
+@pytest.mark.parametrize("n", [60_000, 120_000, 2_100_000])
+@pytest.mark.parametrize("locked", [(1, 1, 1), (1, 0, 0), (0, 1, 0), (0, 1, 1), (0, 0, 0)])
+def test_page_locked_arrays_beside_pageable_ones(n, locked):
+    print(f"result transfers of {n} voxels, page-locked {locked}", flush=True)
+    shape = (1, n // 100, 100)
+    spacing = (2.0, 200.0 / shape[1], 200.0)
+    dtypes, types = (np.float64, np.uint32, np.float64), (C.c_double, C.c_uint32, C.c_double)
+    lib = capi.hip()
+    blocks = []
+    with backend.Device(0) as dev:
+        w = dev.upload_world(np.zeros(shape, np.uint8), np.ones(shape, np.float32), spacing, backend.world_extent(shape[::-1], spacing), 1)
+        tables = backend.HostTables(["Water, Liquid"], [1.0], 60.0, 1.0)
+        spec = backend.source_spec(capi.SOURCE_DX, tube_voltage=60.0, al_mm=2.5, sdd=1000.0, field_size=(180.0, 180.0),
+                                   histories_per_exposure=100_000, total_exposures=1)
+        exposures = tables.exposures(spec)
+        t = dev.upload_tables(tables.desc())
+        tally = dev.tally(n)
+        try:
+            dev.run(w, t, exposures, tally, capi.PRECISION_FP32, 1, seed=4)
+            with backend.Device(0) as other:  # the runtime's own threads are there by now
+                other.synchronize()
+            out = []
+            for lock, dtype in zip(locked, dtypes):
+                if lock:
+                    p = C.c_void_p()
+                    assert lib.dxmc_hip_host_alloc(n * np.dtype(dtype).itemsize, C.byref(p)) == 0
+                    blocks.append(p)
+                    out.append(np.frombuffer((C.c_char * (n * np.dtype(dtype).itemsize)).from_address(p.value), dtype))
+                else:
+                    out.append(np.zeros(n, dtype))
+                out[-1][:] = 7
+            before = len(os.listdir("/proc/self/task"))
+            dev._check(lib.dxmc_hip_tally_download(dev.ctx, tally, *[a.ctypes.data_as(C.POINTER(c)) for a, c in zip(out, types)]))
+            started = len(os.listdir("/proc/self/task")) - before
+            want = [_one(dev, tally, n, which) for which in range(3)]
+            assert want[1].sum() > 0
+            for a, b in zip(out, want):
+                assert np.array_equal(a, b)
+            if n < 2_000_000:  # (that world's upload made the chunks)
+                pageable = sum(n * np.dtype(d).itemsize for lock, d in zip(locked, dtypes) if not lock)
+                assert started >= HELPERS if pageable > 1 << 20 else started < HELPERS
+        finally:
+            del out
+            dev.destroy_tally(tally)
+            dev.destroy_tables(t)
+            dev.destroy_world(w)
+            for p in blocks:
+                assert lib.dxmc_hip_host_free(p) == 0
