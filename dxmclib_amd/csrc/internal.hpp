@@ -96,6 +96,11 @@ struct dxmc_ctx {
     // 87; the link alone takes 49.
     static constexpr size_t RING_BYTES = size_t { 1 } << 20;
     static constexpr size_t STAGE_CHUNK = size_t { 16 } << 20;
+    // bytes of a chunk in a transfer of 'total': below 22 MiB half chunks, so
+    // that DMA and host copy still overlap (one array of 12 MiB down 0.36 ms
+    // in one chunk, 0.31 in two; 15.9 MiB 0.46 and 0.41; three arrays of 20
+    // MiB 0.54 as 16 + 4, 0.48 in three; of 24 MiB 0.58 and 0.62)
+    static constexpr size_t chunkOf(size_t total) { return 8 * total < 11 * STAGE_CHUNK ? STAGE_CHUNK / 2 : STAGE_CHUNK; }
     unsigned char* ring = nullptr;
     size_t ringNext = 0;
     void* stage[2] = { nullptr, nullptr };
@@ -160,9 +165,10 @@ struct dxmc_ctx {
         }
         const auto* from = static_cast<const char*>(src);
         auto* to = static_cast<char*>(dst);
-        for (size_t off = 0, i = 0; off < bytes; off += STAGE_CHUNK, ++i) {
+        const size_t chunk = chunkOf(bytes);
+        for (size_t off = 0, i = 0; off < bytes; off += chunk, ++i) {
             const int b = static_cast<int>(i & 1);
-            const size_t len = std::min(STAGE_CHUNK, bytes - off);
+            const size_t len = std::min(chunk, bytes - off);
             // the chunk's previous DMA (two chunks back) has to be done
             if (i >= 2)
                 if (int st = check(hipEventSynchronize(stageDone[b])))
@@ -207,7 +213,7 @@ struct dxmc_ctx {
         if (unsigned char* p = left ? ringSpace(pageableBytes) : nullptr)
             return downloadRing(p, pageable.data(), left); // waits for the direct ones too
         if (left && staging()) {
-            if (int st = downloadChunks(pageable.data(), left))
+            if (int st = downloadChunks(pageable.data(), left, chunkOf(pageableBytes)))
                 return st;
         } else {
             for (const Fetch& f : pageable)
@@ -237,20 +243,15 @@ struct dxmc_ctx {
         return DXMC_OK;
     }
     // the arrays as one stream of bytes through the staging chunks
-    int downloadChunks(const Fetch* list, int count)
+    int downloadChunks(const Fetch* list, int count, size_t chunk)
     {
         // chunks across the arrays: a chunk holds the end of one and the
         // start of the next
-        struct Part {
-            char* dst;
-            size_t at, len;
-        };
-        std::vector<Part> parts[2];
+        std::vector<dxmc_backend::CopyHelpers::Block> parts[2];
         auto drain = [&](int b) {
             if (int st = check(hipEventSynchronize(stageDone[b])))
                 return st;
-            for (const Part& q : parts[b])
-                helpers.copy(q.dst, static_cast<char*>(stage[b]) + q.at, q.len);
+            helpers.copy(parts[b].data(), static_cast<int>(parts[b].size()));
             parts[b].clear();
             return 0;
         };
@@ -258,14 +259,14 @@ struct dxmc_ctx {
         size_t done = 0; // of the current array
         for (int b = 0; array < count; b ^= 1) {
             size_t used = 0;
-            while (array < count && used < STAGE_CHUNK) {
+            while (array < count && used < chunk) {
                 const Fetch& f = list[array];
-                const size_t len = std::min(STAGE_CHUNK - used, f.bytes - done);
+                const size_t len = std::min(chunk - used, f.bytes - done);
                 if (len) {
                     if (int st = check(hipMemcpyAsync(static_cast<char*>(stage[b]) + used, static_cast<const char*>(f.src) + done, len,
                             hipMemcpyDeviceToHost, stream)))
                         return st;
-                    parts[b].push_back({ static_cast<char*>(f.dst) + done, used, len });
+                    parts[b].push_back({ static_cast<char*>(f.dst) + done, static_cast<char*>(stage[b]) + used, len });
                 }
                 used += len;
                 done += len;

@@ -1,10 +1,12 @@
 // Unit check of the host copies of the staged transfers (CopyHelpers,
-// dxmclib_amd/csrc/hostcopy.hpp): lengths below, at and around the part
-// threshold and the 8 MiB staging chunk, odd lengths and unaligned
-// addresses, repeated copies on the same helpers, and copies without
-// helpers. Prints "ok" and exits 0, or names the failing case and exits 1.
+// dxmclib_amd/csrc/hostcopy.hpp): lengths below, at and around 4 MiB
+// and the 8 MiB half chunk, odd lengths and unaligned
+// addresses, repeated copies on the same helpers, copies without helpers, and
+// copies of several blocks (empty, small and large ones, whose ends fall
+// anywhere in the threads' parts). Prints "ok" and exits 0, or names the failing case and exits 1.
 #include "../../dxmclib_amd/csrc/hostcopy.hpp"
 
+#include <algorithm>
 #include <cstdint>
 #include <cstdio>
 #include <vector>
@@ -45,6 +47,34 @@ int main()
                         }
                     }
                 }
+    }
+    using Block = CopyHelpers::Block;
+    CopyHelpers many;
+    for (int round = 0; round < 2; ++round) {
+        if (round == 1 && !many.start()) {
+            std::printf("helpers did not start\n");
+            return 1;
+        }
+        const std::size_t sets[][3] = { { 0, 0, 0 }, { 1, 2, 3 }, { 0, MiB, 0 }, { 500 * 1024, 7, 24 * 1024 - 7 }, { 500 * 1024, 7, 24 * 1024 - 8 },
+            { 3 * MiB + 1, 0, 5 }, { 5, 2 * MiB + 3, 3 * MiB }, { MiB, MiB / 2, MiB } };
+        for (const auto& set : sets) {
+            std::fill(dst.begin(), dst.end(), 0xA5);
+            Block list[3];
+            std::size_t from = 3, to = 5; // gaps between the blocks on both sides
+            for (int i = 0; i < 3; ++i) {
+                list[i] = { reinterpret_cast<char*>(dst.data() + to), reinterpret_cast<const char*>(src.data() + from), set[i] };
+                from += set[i] + 9;
+                to += set[i] + 2;
+            }
+            many.copy(list, 3);
+            std::vector<unsigned char> want(maxLen, 0xA5);
+            for (const Block& b : list)
+                std::copy(b.src, b.src + b.len, want.data() + (b.dst - reinterpret_cast<char*>(dst.data())));
+            if (want != dst) {
+                std::printf("round %d blocks %zu %zu %zu differ\n", round, set[0], set[1], set[2]);
+                return 1;
+            }
+        }
     }
     std::printf("ok\n");
     return 0;

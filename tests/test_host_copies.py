@@ -1,8 +1,9 @@
 """Host side of the staged host<->device transfers
 (dxmclib_amd/csrc/hostcopy.hpp): the persistent helper threads that copy a
 staging chunk in parts. Built as tests/cpp/bin/copy_helpers; it checks odd
-lengths around the 4 MiB part threshold and the 8 MiB chunk, unaligned
-addresses, repeated copies and copies without helper threads."""
+lengths around 4 MiB and the 8 MiB half chunk, unaligned addresses, repeated
+copies, copies without helper threads, and copies of several blocks below, at
+and above the 512 KiB from which the threads take part."""
 import os
 import subprocess
 

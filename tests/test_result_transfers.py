@@ -1,6 +1,6 @@
 """Result arrays come to the host as one stream of bytes: through a 1 MiB
-page-locked ring when they fit it together, else through 16 MiB chunks that
-may hold the end of one array and the start of the next. Sizes at the ring's
+page-locked ring when they fit it together, else through chunks (of 8 MiB
+below 22 MiB in all, else of 16 MiB) that may hold the end of one array and the start of the next. Sizes at the ring's
 and the chunks' ends give the arrays that downloads one by one give. Arrays in
 page-locked memory go direct, each by itself: beside them pageable ones keep
 the chunks, and without pageable ones a context makes no chunks (and starts no
@@ -27,7 +27,8 @@ def _one(device, tally, n, which):
     return out[which]
 
 
-@pytest.mark.parametrize("dims", [(1, 1, 1), (52428, 1, 1), (52429, 1, 1), (1 << 10, 1 << 11, 1), ((1 << 21) + 1, 1, 1), (1 << 11, 1 << 11, 1), (1999, 1709, 1)])
+@pytest.mark.parametrize("dims", [(1, 1, 1), (52428, 1, 1), (52429, 1, 1), (431, 1009, 1), (1 << 10, 1 << 10, 1), (1153433, 1, 1),
+                                  (1153434, 1, 1), (1 << 10, 1 << 11, 1), ((1 << 21) + 1, 1, 1), (1 << 11, 1 << 11, 1), (1999, 1709, 1)])
 def test_arrays_together_and_alone(device, dims):
     print(f"result transfers {dims}", flush=True)
     shape = dims[::-1]
@@ -104,3 +105,25 @@ def test_page_locked_arrays_beside_pageable_ones(n, locked):
             dev.destroy_world(w)
             for p in blocks:
                 assert lib.dxmc_hip_host_free(p) == 0
+
+
+@pytest.mark.parametrize("n", [(1 << 20) + 3, 2_883_583, 2_883_584, 5_000_011])
+def test_uploads_keep_their_order(device, n):
+    """Arrays of 8, 22 and 38 MiB with ragged ends go up in two, three, two and
+    three chunks: every element arrives in its place."""
+    print(f"uploads of {n} energies", flush=True)
+    names = ["Water, Liquid", "Bone, Cortical (ICRU)"]
+    h = backend.HostTables(names, [1.0, 1.92], 120.0, 1.0)
+    t = device.upload_tables(h.desc())
+    rng = np.random.default_rng(3)
+    mat = rng.integers(0, 2, n)
+    energy = 10 ** rng.uniform(0.0, np.log10(120.0), n)
+    try:
+        att, maj = device.lut_lookup(t, capi.PRECISION_FP64, mat, energy)
+        # the same elements by pieces that fit the ring
+        for k in range(0, n, 1 << 16):
+            s = slice(k, k + (1 << 16))
+            a, m = device.lut_lookup(t, capi.PRECISION_FP64, mat[s], energy[s])
+            assert np.array_equal(a, att[s]) and np.array_equal(m, maj[s])
+    finally:
+        device.destroy_tables(t)
