@@ -75,20 +75,19 @@ __device__ inline uint32_t blockIndexFast(const World<T>& w, uint3 v)
 // them from L1. Staging level: 1 none, 2 all but the attenuation
 // coefficients, 3 all. Of the interaction tables only those of the run's
 // low-energy model are staged (RITA for L >= 1, the scatter-function spline
-// for L = 1, the shells for L = 2). The total-attenuation bounds stay in
-// global memory: in LDS they cost a resident block per CU.
+// for L = 1, the shells for L = 2).
 enum : uint32_t { STAGE_NONE = 1, STAGE_SMALL = 2, STAGE_ALL = 3 };
 
-__host__ __device__ constexpr uint32_t ldsAlign(uint64_t bytes) { return static_cast<uint32_t>((bytes + 15) & ~uint64_t(15)); }
+__host__ __device__ constexpr uint64_t ldsAlign(uint64_t bytes) { return (bytes + 15) & ~uint64_t(15); }
 
 // bytes of LDS a staging level needs for low-energy model L (the same walk
 // as stageTables)
 template <typename T>
-__host__ __device__ inline uint32_t ldsBytes(const Tables<T>& t, uint32_t level, int L)
+__host__ __device__ inline uint64_t ldsBytes(const Tables<T>& t, uint32_t level, int L)
 {
     if (level <= STAGE_NONE)
         return 0;
-    uint32_t b = 0;
+    uint64_t b = 0;
     if (L >= 1)
         b += ldsAlign(uint64_t(t.nMaterials) * 4 * 56 * sizeof(T));
     if (L == 1)
@@ -111,7 +110,7 @@ __host__ __device__ inline uint32_t ldsBytes(const Tables<T>& t, uint32_t level,
 // adds: a flight reads them after the block code (and the voxel code); from
 // LDS instead of L1 they took the CT spiral from 201 to 180 ms
 template <typename T>
-__host__ __device__ inline uint32_t boundsBytes(const Tables<T>& t)
+__host__ __device__ inline uint64_t boundsBytes(const Tables<T>& t)
 {
     return ldsAlign(uint64_t(t.nMaterials) * t.lutNodes * sizeof(float2)) + 256 * sizeof(float2);
 }
@@ -235,6 +234,50 @@ __device__ inline void scoreWave(const Tally& tally, bool has, uint64_t idx, T e
 // of other beams score all over the world and would only fill it.
 constexpr uint32_t SCORE_CACHE_ENTRIES = 256;
 constexpr uint32_t SCORE_CACHE_BYTES = SCORE_CACHE_ENTRIES * (3 * sizeof(double) + sizeof(uint32_t));
+
+// Slots of a wave's photon pool: sampling leaves POOL_RESERVE for photons that
+// become pending, and a wave uses at most POOL_MAX.
+constexpr uint32_t POOL_RESERVE = 16;
+constexpr uint32_t POOL_MAX = 128;
+
+// What a block holds in LDS ahead of its waves' pools: tables of a staging
+// level, on worlds of 1-byte codes also the density and attenuation bounds, in
+// a run of pencil beams the score cache.
+struct LdsPlan {
+    uint32_t stage;
+    bool bounds;
+    uint32_t bytes;
+    uint32_t block, slotBytes;
+    // slots of each wave's pool in a block of so many waves
+    uint32_t slots(uint32_t waves) const { return block <= bytes ? 0u : least(POOL_MAX, (block - bytes) / waves / slotBytes); }
+    static constexpr uint32_t least(uint32_t a, uint32_t b) { return b < a ? b : a; }
+};
+
+// The plan of a launch whose blocks have 'block' bytes of LDS and 'waves'
+// waves: of the requested level, or what of it leaves each pool 'poolMin' slots
+// (set where a fuller pool is worth more than the tables, measured in each
+// kernel's file). The bounds go first: they and the sampling tables take 1.1 KB
+// a material each (FP32; FP64 2.2 KB of tables), so the tables alone fit with
+// about twice the materials. Dropped together, code worlds of 20 and more
+// materials read everything from global memory (20 materials, 192x160x120, 2e7
+// histories FP32, L = 1: 3.85 ms; with the tables 3.35; L = 2, 24 materials
+// 7.45 and 6.35).
+template <typename T>
+inline LdsPlan planLds(const Tables<T>& t, uint32_t level, int L, bool codes8, bool pencil, uint32_t block, uint32_t waves, uint32_t slotBytes,
+    uint32_t poolMin)
+{
+    const uint64_t pools = uint64_t(waves) * poolMin * slotBytes;
+    for (;; --level) {
+        const uint64_t tables = ldsBytes(t, level, L) + (pencil ? SCORE_CACHE_BYTES : 0u);
+        if (level <= STAGE_NONE)
+            return { STAGE_NONE, false, static_cast<uint32_t>(tables), block, slotBytes };
+        if (codes8 && tables + boundsBytes(t) + pools <= block)
+            return { level, true, static_cast<uint32_t>(tables + boundsBytes(t)), block, slotBytes };
+        // (without the bounds, code worlds have a kernel at level 2 only)
+        if (!(codes8 && level >= STAGE_ALL) && tables + pools <= block)
+            return { level, false, static_cast<uint32_t>(tables), block, slotBytes };
+    }
+}
 
 struct ScoreCache {
     static constexpr uint32_t FREE = 0xffffffffu; // no voxel index where indices fit 24-bit products

@@ -38,7 +38,7 @@
 // by multiplication with the reciprocal spacing, FP32 denormals flushed);
 // each scoring event is added to the FP64 tallies with hardware FP64
 // atomics. The kernel is compiled per low-energy model, register budget
-// (4 or 6 waves per SIMD), LDS staging level and world kind.
+// (4 or 6 waves per SIMD), LDS staging and world kind.
 #include "device/persistent.hpp"
 #include "internal.hpp"
 
@@ -74,9 +74,6 @@ constexpr float LN2F = 0.693147180559945309f;
 // computed again when a lane takes the photon.
 constexpr uint32_t SLOT_WORDS = 13;
 constexpr uint32_t SLOT_BYTES = SLOT_WORDS * 4;
-constexpr uint32_t POOL_RESERVE = 16; // slots that sampling leaves for photons that become pending
-constexpr uint32_t POOL_MAX = 128; // most slots a wave uses
-constexpr uint32_t POOL_MIN = 48;
 constexpr uint32_t FLIGHTS_PER_LOOP = 64; // most flights before the outer loop runs
 
 // Waves of a block: two blocks fill a CU's 4 W waves, so the staged tables
@@ -99,9 +96,10 @@ __device__ inline bool roulette(Particle<float>& p, Rng& rng)
 // (128 VGPRs; CT spiral 206 ms, 6: 180). Blocks of 10 or 14 waves load the
 // SIMDs unevenly, so that a CU holds one instead of two (340 ms); 16 waves
 // with 64 VGPRs spill (282 ms).
-// S: LDS staging level. K: world kind. The autotuner picks among the register
-// budgets and staging levels.
-template <int L, int W, uint32_t S, uint32_t K>
+// S: LDS staging level. K: world kind. BOUNDS_LDS: density intervals and
+// attenuation bounds of a code world in LDS too. The autotuner picks among the
+// register budgets and staging levels.
+template <int L, int W, uint32_t S, uint32_t K, bool BOUNDS_LDS>
 __global__ __launch_bounds__(64 * blockWaves(W)) __attribute__((amdgpu_waves_per_eu(W, 8))) void transportPersistent(World<float> w, Tables<float> tg, const Exposure<float>* exps, const uint64_t* expStart,
     uint32_t nExp, uint64_t hBegin, uint64_t hEnd, uint64_t seed, uint64_t firstHistory, Tally tally, Counters* ctr, unsigned long long* next,
     uint32_t refillThreshold, uint32_t interactThreshold, uint32_t poolSize, uint32_t slots, bool pencil)
@@ -109,8 +107,7 @@ __global__ __launch_bounds__(64 * blockWaves(W)) __attribute__((amdgpu_waves_per
     extern __shared__ __align__(16) unsigned char lds[];
     Tables<float> t = tg;
     stageTables<float, S, L>(t, lds);
-    const float2* bounds = nullptr; // CODES8, staged: density interval of each code
-    constexpr bool BOUNDS_LDS = K == WORLD_CODES8 && S >= STAGE_SMALL;
+    const float2* bounds = nullptr; // staged: density interval of each code
     if constexpr (BOUNDS_LDS) {
         unsigned char* c = lds + ldsBytes(tg, S, L);
         t.lutSumBound = stageArray(t.lutSumBound, uint64_t(t.nMaterials) * t.lutNodes, c);
@@ -147,7 +144,7 @@ __global__ __launch_bounds__(64 * blockWaves(W)) __attribute__((amdgpu_waves_per
     const uint64_t launchFirst = firstHistory + hBegin;
     const uint32_t lane = __lane_id();
 
-    uint32_t poolAt = ldsBytes(tg, S, L) + (BOUNDS_LDS ? boundsBytes(tg) : 0u);
+    uint32_t poolAt = static_cast<uint32_t>(ldsBytes(tg, S, L) + (BOUNDS_LDS ? boundsBytes(tg) : 0u));
     const ScoreCache cache(lds + poolAt);
     if (pencil) {
         poolAt += SCORE_CACHE_BYTES;
@@ -495,30 +492,35 @@ using KernelFn = void (*)(World<float>, Tables<float>, const Exposure<float>*, c
     Tally, Counters*, unsigned long long*, uint32_t, uint32_t, uint32_t, uint32_t, bool);
 
 // waves: resolved by wavesFp32
-template <int L, uint32_t S, uint32_t K>
+template <int L, uint32_t S, uint32_t K, bool B>
 KernelFn variant(uint32_t waves)
 {
-    return waves >= 6 ? transportPersistent<L, 6, S, K> : transportPersistent<L, 4, S, K>;
+    return waves >= 6 ? transportPersistent<L, 6, S, K, B> : transportPersistent<L, 4, S, K, B>;
 }
 
 template <int L, uint32_t K>
-KernelFn variant(uint32_t waves, uint32_t stage)
+KernelFn variant(uint32_t waves, const LdsPlan& plan)
 {
-    return stage >= STAGE_ALL ? variant<L, STAGE_ALL, K>(waves) : stage >= STAGE_SMALL ? variant<L, STAGE_SMALL, K>(waves) : variant<L, STAGE_NONE, K>(waves);
+    constexpr bool B = K == WORLD_CODES8;
+    if (plan.stage >= STAGE_ALL)
+        return variant<L, STAGE_ALL, K, B>(waves);
+    if (plan.stage < STAGE_SMALL)
+        return variant<L, STAGE_NONE, K, false>(waves);
+    return B && plan.bounds ? variant<L, STAGE_SMALL, K, B>(waves) : variant<L, STAGE_SMALL, K, false>(waves);
 }
 
 template <int L>
-KernelFn variant(uint32_t waves, uint32_t stage, uint32_t kind)
+KernelFn variant(uint32_t waves, const LdsPlan& plan, uint32_t kind)
 {
-    return kind == WORLD_CODES8 ? variant<L, WORLD_CODES8>(waves, stage)
-        : kind == WORLD_PALETTE8          ? variant<L, WORLD_PALETTE8>(waves, stage)
-        : kind == WORLD_PALETTE8_MEASURED ? variant<L, WORLD_PALETTE8_MEASURED>(waves, stage)
-                                          : variant<L, WORLD_ANY>(waves, stage);
+    return kind == WORLD_CODES8 ? variant<L, WORLD_CODES8>(waves, plan)
+        : kind == WORLD_PALETTE8          ? variant<L, WORLD_PALETTE8>(waves, plan)
+        : kind == WORLD_PALETTE8_MEASURED ? variant<L, WORLD_PALETTE8_MEASURED>(waves, plan)
+                                          : variant<L, WORLD_ANY>(waves, plan);
 }
 
-KernelFn kernelFor(int L, uint32_t waves, uint32_t stage, uint32_t kind)
+KernelFn kernelFor(int L, uint32_t waves, const LdsPlan& plan, uint32_t kind)
 {
-    return L == 0 ? variant<0>(waves, stage, kind) : L == 1 ? variant<1>(waves, stage, kind) : variant<2>(waves, stage, kind);
+    return L == 0 ? variant<0>(waves, plan, kind) : L == 1 ? variant<1>(waves, plan, kind) : variant<2>(waves, plan, kind);
 }
 
 // the kind a world and its tables run as (after launchFp32 has dropped the
@@ -544,24 +546,24 @@ uint32_t wavesFp32(uint32_t requested, int L)
     return requested == 0 ? (L == 2 ? 4u : 6u) : requested >= 6 ? 6u : 4u;
 }
 
-// slots of a wave's pool in blocks of 'blockOf' waves beside the staged
-// tables (half a CU's 160 KiB less an allocation granule)
-uint32_t poolSlots(const Tables<float>& t, uint32_t stage, int L, uint32_t blockOf, uint32_t kind, bool pencil)
-{
-    const uint32_t tables = ldsBytes(t, stage, L) + (pencil ? SCORE_CACHE_BYTES : 0u) + (kind == WORLD_CODES8 && stage >= STAGE_SMALL ? boundsBytes(t) : 0u), block = 80 * 1024 - 1280;
-    return tables >= block ? 0u : std::min(POOL_MAX, (block - tables) / blockOf / SLOT_BYTES);
-}
+// bytes of LDS of a block: half a CU's 160 KiB less an allocation granule
+constexpr uint32_t BLOCK_LDS = 80 * 1024 - 1280;
+// Slots the staged tables have to leave a wave's pool. Code worlds of
+// 192x160x120, 2e7 histories, ms at 48, 60, 72, 84, 96: 14 materials 3.28 3.32
+// 3.02 3.04 3.63, 18 materials 3.68 3.29 3.30 3.27 3.78, 36 materials 4.17 4.03
+// 4.04 4.06 4.09; L = 2, 18 materials 6.83 6.90 5.95 6.01 5.99, 30 materials
+// 7.12 7.05 7.04 7.56 7.49.
+constexpr uint32_t POOL_MIN = 72;
 
-// staging level of a run: the requested one, or by default the sampling
-// tables, lowered while the tables leave a wave's pool too few slots. The
-// attenuation coefficients are staged on request only: they are read once an
-// interaction, and the pool slots they would take are worth more.
-uint32_t stageLevelFp32(const dxmc_run_cfg& cfg, const Tables<float>& t, uint32_t W, uint32_t kind, bool pencil)
+// what a run stages: the requested level, or by default the sampling tables
+// (with the bounds of code worlds), less what leaves a wave's pool too few
+// slots. The attenuation coefficients are staged on request only: they are
+// read once an interaction, and the pool slots they would take are worth more.
+LdsPlan planFp32(const dxmc_run_cfg& cfg, const Tables<float>& t, uint32_t W, uint32_t kind, bool pencil)
 {
-    uint32_t level = cfg.lds_tables >= STAGE_NONE && cfg.lds_tables <= STAGE_ALL ? cfg.lds_tables : STAGE_SMALL;
-    while (level > STAGE_NONE && poolSlots(t, level, cfg.low_energy_correction, blockWaves(W), kind, pencil) < POOL_MIN)
-        --level;
-    return level;
+    const uint32_t level = cfg.lds_tables >= STAGE_NONE && cfg.lds_tables <= STAGE_ALL ? cfg.lds_tables : STAGE_SMALL;
+    return planLds(t, level, cfg.low_energy_correction, kind == WORLD_CODES8, pencil, BLOCK_LDS, blockWaves(W), SLOT_BYTES,
+        POOL_MIN);
 }
 
 void launchFp32(dxmc_ctx* c, const dxmc_run_cfg& cfg, const World<float>& w, const Tables<float>& t, const Exposure<float>* exps,
@@ -601,9 +603,9 @@ void launchFp32(dxmc_ctx* c, const dxmc_run_cfg& cfg, const World<float>& w, con
     // of fewer waves, spread over the CUs
     const uint64_t wavesNeeded = (he - hb + 63) / 64;
     const uint32_t wavesPerBlock = static_cast<uint32_t>(std::clamp<uint64_t>((wavesNeeded + c->numCU - 1) / c->numCU, 1, blockWaves(waves)));
-    const uint32_t stage = stageLevelFp32(cfg, tables, waves, kind, pencil);
-    const uint32_t slots = poolSlots(tables, stage, cfg.low_energy_correction, wavesPerBlock, kind, pencil);
-    const uint32_t lds = ldsBytes(tables, stage, cfg.low_energy_correction) + (pencil ? SCORE_CACHE_BYTES : 0u) + (kind == WORLD_CODES8 && stage >= STAGE_SMALL ? boundsBytes(tables) : 0u) + wavesPerBlock * slots * SLOT_BYTES;
+    const LdsPlan plan = planFp32(cfg, tables, waves, kind, pencil);
+    const uint32_t slots = plan.slots(wavesPerBlock);
+    const uint32_t lds = plan.bytes + wavesPerBlock * slots * SLOT_BYTES;
     const uint32_t perCU = cfg.blocks_per_cu ? cfg.blocks_per_cu : 2u;
     // lanes without a photon before they are refilled (ms: CT spiral 8 185,
     // 12 180.5, 16 178.8, 20 181; DX 12 19.6, 16 19.3; impulse approximation
@@ -615,7 +617,7 @@ void launchFp32(dxmc_ctx* c, const dxmc_run_cfg& cfg, const World<float>& w, con
     const uint64_t grid = std::clamp<uint64_t>((wavesNeeded + wavesPerBlock - 1) / wavesPerBlock, 1, static_cast<uint64_t>(c->numCU) * perCU);
     // histories a wave claims per atomic on the global counter
     const uint32_t pool = cfg.queue_depth ? std::clamp<uint32_t>(cfg.queue_depth, 64u, 1u << 16) : historiesPerClaim(he - hb, grid * wavesPerBlock);
-    hipLaunchKernelGGL(kernelFor(cfg.low_energy_correction, waves, stage, kind), dim3(static_cast<uint32_t>(grid)), dim3(64 * wavesPerBlock), lds, c->stream,
+    hipLaunchKernelGGL(kernelFor(cfg.low_energy_correction, waves, plan, kind), dim3(static_cast<uint32_t>(grid)), dim3(64 * wavesPerBlock), lds, c->stream,
         world, tables, exps, expStart, nExp, hb, he, cfg.seed, cfg.first_history, tally, ctr, nx, refill, interact, pool, slots, pencil);
 }
 }

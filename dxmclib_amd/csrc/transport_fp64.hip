@@ -45,10 +45,14 @@ constexpr float FILTER_MARGIN = 1e-4f;
 constexpr uint32_t SLOT_DOUBLES = 10;
 constexpr uint32_t SLOT_WORDS = 2 * SLOT_DOUBLES + 5;
 constexpr uint32_t SLOT_BYTES = SLOT_WORDS * 4;
-constexpr uint32_t POOL_RESERVE = 16; // slots that sampling leaves for photons that become pending
-constexpr uint32_t POOL_MAX = 128, POOL_MIN = 48;
 constexpr uint32_t FLIGHTS_PER_LOOP = 64; // most flights before the outer loop runs
 constexpr uint32_t WAVES_PER_CU = 8; // 2 a SIMD
+// Slots the staged tables have to leave a wave's pool. Code worlds of
+// 192x160x120, 5e6 histories, ms at 48, 60, 72, 84, 96: 27 materials 3.38 3.42
+// 3.68 3.33 3.32, 30 materials 3.62 3.00 3.04 2.91 2.95, 40 materials 3.30 3.32
+// 3.32 3.23 3.11; L = 2, 24 materials 5.16 5.06 4.55 4.40 4.41, 30 materials
+// 4.91 4.91 4.86 4.88 4.56, 36 materials 7.05 7.20 6.18 6.23 6.17.
+constexpr uint32_t POOL_MIN = 96;
 
 // voxel coordinate (uint32_t)((pos - lower) / spacing) of the plain method,
 // clamped to the grid: the product q with the reciprocal differs from the
@@ -97,23 +101,23 @@ __device__ inline const Args64& loopArgs()
 }
 
 // K: world kind (WORLD_CODES8 with block codes, or WORLD_ANY: palette or
-// 8-byte records). S: LDS staging level. Two waves per SIMD (256 VGPRs): the
+// 8-byte records). S: LDS staging level. BOUNDS_LDS: the bounds of a code world
+// staged too. Two waves per SIMD (256 VGPRs): the
 // FP64 samplers' temporaries spill with less. CT spiral 384x384x200, 4e7
 // histories: 148 ms for the plain form (one thread a history); without pools
 // 50.5 ms with 5 waves, 33.7 with 4, 28.4 with 3; with pools 31.6 with 4, 22.4
 // with 3, 21.8 with 2 (181 wave instructions a history, vector issue 59 %
 // busy). CTDI phantom, 2e7 histories: 19.9 ms plain, 8.7 without pools, 6.8.
-template <int L, uint32_t S, uint32_t K>
+template <int L, uint32_t S, uint32_t K, bool BOUNDS_LDS>
 __global__ __launch_bounds__(64 * WAVES_PER_CU) __attribute__((amdgpu_waves_per_eu(2, 8))) void transportPersistent64(Args64 args)
 {
     extern __shared__ __align__(16) unsigned char lds[];
     Tables<double> t = args.t;
     stageTables<double, S, L>(t, lds);
     // density intervals and attenuation bounds of code worlds
-    constexpr bool BOUNDS_LDS = K == WORLD_CODES8 && S >= STAGE_SMALL;
     const float2* sumBound = args.sumBound;
     const float2* bounds = nullptr;
-    uint32_t poolAt = ldsBytes(args.t, S, L);
+    uint32_t poolAt = static_cast<uint32_t>(ldsBytes(args.t, S, L));
     if constexpr (BOUNDS_LDS) {
         unsigned char* c = lds + poolAt;
         sumBound = stageArray(args.sumBound, uint64_t(t.nMaterials) * t.lutNodes, c);
@@ -121,7 +125,7 @@ __global__ __launch_bounds__(64 * WAVES_PER_CU) __attribute__((amdgpu_waves_per_
         for (uint32_t i = threadIdx.x; i < 256; i += blockDim.x)
             d[i] = make_float2(args.w.bounds[i].lo, args.w.bounds[i].hi);
         bounds = d;
-        poolAt += boundsBytes(args.t);
+        poolAt += static_cast<uint32_t>(boundsBytes(args.t));
         __syncthreads();
     }
     Particle<double> p;
@@ -473,18 +477,17 @@ __global__ void clearCounter(unsigned long long* counter) { *counter = 0; }
 
 using KernelFn = void (*)(Args64);
 
-template <int L, uint32_t S>
-KernelFn variant(uint32_t kind)
+template <int L>
+KernelFn variant(const LdsPlan& plan, uint32_t kind)
 {
-    return kind == WORLD_CODES8 ? transportPersistent64<L, S, WORLD_CODES8> : transportPersistent64<L, S, WORLD_ANY>;
+    if (kind != WORLD_CODES8)
+        return plan.stage >= STAGE_SMALL ? transportPersistent64<L, STAGE_SMALL, WORLD_ANY, false> : transportPersistent64<L, STAGE_NONE, WORLD_ANY, false>;
+    return plan.bounds ? transportPersistent64<L, STAGE_SMALL, WORLD_CODES8, true>
+        : plan.stage >= STAGE_SMALL ? transportPersistent64<L, STAGE_SMALL, WORLD_CODES8, false>
+                                    : transportPersistent64<L, STAGE_NONE, WORLD_CODES8, false>;
 }
 
-KernelFn kernelFor(int L, bool staged, uint32_t kind)
-{
-    if (staged)
-        return L == 0 ? variant<0, STAGE_SMALL>(kind) : L == 1 ? variant<1, STAGE_SMALL>(kind) : variant<2, STAGE_SMALL>(kind);
-    return L == 0 ? variant<0, STAGE_NONE>(kind) : L == 1 ? variant<1, STAGE_NONE>(kind) : variant<2, STAGE_NONE>(kind);
-}
+KernelFn kernelFor(int L, const LdsPlan& plan, uint32_t kind) { return L == 0 ? variant<0>(plan, kind) : L == 1 ? variant<1>(plan, kind) : variant<2>(plan, kind); }
 
 }
 
@@ -506,17 +509,10 @@ void launchFp64(dxmc_ctx* c, const dxmc_run_cfg& cfg, const World<double>& w, co
     const uint32_t fullBlock = cfg.block_size ? cfg.block_size / 64 : WAVES_PER_CU;
     const uint32_t perCU = cfg.blocks_per_cu ? cfg.blocks_per_cu : WAVES_PER_CU / fullBlock;
     const uint32_t wavesPerBlock = static_cast<uint32_t>(std::clamp<uint64_t>((wavesNeeded + c->numCU - 1) / c->numCU, 1, fullBlock));
-    auto tablesBytes = [&](uint32_t stage) {
-        return ldsBytes(t, stage, L) + (pencil ? SCORE_CACHE_BYTES : 0u) + (kind == WORLD_CODES8 && stage >= STAGE_SMALL ? boundsBytes(t) : 0u);
-    };
-    auto poolSlots = [&](uint32_t stage, uint32_t waves) {
-        const uint32_t block = 160 * 1024 / (WAVES_PER_CU / fullBlock) - 1280, tables = tablesBytes(stage);
-        return tables >= block ? 0u : std::min(POOL_MAX, (block - tables) / waves / SLOT_BYTES);
-    };
-    const bool staged = poolSlots(STAGE_SMALL, fullBlock) >= POOL_MIN;
-    const uint32_t stage = staged ? STAGE_SMALL : STAGE_NONE;
-    const uint32_t slots = poolSlots(stage, wavesPerBlock);
-    const uint32_t lds = tablesBytes(stage) + wavesPerBlock * slots * SLOT_BYTES;
+    const LdsPlan plan = planLds(t, STAGE_SMALL, L, kind == WORLD_CODES8, pencil, 160 * 1024 / (WAVES_PER_CU / fullBlock) - 1280, fullBlock, SLOT_BYTES,
+        POOL_MIN);
+    const uint32_t slots = plan.slots(wavesPerBlock);
+    const uint32_t lds = plan.bytes + wavesPerBlock * slots * SLOT_BYTES;
     // thresholds on CT spiral, ms: interaction 48 22.3, 56 21.8, 64 21.9;
     // refill 10 22.2, 16 21.9, 20 21.9, 28 22.5
     const uint32_t refill = cfg.regeneration_threshold ? std::min<uint32_t>(cfg.regeneration_threshold, 64u) : 16u;
@@ -526,6 +522,6 @@ void launchFp64(dxmc_ctx* c, const dxmc_run_cfg& cfg, const World<double>& w, co
     const uint32_t pool = cfg.queue_depth ? std::clamp<uint32_t>(cfg.queue_depth, 64u, 1u << 16) : historiesPerClaim(he - hb, grid * wavesPerBlock);
     const Args64 args { w, t, { 1.0 / w.spacing[0], 1.0 / w.spacing[1], 1.0 / w.spacing[2] }, t32.lutCoef, t32.lutSumBound, exps, expStart, hb, he,
         cfg.seed, cfg.first_history, tally, ctr, historyCounter, nExp, refill, interact, pool, slots, (cfg.flags & DXMC_RUN_EXACT_STEPS) != 0, pencil };
-    hipLaunchKernelGGL(kernelFor(L, staged, kind), dim3(static_cast<uint32_t>(grid)), dim3(64 * wavesPerBlock), lds, c->stream, args);
+    hipLaunchKernelGGL(kernelFor(L, plan, kind), dim3(static_cast<uint32_t>(grid)), dim3(64 * wavesPerBlock), lds, c->stream, args);
 }
 }
