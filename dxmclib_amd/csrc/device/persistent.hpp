@@ -279,6 +279,24 @@ inline LdsPlan planLds(const Tables<T>& t, uint32_t level, int L, bool codes8, b
     }
 }
 
+// Whether a run with this plan uses a world's codes (one that sets block_bounds
+// does in any case). Worlds of 8-byte records always do. A palette's records can be as fast where the bounds are not in
+// LDS (18 and more materials): FP64 drew or lost up to 7 % with codes (30
+// materials, 1e6 to 6.7e7 voxels, 5e6 histories: 3.45 ms with records, 3.57
+// with codes). FP32 gains 5 to 59 % on palettes of more than 256 records
+// (CT numbers); on smaller ones it loses 2 to 7 % (30 materials, 3.7e6 voxels,
+// 2e7 histories: 3.44 ms with records, 3.63 with codes) up to 2e7 voxels, at
+// L = 0 below 3.7e6, and gains 3 to 14 % beyond.
+template <typename T>
+inline bool codesPay(const LdsPlan& plan, uint32_t voxelBytes, uint64_t voxels, int L)
+{
+    if (voxelBytes == 8 || plan.bounds)
+        return true;
+    if (sizeof(T) == 8)
+        return false;
+    return voxelBytes == 2 || voxels >= (uint64_t(1) << (L == 0 ? 22 : 25));
+}
+
 struct ScoreCache {
     static constexpr uint32_t FREE = 0xffffffffu; // no voxel index where indices fit 24-bit products
     double* sums; // dose, variance, events of each entry

@@ -551,6 +551,9 @@ int dxmc_hip_run_monitored(dxmc_ctx* c, const dxmc_world* w, const dxmc_tables* 
         return st;
     DXMC_CHECK(c, hipSetDevice(c->device));
     dxmc_run_cfg run = *cfg;
+    // before tuning, so that the trials run the kernel the run will
+    if ((st = preparePaletteCodes(c, w, t, exposures, nExp, run, true)))
+        return st;
     if (run.flags & DXMC_RUN_AUTOTUNE) {
         const auto key = tuneKey(w, t, run);
         auto it = c->tuned.find(key);
@@ -858,7 +861,7 @@ int runTransport(dxmc_ctx* c, const dxmc_world* w, const dxmc_tables* t, const d
     DXMC_CHECK(c, hipSetDevice(c->device));
     RunBuffers rb(c);
     int st = uploadExposures(c, x, nExp, cfg.precision, rb);
-    if (st || (st = preparePaletteCodes(c, w, rb.totalHistories)))
+    if (st)
         return st;
     const bool counters = (cfg.flags & 1u) != 0 || stats;
     const bool fp64 = cfg.precision == DXMC_PRECISION_FP64;

@@ -322,13 +322,14 @@ struct dxmc_world {
     uint32_t nPalette = 0;
     // Bounded-density code per voxel (u8/u16) and the interval of each code
     // (DensityBound[nCodes]); codeBytes 0: none. 8-byte-record worlds get
-    // them at upload, palette worlds by their first large run (under the
-    // context's lock, hence mutable).
+    // them at upload, palette worlds by a run, once runs pay for them (under
+    // the context's lock, hence mutable).
     mutable void* codes = nullptr;
     mutable void* bounds = nullptr;
     mutable uint32_t codeBytes = 0;
     mutable uint32_t nCodes = 0;
     mutable bool codesTried = false; // palette worlds: the run-time build was done (or failed)
+    mutable uint64_t codeHistories = 0; // palette worlds: histories of the large runs that could use codes
     // 1-byte code worlds: a 2-byte code per block of voxels (smallest |
     // largest code << 8 of a one-material block, else BLOCK_MIXED)
     mutable void* blocks = nullptr;
@@ -500,8 +501,12 @@ inline std::tuple<const void*, const void*, int, int> tuneKey(const dxmc_world* 
 // autotune.hip
 int autotune(dxmc_ctx* c, const dxmc_world* w, const dxmc_tables* t, const dxmc_exposure* x, uint64_t nExp, const dxmc_run_cfg& base,
     uint64_t trialHistories, dxmc_run_cfg& best, dxmc_tune_report* report);
-// codes of a palette world, for a run of so many histories (world.hip)
-int preparePaletteCodes(dxmc_ctx* c, const dxmc_world* w, uint64_t histories);
+// codes of a palette world, once its runs and this one pay for them
+// (world.hip). counts: the run takes place (else it is only being tuned for)
+int preparePaletteCodes(dxmc_ctx* c, const dxmc_world* w, const dxmc_tables* t, const dxmc_exposure* x, uint64_t nExp, const dxmc_run_cfg& cfg, bool counts);
+// whether a run on a world of such voxels with these tables uses 1-byte codes
+bool usesCodesFp32(const dxmc_run_cfg& cfg, const dxmc_dev::Tables<float>& t, uint32_t voxelBytes, uint64_t voxels, bool pencil);
+bool usesCodesFp64(const dxmc_run_cfg& cfg, const dxmc_dev::Tables<double>& t, uint32_t voxelBytes, uint64_t voxels, bool pencil);
 int runTransport(dxmc_ctx* c, const dxmc_world* w, const dxmc_tables* t, const dxmc_exposure* x, uint64_t nExp, const dxmc_run_cfg& cfg,
     dxmc_tally* tally, const dxmc_run_monitor* monitor, dxmc_run_stats* stats);
 // device inputs of a run's launches: exposure records of the run's precision

@@ -566,10 +566,18 @@ LdsPlan planFp32(const dxmc_run_cfg& cfg, const Tables<float>& t, uint32_t W, ui
         POOL_MIN);
 }
 
+bool usesCodesFp32(const dxmc_run_cfg& cfg, const Tables<float>& t, uint32_t voxelBytes, uint64_t voxels, bool pencil)
+{
+    const int L = cfg.low_energy_correction;
+    return cfg.block_bounds != 0 || codesPay<float>(planFp32(cfg, t, wavesFp32(cfg.waves_per_simd, L), WORLD_CODES8, pencil), voxelBytes, voxels, L);
+}
+
 void launchFp32(dxmc_ctx* c, const dxmc_run_cfg& cfg, const World<float>& w, const Tables<float>& t, const Exposure<float>* exps,
     const uint64_t* expStart, uint32_t nExp, uint64_t hb, uint64_t he, const Tally& tally, Counters* ctr, unsigned long long* historyCounter, bool pencilBeam)
 {
     const bool pencil = pencilBeam && w.index24;
+    const int L = cfg.low_energy_correction;
+    const uint64_t voxels = uint64_t(w.nx) * w.ny * w.nz;
     // the work counter is cleared by a kernel, not a memset, so the launch
     // sequence stays valid under stream capture
     auto* nx = historyCounter;
@@ -579,7 +587,7 @@ void launchFp32(dxmc_ctx* c, const dxmc_run_cfg& cfg, const World<float>& w, con
     // the attenuation bounds pay where they also spare the record read
     // (worlds with codes); elsewhere the extra lookup costs more than the
     // evaluations it skips in diverged waves
-    if ((cfg.flags & DXMC_RUN_EXACT_STEPS) || world.codeBytes == 0) {
+    if ((cfg.flags & DXMC_RUN_EXACT_STEPS) || world.codeBytes == 0 || !usesCodesFp32(cfg, t, w.voxelBytes, voxels, pencil)) {
         world.codeBytes = 0;
         tables.lutSumBound = nullptr;
     }
@@ -590,15 +598,15 @@ void launchFp32(dxmc_ctx* c, const dxmc_run_cfg& cfg, const World<float>& w, con
     // from the Infinity Cache saves (401x333x151: 41.1 ms against 39.4), but
     // not more than one from HBM
     constexpr uint64_t INFINITY_CACHE_BYTES = uint64_t(256) << 20;
-    const uint64_t codeArrayBytes = uint64_t(world.nx) * world.ny * world.nz * world.codeBytes;
+    const uint64_t codeArrayBytes = voxels * world.codeBytes;
     const bool blocksOn = world.codeBytes == 1 && world.blocks
-        && (cfg.block_bounds == 1 || (cfg.block_bounds == 0 && !(cfg.low_energy_correction == 2 && codeArrayBytes <= INFINITY_CACHE_BYTES)));
+        && (cfg.block_bounds == 1 || (cfg.block_bounds == 0 && !(L == 2 && codeArrayBytes <= INFINITY_CACHE_BYTES)));
     if (!blocksOn)
         world.blocks = nullptr;
     uint32_t kind = worldKind(world, tables);
-    if (kind == WORLD_CODES8 && !world.blocks && cfg.low_energy_correction < 2)
+    if (kind == WORLD_CODES8 && !world.blocks && L < 2)
         kind = WORLD_ANY;
-    const uint32_t waves = wavesFp32(cfg.waves_per_simd, cfg.low_energy_correction);
+    const uint32_t waves = wavesFp32(cfg.waves_per_simd, L);
     // launches with too few histories for full blocks on every CU get blocks
     // of fewer waves, spread over the CUs
     const uint64_t wavesNeeded = (he - hb + 63) / 64;
@@ -610,14 +618,14 @@ void launchFp32(dxmc_ctx* c, const dxmc_run_cfg& cfg, const World<float>& w, con
     // lanes without a photon before they are refilled (ms: CT spiral 8 185,
     // 12 180.5, 16 178.8, 20 181; DX 12 19.6, 16 19.3; impulse approximation
     // 12 40.9, 16 39.4, 20 38.3, 24 38.7)
-    const uint32_t refill = cfg.regeneration_threshold ? std::min<uint32_t>(cfg.regeneration_threshold, 64u) : cfg.low_energy_correction == 2 ? 20u : 16u;
+    const uint32_t refill = cfg.regeneration_threshold ? std::min<uint32_t>(cfg.regeneration_threshold, 64u) : L == 2 ? 20u : 16u;
     // photons due before they interact, at most half the pool (CT spiral,
     // ms: 32 207, 40 202.4, 48 199.4, 56 198.7 before the bounds were in LDS)
     const uint32_t interact = std::min<uint32_t>(cfg.interaction_threshold ? std::min<uint32_t>(cfg.interaction_threshold, 64u) : 48u, slots / 2);
     const uint64_t grid = std::clamp<uint64_t>((wavesNeeded + wavesPerBlock - 1) / wavesPerBlock, 1, static_cast<uint64_t>(c->numCU) * perCU);
     // histories a wave claims per atomic on the global counter
     const uint32_t pool = cfg.queue_depth ? std::clamp<uint32_t>(cfg.queue_depth, 64u, 1u << 16) : historiesPerClaim(he - hb, grid * wavesPerBlock);
-    hipLaunchKernelGGL(kernelFor(cfg.low_energy_correction, waves, plan, kind), dim3(static_cast<uint32_t>(grid)), dim3(64 * wavesPerBlock), lds, c->stream,
+    hipLaunchKernelGGL(kernelFor(L, waves, plan, kind), dim3(static_cast<uint32_t>(grid)), dim3(64 * wavesPerBlock), lds, c->stream,
         world, tables, exps, expStart, nExp, hb, he, cfg.seed, cfg.first_history, tally, ctr, nx, refill, interact, pool, slots, pencil);
 }
 }

@@ -493,6 +493,26 @@ KernelFn kernelFor(int L, const LdsPlan& plan, uint32_t kind) { return L == 0 ? 
 
 namespace dxmc_backend {
 
+namespace {
+
+// (a block size that is no multiple of 64 is refused before a launch)
+uint32_t blockWaves(const dxmc_run_cfg& cfg) { return cfg.block_size ? std::clamp(cfg.block_size / 64, 1u, WAVES_PER_CU) : WAVES_PER_CU; }
+
+// what a run stages: a block's share of the CU's 160 KiB less an allocation
+// granule
+LdsPlan planFp64(const dxmc_run_cfg& cfg, const Tables<double>& t, bool codes, bool pencil)
+{
+    const uint32_t waves = blockWaves(cfg);
+    return planLds(t, STAGE_SMALL, cfg.low_energy_correction, codes, pencil, 160 * 1024 / (WAVES_PER_CU / waves) - 1280, waves, SLOT_BYTES, POOL_MIN);
+}
+
+}
+
+bool usesCodesFp64(const dxmc_run_cfg& cfg, const Tables<double>& t, uint32_t voxelBytes, uint64_t voxels, bool pencil)
+{
+    return cfg.block_bounds != 0 || codesPay<double>(planFp64(cfg, t, true, pencil), voxelBytes, voxels, cfg.low_energy_correction);
+}
+
 void launchFp64(dxmc_ctx* c, const dxmc_run_cfg& cfg, const World<double>& w, const Tables<double>& t, const Tables<float>& t32,
     const Exposure<double>* exps, const uint64_t* expStart, uint32_t nExp, uint64_t hb, uint64_t he, const Tally& tally, Counters* ctr,
     unsigned long long* historyCounter, bool pencilBeam)
@@ -501,16 +521,17 @@ void launchFp64(dxmc_ctx* c, const dxmc_run_cfg& cfg, const World<double>& w, co
     // cleared by a kernel, not a memset, so the sequence stays valid under capture
     hipLaunchKernelGGL(clearCounter, dim3(1), dim3(1), 0, c->stream, historyCounter);
     const int L = cfg.low_energy_correction;
-    const uint32_t kind = w.index24 && w.codeBytes == 1 && w.blocks && t32.lutSumBound ? WORLD_CODES8 : WORLD_ANY;
+    const bool codes = w.index24 && w.codeBytes == 1 && w.blocks && t32.lutSumBound
+        && usesCodesFp64(cfg, t, w.voxelBytes, uint64_t(w.nx) * w.ny * w.nz, pencil);
+    const uint32_t kind = codes ? WORLD_CODES8 : WORLD_ANY;
     // one block of 8 waves a CU, so the tables are held once and the rest of
     // the LDS is the waves' pools; a block size asked for divides them.
     // Launches with too few histories get blocks of fewer waves.
     const uint64_t wavesNeeded = (he - hb + 63) / 64;
-    const uint32_t fullBlock = cfg.block_size ? cfg.block_size / 64 : WAVES_PER_CU;
+    const uint32_t fullBlock = blockWaves(cfg);
     const uint32_t perCU = cfg.blocks_per_cu ? cfg.blocks_per_cu : WAVES_PER_CU / fullBlock;
     const uint32_t wavesPerBlock = static_cast<uint32_t>(std::clamp<uint64_t>((wavesNeeded + c->numCU - 1) / c->numCU, 1, fullBlock));
-    const LdsPlan plan = planLds(t, STAGE_SMALL, L, kind == WORLD_CODES8, pencil, 160 * 1024 / (WAVES_PER_CU / fullBlock) - 1280, fullBlock, SLOT_BYTES,
-        POOL_MIN);
+    const LdsPlan plan = planFp64(cfg, t, codes, pencil);
     const uint32_t slots = plan.slots(wavesPerBlock);
     const uint32_t lds = plan.bytes + wavesPerBlock * slots * SLOT_BYTES;
     // thresholds on CT spiral, ms: interaction 48 22.3, 56 21.8, 64 21.9;

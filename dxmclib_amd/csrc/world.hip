@@ -18,7 +18,7 @@
 //                   its material and a density interval (Woodcock decisions
 //                   settled from the interval at most steps)
 //   paletteBounds, paletteCodes  the same codes for worlds of palette
-//                   indices, made by the first large FP32 or FP64 run
+//                   indices, made by an FP32 or FP64 run once they pay
 //   blockCodes      with 1-byte codes, the code range of every block of
 //                   8^3 to 64^3 voxels that holds one material (decisions
 //                   settled from the block's interval without reading the
@@ -570,14 +570,35 @@ int fillVoxelRecords(dxmc_ctx* c, dxmc_world* w, ScanResult* dev, ScanResult& ho
 namespace dxmc_backend {
 
 // Gives a palette world the 1-byte codes and block codes that settle most
-// Woodcock decisions without its voxels' records. Made by the first run of
-// 2^22 histories or more rather than at upload: three launches and a byte a
-// voxel, about 60 us with its allocations, which a run of a millisecond
-// repays and a small one does not. Worlds with measurement flags, more than
-// 64 materials or no 24-bit index keep their records.
-int preparePaletteCodes(dxmc_ctx* c, const dxmc_world* w, uint64_t histories)
+// Woodcock decisions without its voxels' records. Made by a run rather than at
+// upload: three launches, a byte a voxel and its allocations take 0.1 ms and 4
+// ps a voxel (8.4e6 voxels 0.13 ms, 6.7e7 0.3-0.5, 1.34e8 0.57-0.7; a process's
+// first 0.2-0.3 ms more), and a history then saves 0.01 to 0.065 ns (segmented,
+// 7 materials; the larger the world the more) or 0.04 to 0.13 ns (CT numbers).
+// They are made by the first run of 2^22 histories that brings such runs to a
+// history for 16 voxels (32 where there are more than 256 records, as CT numbers
+// have): 1.34e8 voxels break even at 9e6-1.2e7 histories segmented and 5e6 with
+// CT numbers, 6.7e7 at 7e6-1e7 and 3e6. By histories alone one run of 4.3e6
+// histories on 1.34e8 segmented voxels took 2.53 ms, without codes 2.22. Worlds
+// with measurement flags, more than 64 materials or no 24-bit index keep their
+// records, and runs that would not use codes neither make them nor count.
+int preparePaletteCodes(dxmc_ctx* c, const dxmc_world* w, const dxmc_tables* t, const dxmc_exposure* x, uint64_t nExp, const dxmc_run_cfg& cfg, bool counts)
 {
-    if (histories < (uint64_t(1) << 22) || w->codesTried || w->voxelBytes > 2 || w->hasMeasurement || w->nMaterials > 64 || !hasIndex24(w))
+    if (w->codesTried || w->voxelBytes > 2 || w->hasMeasurement || w->nMaterials > 64 || !hasIndex24(w) || (cfg.flags & DXMC_RUN_EXACT_STEPS))
+        return DXMC_OK;
+    uint64_t histories = 0;
+    for (uint64_t i = 0; i < nExp; ++i)
+        histories += x[i].n_histories;
+    if (histories < uint64_t(1) << 22)
+        return DXMC_OK;
+    const bool pencil = pencilBeams(x, nExp);
+    if (!(cfg.precision == DXMC_PRECISION_FP64 ? usesCodesFp64(cfg, t->f64, w->voxelBytes, w->n, pencil)
+                                               : usesCodesFp32(cfg, t->f32, w->voxelBytes, w->n, pencil)))
+        return DXMC_OK;
+    histories += w->codeHistories;
+    if (counts)
+        w->codeHistories = histories;
+    if (histories < w->n / (w->voxelBytes == 2 ? 32 : 16))
         return DXMC_OK;
     w->codesTried = true;
     const uint32_t bins = 255 / w->nMaterials;

@@ -99,7 +99,8 @@ typedef struct {
 int dxmc_hip_world_upload(dxmc_ctx* ctx, const dxmc_world_desc* desc, dxmc_world** out);
 int dxmc_hip_world_destroy(dxmc_ctx* ctx, dxmc_world* world);
 /* Bytes the world occupies on the device (a world of palette indices gains a
- * byte a voxel and its block codes in its first run of 2^22 histories or more). */
+ * byte a voxel and its block codes in a run of 2^22 histories or more, the one
+ * that brings such runs to a history for 16 voxels). */
 int dxmc_hip_world_bytes(const dxmc_world* world, uint64_t* bytes);
 /* Largest density of each material over the world's voxels (0 for a material
  * no voxel uses), computed on the device at upload: the scan of

@@ -1,5 +1,7 @@
-"""A palette world's first run of 2^22 histories or more gives it 1-byte codes
-and block codes, as worlds of 8-byte records have from the start. Its
+"""A palette world's first run of 2^22 histories or more (the one that brings
+such runs to a history for 16 voxels) gives it 1-byte codes and block codes, as
+worlds of 8-byte records have from the start; runs that read no codes do not.
+Its
 histories stay those of reading every voxel's record: FP32 and FP64, few and
 many densities a material, empty and odd densities, ragged grids, full and
 part-used material maps."""
@@ -74,3 +76,66 @@ def test_codes_of_palette_worlds_change_nothing(device, kind):
     finally:
         device.destroy_tables(t)
         device.destroy_world(w)
+
+
+def _layers(n_materials, shape, steps=1):
+    names = (NAMES * 16)[:n_materials]
+    mat = np.zeros(shape, np.uint8)
+    mat[:] = (np.arange(shape[1]) * n_materials // shape[1])[None, :, None]
+    dens = np.array((DENSITIES * 16)[:n_materials], np.float32)[mat]
+    if steps > 1:
+        dens = dens * (1 + np.arange(shape[2], dtype=np.float32) % steps / np.float32(1000))
+    return names, mat, dens
+
+
+def _runs(device, names, mat, dens, settings):
+    """world_bytes gained in each of the runs (precision, low-energy model, histories, run fields) on one world"""
+    spacing = tuple(200.0 / s for s in mat.shape[::-1])
+    w = device.upload_world(mat, dens, spacing, backend.world_extent(mat.shape[::-1], spacing), len(names))
+    tables = backend.HostTables(names, device.world_max_density(w, len(names)), 90.0, 1.0)
+    spec = backend.source_spec(capi.SOURCE_DX, tube_voltage=90.0, al_mm=2.5, sdd=1000.0, field_size=(180.0, 180.0), histories_per_exposure=1, total_exposures=4)
+    exposures = tables.exposures(spec)
+    t = device.upload_tables(tables.desc())
+    tally = device.tally(mat.size)
+    gained = []
+    try:
+        for precision, model, histories, fields in settings:
+            print(f"palette codes of {len(names)} materials, {mat.size} voxels: precision {precision} L={model} histories {histories} {fields}", flush=True)
+            for x in exposures:
+                x.n_histories = histories // 4
+            cfg = capi.RunCfg()
+            for k, v in fields.items():
+                setattr(cfg, k, v)
+            before = device.world_bytes(w)
+            device.run(w, t, exposures, tally, precision, model, seed=3, tuning=cfg)
+            gained.append(device.world_bytes(w) - before)
+    finally:
+        device.destroy_tally(tally)
+        device.destroy_tables(t)
+        device.destroy_world(w)
+    return gained
+
+
+def test_codes_come_with_the_histories_that_pay_for_them(device):
+    enough = 1 << 22
+    small = _layers(4, (32, 40, 48))
+    exact = dict(flags=capi.RUN_EXACT_STEPS)
+    for precision in (capi.PRECISION_FP32, capi.PRECISION_FP64):
+        g = _runs(device, *small, [(precision, 1, enough, exact), (precision, 1, enough - 4, {}), (precision, 1, enough, {}), (precision, 1, enough, {})])
+        assert g[0] == g[1] == g[3] == 0 and g[2] >= small[1].size
+    # 7.2e7 voxels need 4.5e6 histories, of large runs that can use codes
+    large = _layers(1, (112, 800, 800))
+    g = _runs(device, *large, [(capi.PRECISION_FP32, 1, enough, exact), (capi.PRECISION_FP32, 1, enough, {}), (capi.PRECISION_FP32, 1, enough, {})])
+    assert g[0] == g[1] == 0 and g[2] >= large[1].size
+
+
+def test_worlds_that_are_as_fast_on_records_keep_them(device):
+    enough = 1 << 22
+    # 40 materials: the bounds are not in LDS
+    segmented, levels = _layers(40, (32, 80, 48)), _layers(40, (32, 80, 48), 40)
+    assert len(np.unique(segmented[2])) <= 256 < len(np.unique(levels[2].astype(np.float64) + 10 * levels[1]))
+    g = _runs(device, *segmented, [(capi.PRECISION_FP64, 1, enough, {}), (capi.PRECISION_FP32, 1, enough, {}), (capi.PRECISION_FP32, 0, enough, {}),
+                                   (capi.PRECISION_FP32, 1, enough, dict(block_bounds=1))])
+    assert g[:3] == [0, 0, 0] and g[3] >= segmented[1].size
+    g = _runs(device, *levels, [(capi.PRECISION_FP64, 1, enough, {}), (capi.PRECISION_FP32, 1, enough, {})])
+    assert g[0] == 0 and g[1] >= levels[1].size
