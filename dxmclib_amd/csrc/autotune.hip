@@ -8,8 +8,12 @@
 //                           regeneration threshold, interaction threshold,
 //                           queue depth (histories per pool refill), resident
 //                           blocks per CU
-//   FP64 kernel:            block size
-// Each candidate is timed twice (best of two) from HIP events on the stream
+//   FP64 kernel:            block size, regeneration threshold, interaction
+//                           threshold, queue depth; on worlds with block
+//                           codes whether they are used where that is not
+//                           the default
+// A palette world that the run would give its codes gets them before the first
+// trial, so the trials run the run's kernel. Each candidate is timed twice (best of two) from HIP events on the stream
 // the kernel runs on. The tuning fields only change scheduling: every
 // history keeps its own random stream, so results do not depend on them.
 #include "dxmc_hip.h"
@@ -112,12 +116,21 @@ int autotune(dxmc_ctx* c, const dxmc_world* w, const dxmc_tables* t, const dxmc_
                 st = searchField(tr, cfg, &dxmc_run_cfg::lds_tables, { 1, 2, 3 }, bestRate);
             if (!st && w->blocks)
                 st = searchField(tr, cfg, &dxmc_run_cfg::block_bounds, { 1, 2 }, bestRate);
-            if (!st && !(st = searchField(tr, cfg, &dxmc_run_cfg::regeneration_threshold, { 4, 6, 10, 12, 16 }, bestRate))
-                && !(st = searchField(tr, cfg, &dxmc_run_cfg::interaction_threshold, { 24, 32, 40, 44 }, bestRate))
+            // on both sides of the defaults (16, at L = 2 20; 48)
+            const std::vector<uint32_t> refill = cfg.low_energy_correction == 2 ? std::vector<uint32_t> { 12, 16, 24, 28, 32 }
+                                                                                : std::vector<uint32_t> { 8, 12, 20, 24, 32 };
+            if (!st && !(st = searchField(tr, cfg, &dxmc_run_cfg::regeneration_threshold, refill, bestRate))
+                && !(st = searchField(tr, cfg, &dxmc_run_cfg::interaction_threshold, { 32, 40, 56, 64 }, bestRate))
                 && !(st = searchField(tr, cfg, &dxmc_run_cfg::queue_depth, { 128, 256, 512, 1024, 2048, 4096 }, bestRate)))
                 st = searchField(tr, cfg, &dxmc_run_cfg::blocks_per_cu, { 1 }, bestRate);
         } else {
-            st = searchField(tr, cfg, &dxmc_run_cfg::block_size, { 64, 128, 256 }, bestRate);
+            // on both sides of the defaults (one block of 512 threads a CU;
+            // 16; 56; 128 to 512 by the launch's size)
+            if (!(st = searchField(tr, cfg, &dxmc_run_cfg::block_size, { 64, 128, 256 }, bestRate)) && w->blocks)
+                st = searchField(tr, cfg, &dxmc_run_cfg::block_bounds, { 1 }, bestRate);
+            if (!st && !(st = searchField(tr, cfg, &dxmc_run_cfg::regeneration_threshold, { 8, 24 }, bestRate))
+                && !(st = searchField(tr, cfg, &dxmc_run_cfg::interaction_threshold, { 40, 64 }, bestRate)))
+                st = searchField(tr, cfg, &dxmc_run_cfg::queue_depth, { 128, 1024 }, bestRate);
         }
     }
     dxmc_hip_tally_destroy(c, scratch);
@@ -145,6 +158,8 @@ extern "C" int dxmc_hip_autotune(dxmc_ctx* c, const dxmc_world* w, const dxmc_ta
     if (st)
         return st;
     DXMC_CHECK(c, hipSetDevice(c->device));
+    if ((st = preparePaletteCodes(c, w, t, x, nExp, *base, false)))
+        return st;
     st = autotune(c, w, t, x, nExp, *base, trialHistories, *best, report);
     if (st)
         return st;

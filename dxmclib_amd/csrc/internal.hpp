@@ -42,8 +42,9 @@ struct dxmc_ctx {
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     void* historyCounter = nullptr; // u64 work counter of the persistent kernel
     void* scratch = nullptr; // device address of the no-allocation run's scratch array (null: unavailable)
-    // autotuner results per (world, tables, precision, low energy correction)
-    std::map<std::tuple<const void*, const void*, int, int>, dxmc_run_cfg> tuned;
+    // autotuner results per (world, tables, precision, low energy correction,
+    // whether the world had codes)
+    std::map<std::tuple<const void*, const void*, int, int, bool>, dxmc_run_cfg> tuned;
     // Held by every entry point for the whole call: the staging chunks, the
     // work counter, the autotuner map and the stream's order of a call's
     // steps are per context, so calls from several threads on one context
@@ -494,9 +495,9 @@ int uploadExposures(dxmc_ctx* c, const dxmc_exposure* x, uint64_t nExp, int prec
 // argument checks shared by dxmc_hip_run and dxmc_hip_autotune (tally may be null)
 int validateRun(dxmc_ctx* c, const dxmc_world* w, const dxmc_tables* t, const dxmc_exposure* x, uint64_t nExp, const dxmc_run_cfg* cfg,
     const dxmc_tally* tally);
-inline std::tuple<const void*, const void*, int, int> tuneKey(const dxmc_world* w, const dxmc_tables* t, const dxmc_run_cfg& cfg)
+inline std::tuple<const void*, const void*, int, int, bool> tuneKey(const dxmc_world* w, const dxmc_tables* t, const dxmc_run_cfg& cfg)
 {
-    return { w, t, cfg.precision, cfg.low_energy_correction };
+    return { w, t, cfg.precision, cfg.low_energy_correction, w->codeBytes != 0 };
 }
 // autotune.hip
 int autotune(dxmc_ctx* c, const dxmc_world* w, const dxmc_tables* t, const dxmc_exposure* x, uint64_t nExp, const dxmc_run_cfg& base,

@@ -229,7 +229,7 @@ typedef struct {
 
 /* dxmc_run_cfg.flags */
 #define DXMC_RUN_COUNTERS 1u /* collect step/event counters */
-#define DXMC_RUN_AUTOTUNE 2u /* fill zero tuning fields from the autotuner (tuned once per world/tables/precision/L and kept in the context) */
+#define DXMC_RUN_AUTOTUNE 2u /* fill zero tuning fields from the autotuner (tuned once per world/tables/precision/L, and again once a palette world has its codes; kept in the context) */
 #define DXMC_RUN_EXACT_STEPS 4u /* evaluate every Woodcock step from the voxel and the full attenuation (in the run's precision), without the bounds that settle most steps (same results, for checks) */
 
 typedef struct {
@@ -299,7 +299,10 @@ int dxmc_hip_run_noalloc(dxmc_ctx* ctx, const dxmc_world* world, const dxmc_tabl
  * searches, one parameter at a time from the defaults, over
  *   FP32: waves_per_simd, lds_tables, block_bounds, regeneration_threshold,
  *         interaction_threshold, queue_depth, blocks_per_cu;
- *   FP64: block_size.
+ *   FP64: block_size, block_bounds (1), regeneration_threshold,
+ *         interaction_threshold, queue_depth.
+ * A palette world that a run of these exposures would give its codes
+ * (dxmc_hip_world_bytes) gets them first.
  * Tuning fields that are non-zero in 'base' are kept fixed. 'best' receives
  * 'base' with the chosen values filled in; the choice is also kept in the
  * context for DXMC_RUN_AUTOTUNE runs on the same world and tables. The
