@@ -1,14 +1,11 @@
 // Pieces shared by the two persistent transport kernels (transport_fp32.hip,
-// transport_fp64.hip): lane phases, ranks among lanes, table access by 32-bit
-// offsets, and the copy of tables into LDS.
+// transport_fp64.hip): world kinds, ranks among lanes, table access by 32-bit
+// offsets, the copy of tables into LDS and the plan of a block's LDS, claims of
+// histories, and the scores of a wave and of a pencil beam's block.
 #pragma once
 #include "physics.hpp"
 
 namespace dxmc_dev {
-
-// A lane of a persistent kernel holds no photon (waits for regeneration),
-// advances Woodcock flights, or has a real interaction due.
-enum : uint32_t { DEAD = 0, FLYING = 1, PENDING = 2 };
 
 // World kinds the persistent kernels are compiled for: the two common layouts
 // get their code width, record width, 24-bit index and bounds table fixed at
@@ -58,6 +55,11 @@ __device__ inline T loadAt(const T* base, uint32_t index)
 {
     return *reinterpret_cast<const T*>(reinterpret_cast<const unsigned char*>(base) + index * static_cast<uint32_t>(sizeof(T)));
 }
+
+// Whether q, a coordinate times the reciprocal spacing, is so near a whole
+// number that the rounded quotient may truncate differently: the product is
+// within 2^-51 q of it.
+__host__ __device__ inline bool nearWhole(double q) { return fabs(q - rint(q)) <= fabs(q) * 0x1p-50; }
 
 // block of a voxel (1-byte code worlds: 24-bit products hold)
 template <typename T>
@@ -228,8 +230,8 @@ __device__ inline void scoreWave(const Tally& tally, bool has, uint64_t idx, T e
 }
 
 // Scores of pencil beams. Their photons interact on one line of voxels, whose
-// cache lines all XCDs then change in turn (95 ns a change of owner against 4
-// ns within an XCD), so a block keeps the sums of up to 256 voxels in LDS,
+// cache lines all XCDs then change in turn (a line's score of three atomics
+// takes 95 ns when all XCDs add to it, 12 ns when one does), so a block keeps the sums of up to 256 voxels in LDS,
 // first come, first served, and adds them to the tally once, at its end. Runs
 // of other beams score all over the world and would only fill it.
 constexpr uint32_t SCORE_CACHE_ENTRIES = 256;

@@ -124,16 +124,17 @@ struct Exposure {
     int32_t spectrum, heel, bowtie, pad;
 };
 
-// Voxel world. FP64 plain path: separate material / density / measurement
-// arrays as the reference. FP32 path: a record per distinct voxel content
-// (x = FP32 density bits, y = material | measurement << 24) in 'palette' and
-// a 1- or 2-byte palette index per voxel in 'voxels' (voxelBytes 1 or 2);
-// worlds with more than 65536 distinct records keep the 8-byte record itself
-// per voxel (voxelBytes 8, palette unused). Such a world may also carry a
-// 1- or 2-byte code per voxel (codeBytes 1 or 2, else 0) that names the
-// voxel's material and an interval holding its density ('bounds'): the
-// Woodcock decision is settled from the interval at most steps, and the
-// 8-byte record is read only when the draw falls inside the interval's
+// Voxel world. A record per distinct voxel content (x = FP32 density bits, y =
+// material | measurement << 24) in 'palette' and a 1- or 2-byte palette index
+// per voxel in 'voxels' (voxelBytes 1 or 2); worlds with more than 65536
+// distinct records keep the 8-byte record itself per voxel (voxelBytes 8,
+// palette unused). The FP64 density of each voxel is in 'density': the FP64
+// kernel decides from it what FP32 bounds leave open. Worlds of 8-byte records
+// without measurement flags carry a 1- or 2-byte code per voxel (codeBytes 1 or
+// 2, else 0) that names the voxel's material and an interval holding its
+// density ('bounds'), palette worlds a 1-byte one once their runs pay for it:
+// the Woodcock decision is settled from the interval at most steps, and the
+// voxel's density is read only when the draw falls inside the interval's
 // acceptance band. A world with 1-byte codes also carries 'blocks': per
 // block of 2^blockShift voxels per edge (8 to 64, the smallest whose table
 // fits 64 KiB; clipped at the grid's upper faces) the smallest

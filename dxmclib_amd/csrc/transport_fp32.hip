@@ -21,9 +21,9 @@
 // and 21 interacted (126 vector instructions a history on the CT spiral
 // workload, 91 with it).
 //
-// What bounds it: the latency of a flight's chain (block code from L2, then
-// intervals and segment bounds from LDS) and vector issue (75 % busy before
-// the bounds moved to LDS). CT spiral 512x512x300, 1e9 histories: 228 ms
+// What bounds it: vector issue (CT spiral: busy 94 % of the cycles, with 58 %
+// of the lanes at work; 75 % before the bounds moved to LDS, when flights
+// waited on them). CT spiral 512x512x300, 1e9 histories: 228 ms
 // with due photons on their lanes and 7 waves a SIMD, 197 with pools and 6
 // waves, 180 with density intervals and attenuation bounds in LDS; axial
 // 1024x1024x128, 4e8: 77, 69, 60 ms; impulse approximation, 401x333x151,
@@ -619,8 +619,9 @@ void launchFp32(dxmc_ctx* c, const dxmc_run_cfg& cfg, const World<float>& w, con
     // 12 180.5, 16 178.8, 20 181; DX 12 19.6, 16 19.3; impulse approximation
     // 12 40.9, 16 39.4, 20 38.3, 24 38.7)
     const uint32_t refill = cfg.regeneration_threshold ? std::min<uint32_t>(cfg.regeneration_threshold, 64u) : L == 2 ? 20u : 16u;
-    // photons due before they interact, at most half the pool (CT spiral,
-    // ms: 32 207, 40 202.4, 48 199.4, 56 198.7 before the bounds were in LDS)
+    // photons due before they interact, 48 or half the pool, 46 of its 93
+    // slots on CT spiral (ms before the bounds were in LDS, with 48 and more
+    // slots to half: 32 207, 40 202.4, 48 199.4, 56 198.7)
     const uint32_t interact = std::min<uint32_t>(cfg.interaction_threshold ? std::min<uint32_t>(cfg.interaction_threshold, 64u) : 48u, slots / 2);
     const uint64_t grid = std::clamp<uint64_t>((wavesNeeded + wavesPerBlock - 1) / wavesPerBlock, 1, static_cast<uint64_t>(c->numCU) * perCU);
     // histories a wave claims per atomic on the global counter

@@ -55,11 +55,8 @@ constexpr uint32_t WAVES_PER_CU = 8; // 2 a SIMD
 constexpr uint32_t POOL_MIN = 96;
 
 // voxel coordinate (uint32_t)((pos - lower) / spacing) of the plain method,
-// clamped to the grid: the product q with the reciprocal differs from the
-// rounded quotient by less than 2^-51 q, so they truncate alike unless q is
-// that near a whole number
-__device__ inline bool nearWhole(double q) { return fabs(q - rint(q)) <= fabs(q) * 0x1p-50; }
-
+// clamped to the grid: from the product with the reciprocal, divided where
+// that may truncate differently
 __device__ inline uint3 voxelCoords64(const World<double>& w, const double* pos, const double* inv)
 {
     double q[3];
@@ -106,7 +103,7 @@ __device__ inline const Args64& loopArgs()
 // FP64 samplers' temporaries spill with less. CT spiral 384x384x200, 4e7
 // histories: 148 ms for the plain form (one thread a history); without pools
 // 50.5 ms with 5 waves, 33.7 with 4, 28.4 with 3; with pools 31.6 with 4, 22.4
-// with 3, 21.8 with 2 (181 wave instructions a history, vector issue 59 %
+// with 3, 21.8 with 2 (186 vector instructions a history, vector issue 58 %
 // busy). CTDI phantom, 2e7 histories: 19.9 ms plain, 8.7 without pools, 6.8.
 template <int L, uint32_t S, uint32_t K, bool BOUNDS_LDS>
 __global__ __launch_bounds__(64 * WAVES_PER_CU) __attribute__((amdgpu_waves_per_eu(2, 8))) void transportPersistent64(Args64 args)

@@ -213,7 +213,7 @@ typedef struct {
     uint64_t first_history; /* global index of the first history of exposure 0 */
     uint64_t histories_per_launch; /* 0: automatic; bounds cancel/progress latency; at most 2^32 */
     uint32_t block_size; /* 0: tuned default */
-    uint32_t blocks_per_cu; /* FP32 persistent kernel occupancy, 0: tuned default */
+    uint32_t blocks_per_cu; /* FP32, FP64: blocks launched per CU, 0: as many as are resident */
     uint32_t regeneration_threshold; /* FP32, FP64: lanes of a wave without a photon to fly before they are refilled, 0: tuned */
     uint32_t flags; /* DXMC_RUN_* bits */
     uint32_t interaction_threshold; /* FP32, FP64: photons of a wave with an interaction due before they run, 0: tuned */

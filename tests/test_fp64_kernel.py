@@ -2,15 +2,19 @@
 takes voxel coordinates from products with the reciprocal spacing. Both must
 give what the FP64 evaluation and the division give.
 
-CPU: the coordinate rule over random and near-whole quotients.
+CPU: the coordinate rule over random and near-whole quotients, in numpy and as
+the kernel's own function (nearWhole) compiled for the host.
 GPU: the same histories (steps, events, event counts) with and without the
 bounds, on every world layout, at ragged sizes, for each low-energy model,
 with runs of one history, of fewer than a wave and of several launches.
 """
+import os
+import subprocess
+
 import numpy as np
 import pytest
 
-from dxmclib_amd import backend, capi
+from dxmclib_amd import backend, build, capi
 
 
 def test_reciprocal_coordinate_equals_division():
@@ -30,6 +34,47 @@ def test_reciprocal_coordinate_equals_division():
             assert np.array_equal(np.trunc(q)[~divide], exact[~divide])
     # the rule is needed: the product alone truncates wrongly near faces
     assert np.any(np.trunc(face * inv) != np.trunc(face / spacing))
+
+
+SOURCE = r"""
+#include "device/persistent.hpp"
+#include <cstdio>
+#include <random>
+int main()
+{
+    std::mt19937_64 rng(4);
+    std::uniform_real_distribution<double> u(0.0, 1.0);
+    const double some[] = { 0.7, 0.8, 0.1, 1.0 / 3.0, 1.5, 1e-3 };
+    long needed = 0;
+    for (long i = 0; i < 4000000; ++i) {
+        const double spacing = i % 2 ? some[rng() % 6] : 0.05 + 6.95 * u(rng), inv = 1.0 / spacing;
+        const double whole = static_cast<double>(rng() % 5000);
+        // anywhere in the grid, or within a few ulp of a voxel face
+        const double d = i % 4 < 2 ? 5000.0 * u(rng) * spacing : whole * spacing * (1.0 + (static_cast<int>(rng() % 7) - 3) * 0x1p-53);
+        const double q = d * inv, exact = d / spacing;
+        const bool differ = static_cast<unsigned>(q) != static_cast<unsigned>(exact);
+        needed += differ;
+        if (differ && !dxmc_dev::nearWhole(q)) {
+            std::printf("spacing %a, distance %a: product %a, quotient %a\n", spacing, d, q, exact);
+            return 1;
+        }
+    }
+    std::printf("%ld products truncate differently\n", needed);
+    return needed > 0 ? 0 : 1;
+}
+"""
+
+
+def test_kernel_coordinate_rule_equals_division(tmp_path):
+    if not os.path.exists(build.HIPCC):
+        pytest.skip("no hipcc")
+    src, exe = tmp_path / "near_whole.hip", tmp_path / "near_whole"
+    src.write_text(SOURCE)
+    r = subprocess.run([build.HIPCC, "-O2", "-std=c++20", "-ffp-contract=off", "--offload-host-only", "-I", os.path.join(build.HERE, "csrc"), str(src),
+                        "-o", str(exe)], capture_output=True, text=True)
+    assert r.returncode == 0, r.stderr
+    r = subprocess.run([str(exe)], capture_output=True, text=True, timeout=60)
+    assert r.returncode == 0, r.stdout
 
 
 NAMES = ["Water, Liquid", "Bone, Cortical (ICRU)", "Lung (ICRU)", "Air, Dry (near sea level)", "Adipose Tissue (ICRP)"]
