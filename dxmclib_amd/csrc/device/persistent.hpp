@@ -242,6 +242,15 @@ constexpr uint32_t SCORE_CACHE_BYTES = SCORE_CACHE_ENTRIES * (3 * sizeof(double)
 constexpr uint32_t POOL_RESERVE = 16;
 constexpr uint32_t POOL_MAX = 128;
 
+// Orders a wave's accesses to its pool: a slot that one lane writes is read by
+// another. The LDS unit keeps a wave's order, so this costs no instruction; it
+// keeps the compiler from moving one lane's accesses across another's.
+__device__ inline void poolFence()
+{
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
+    __builtin_amdgcn_wave_barrier();
+}
+
 // What a block holds in LDS ahead of its waves' pools: tables of a staging
 // level, on worlds of 1-byte codes also the density and attenuation bounds, in
 // a run of pencil beams the score cache.

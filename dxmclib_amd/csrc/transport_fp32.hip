@@ -335,6 +335,7 @@ __global__ __launch_bounds__(64 * blockWaves(W)) __attribute__((amdgpu_waves_per
                 q[12] = 0;
             }
         }
+        poolFence(); // slots written above, read below by other lanes
         // lanes without a photon take ready ones from the front of the window
         const uint32_t take = min(nEmpty, ready);
         if (take != 0) {
@@ -349,6 +350,7 @@ __global__ __launch_bounds__(64 * blockWaves(W)) __attribute__((amdgpu_waves_per
             first = first >= slots ? first - slots : first;
             ready -= take;
         }
+        poolFence(); // slots read above, written next by other lanes
         const bool more = poolNext < poolEnd || !claimedAll || ready != 0;
         if (__ballot(flying) == 0) {
             if (!more && pending == 0)

@@ -356,6 +356,7 @@ __global__ __launch_bounds__(64 * WAVES_PER_CU) __attribute__((amdgpu_waves_per_
                 q[24] = 0;
             }
         }
+        poolFence(); // slots written above, read below by other lanes
         // lanes without a photon take ready ones from the front of the window
         const uint32_t take = min(nEmpty, ready);
         if (take != 0) {
@@ -369,6 +370,7 @@ __global__ __launch_bounds__(64 * WAVES_PER_CU) __attribute__((amdgpu_waves_per_
             first = first >= slots ? first - slots : first;
             ready -= take;
         }
+        poolFence(); // slots read above, written next by other lanes
         const bool more = poolNext < poolEnd || !claimedAll || ready != 0;
         if (__ballot(flying) == 0) {
             if (!more && pending == 0)
